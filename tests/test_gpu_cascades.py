@@ -8,8 +8,7 @@
   5-bit bitfield and its popcount bit-exact given identical densities;
 * training rays through the cascades (dt from sqrt(3)/1024 to 16x that,
   cone 1/256): per-ray counts, offsets and every per-sample output bit-exact,
-  with few rays (a wave per ray) and with many (lanes skip empty space for
-  their own rays).
+  with few rays (16 lanes share a ray) and with many (8 lanes do).
 """
 import math
 
@@ -98,10 +97,8 @@ def test_cascade_bitfield_and_update(field):
 
 @pytest.mark.parametrize("n_rays,max_steps", [(2048, 0xFFFFFFFF), (40960, 0xFFFFFFFF), (40960, 48)])
 def test_cascade_marching(field, n_rays, max_steps):
-    """2048 rays: a wave marches one ray at a time. 40960 rays (five per wave
-    of the bounded grid): lanes take their own rays through empty cells and
-    the wave takes each ray's occupied runs together; also with a cap of 48
-    samples per ray, which ends runs part-way. All bit-exact."""
+    """2048 rays (16 lanes per ray) and 40960 rays (8 lanes per ray), also with
+    a cap of 48 samples per ray, which ends runs part-way. All bit-exact."""
     import torch
 
     import oracle

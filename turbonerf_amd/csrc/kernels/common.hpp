@@ -125,27 +125,6 @@ TN_DEVICE uint32_t compact_bits10(uint32_t v) {
 }
 
 // ---------------------------------------------------------------------------
-// Directed-rounding division a / b rounded toward +infinity. q = RN(a/b) is
-// correctly rounded (HIP's default fp32 division), and the residual
-// a - q*b is exact when formed with one fused multiply-add (Boldo & Muller,
-// "Exact and approximated error of the FMA", IEEE TC 2011). A residual with
-// the sign of b means the exact quotient lies above q.
-// ---------------------------------------------------------------------------
-TN_DEVICE float fdiv_ru(float a, float b) {
-    float q = a / b;
-    const float r = __builtin_fmaf(-q, b, a);
-    const bool above = (b > 0.0f) ? (r > 0.0f) : (r < 0.0f);
-    if (above) {
-        uint32_t u = __float_as_uint(q);
-        if (q > 0.0f) u += 1u;
-        else if (q < 0.0f) u -= 1u;
-        else u = 1u;  // +0 -> smallest positive subnormal
-        q = __uint_as_float(u);
-    }
-    return q;
-}
-
-// ---------------------------------------------------------------------------
 // bounding box (same semantics as the reference BoundingBox)
 // ---------------------------------------------------------------------------
 TN_DEVICE bool bbox_contains(const tn_bbox_t& b, float x, float y, float z) {
@@ -200,24 +179,6 @@ TN_DEVICE uint32_t voxel_morton_index(float res_f, uint32_t lim, int level, floa
     yu = min(yu, lim);
     zu = min(zu, lim);
     return morton3d(xu, yu, zu);
-}
-
-// distance along the ray to the next cell boundary of `level`, rounded up to
-// a whole multiple of dt_min through a directed division
-TN_DEVICE float dt_to_next_voxel(float res_f, float inv_res, float px, float py, float pz, float dx,
-                                 float dy, float dz, float idx, float idy, float idz, float dt_min,
-                                 int level) {
-    const float level_size = (float)(1 << level);
-    const float i_level_size = 1.0f / level_size;
-    const float x = (px * i_level_size + 0.5f) * res_f;
-    const float y = (py * i_level_size + 0.5f) * res_f;
-    const float z = (pz * i_level_size + 0.5f) * res_f;
-    const float k = inv_res * level_size;
-    const float tx = k * ((floorf(0.5f * copysignf(1.0f, dx) + x + 0.5f) - x) * idx);
-    const float ty = k * ((floorf(0.5f * copysignf(1.0f, dy) + y + 0.5f) - y) * idy);
-    const float tz = k * ((floorf(0.5f * copysignf(1.0f, dz) + z + 0.5f) - z) * idz);
-    const float t_target = fmaxf(dt_min, fminf(fminf(tx, ty), tz));
-    return fdiv_ru(t_target, dt_min) * dt_min;
 }
 
 // sigma = exp(min(s, 12) - 1) (reference common-network-kernels.cuh:7-10)

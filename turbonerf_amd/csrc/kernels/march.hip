@@ -33,277 +33,253 @@ TN_DEVICE MarchGrid make_grid(const tn_occupancy_grid_t& g) {
     return m;
 }
 
-// Marching runs one wave per ray and reproduces the reference's serial
-// recurrence exactly (contraction off, same operation order). The 64 lanes
-// buy two things:
-//  * runs of occupied steps: from a point t inside the box, lane j forms t_j,
-//    the t after j more occupied steps (the same serial sums), and reads the
-//    occupancy bit of its own cell at its own cascade; the leading lanes whose
-//    steps are inside, within the limits and occupied are taken at once, for
-//    one gather per 64 steps. If lane 0 fails, the cell at t is empty;
-//  * empty-space skipping: the serial DDA skip steps look cells up in a wave
-//    cache. A lookup that misses refills it with 64 parallel loads, lane k
-//    taking the cell at k half-cells further along the ray from the point that
-//    missed (t0). Entries are keyed by (cascade, Morton index) and hold that
-//    cell's own bit, so a prefetched entry can never change a result; lane 0
-//    holds the exact cell of the point that missed.
-struct WaveCache {
-    uint32_t key = 0xFFFFFFFFu;  // per lane
-    uint32_t occ = 0;            // per lane
-    int level = -1;              // wave-uniform from here on
-    float t0 = 0.0f;             // ray t of lane 0's point
-    float inv_h = 0.0f;          // 1 / (half a cell of `level`, in ray t)
+// Marching follows the reference's serial recurrence exactly (contraction
+// off, same operation order): at a ray's t, an occupied cell gives a sample
+// and t += dt(t), an empty one a skip by the distance to the next cell
+// boundary, divided by dt_min rounding upwards and multiplied back (reference
+// src/core/occupancy-grid.cuh:243-282). What bounds
+// it is the length of that dependent chain, several hundred steps for a ray
+// through a mostly empty box, so everything but the chain itself is taken off
+// it:
+//  * a group of G lanes shares a ray. It forms G steps of the recurrence on
+//    the assumption that the cells on the way stay occupied (a run of
+//    samples) or empty (a skip), lane j keeping the j-th t, and then tests the
+//    G points side by side: one gather of occupancy bits for G steps. The
+//    leading points that bear the assumption out are taken, and the group goes
+//    on from the first that does not;
+//  * a skip step needs three axes' distances to their next cell boundary. Lane
+//    j of a group works on axis j % 4 (2 and 3 alike) and the minimum is taken
+//    across the quad, which leaves about a third of the instructions;
+//  * the step's division by dt_min, rounded upwards, is by a constant: its
+//    reciprocal is formed once (div_up);
+//  * the cascade of a point is formed from exponents, without a loop.
+// A skip step is 24 vector instructions in one cascade and 36 in several. A
+// wave per ray that looked every skip step's cell up in turn took 214 us to
+// count and 116 us to generate a batch of 4,369 rays through a unit box with
+// 8 blobs, and 120 us to count 53 rays; this takes 51, 47 and 42 us.
+// G is 16 for up to kGroup16Rays rays and 8 for more (see there).
+struct MarchStep {
+    float cone, dt_min, dt_max, inv_dt_min;
 };
-
-TN_DEVICE void wave_cache_fill(const MarchGrid& g, int level, float t, float x, float y, float z, float dx, float dy,
-                               float dz, WaveCache& wc) {
-    const float half_cell = 0.5f * (float)(1 << level) * g.inv_res;
-    const float tj = (float)__lane_id() * half_cell;  // 0 for lane 0: its point is (x, y, z) exactly
-    const uint32_t m = voxel_morton_index(g.res_f, g.lim, level, x + tj * dx, y + tj * dy, z + tj * dz);
-    wc.key = m;
-    wc.occ = (g.bits[m] >> level) & 1u;
-    wc.level = level;
-    wc.t0 = t;
-    wc.inv_h = 1.0f / half_cell;
-}
-
-TN_DEVICE bool wave_occupied(const MarchGrid& g, int level, float t, float x, float y, float z, float dx, float dy,
-                             float dz, WaveCache& wc) {
-    const uint32_t m = voxel_morton_index(g.res_f, g.lim, level, x, y, z);
-    uint64_t hit = level == wc.level ? __ballot(wc.key == m) : 0ull;
-    if (hit == 0ull) {
-        wave_cache_fill(g, level, t, x, y, z, dx, dy, dz, wc);
-        hit = __ballot(wc.key == m);  // lane 0 at least
-    }
-    return (__ballot(wc.occ != 0u) & hit) != 0ull;
-}
 
 struct MarchRay {
     float ox, oy, oz, dx, dy, dz;
 };
 
-// Leading lanes (at least 0, at most 64) whose step, j occupied steps after
-// t, is inside the box, below t_max, within `budget` and occupied; t_lane =
-// t_j. Each lane still in the running reads its own cell's bit. `empty_stop`
-// tells whether the first lane that failed did so only for an empty cell
-// (the serial loop's next step is then a DDA skip from that lane's t).
-TN_DEVICE uint32_t occupied_run(const MarchGrid& g, const tn_bbox_t& bbox, const MarchRay& r, float t, float t_max,
-                                uint32_t budget, float cone, float dt_min, float dt_max, float& t_lane,
-                                bool& empty_stop) {
+// a / b rounded towards +infinity for positive a and b = dt_min, given y =
+// RN(1 / b): q0 = RN(a y) is within 2 ulp; one correction by its residual
+// leaves a neighbour of a / b (or a / b itself), and the sign of that
+// neighbour's residual, which one fused multiply-add gives exactly, tells
+// whether it lies below (Boldo & Muller, "Exact and approximated error of the
+// FMA", IEEE TC 2011).
+TN_DEVICE float div_up(float a, float b, float y) {
+    const float q0 = a * y;
+    const float q = __builtin_fmaf(__builtin_fmaf(-q0, b, a), y, q0);
+    return __uint_as_float(__float_as_uint(q) + (__builtin_fmaf(-q, b, a) > 0.0f ? 1u : 0u));
+}
+
+// The cascade (grid_level_at) of a point whose largest |coordinate| has the
+// bits m, from the step dt that decides it: level k covers the point when
+// 2^k / 2 > |coordinate| and 2^k inv_res > dt. 2^k only adds k to the exponent,
+// so the first such k follows from the difference of the bit patterns, rounded
+// up to a whole exponent; `bits` is k << 23, which added to a float's pattern
+// multiplies it by 2^k (no zeros or overflows here: n_levels <= 8).
+struct Cascade {
+    int bits;
+    TN_DEVICE int level() const { return bits >> 23; }
+    TN_DEVICE float inv_scale() const { return __uint_as_float(0x3F800000u - (uint32_t)bits); }  // 2^-k
+    TN_DEVICE float scaled(float v) const { return __uint_as_float(__float_as_uint(v) + (uint32_t)bits); }
+};
+constexpr int kExponentOne = 1 << 23;
+TN_DEVICE Cascade cascade_of(int n_levels, float inv_res, uint32_t m, float dt) {
+    const int d1 = (int)m - ((int)0x3F000000 - kExponentOne);  // 0x3F000000: 0.5
+    const int d2 = (int)__float_as_uint(dt) - ((int)__float_as_uint(inv_res) - kExponentOne);
+    const int k = max(d1, d2) & ~(kExponentOne - 1);
+    return Cascade{min(max(k, 0), (n_levels - 1) << 23)};
+}
+// get_dt; dt_min <= dt_max
+TN_DEVICE float step_dt(const MarchStep& st, float t) {
+    return __builtin_amdgcn_fmed3f(t * st.cone, st.dt_min, st.dt_max);
+}
+TN_DEVICE uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7FFFFFFFu; }
+
+// occupancy of the cell at (x, y, z); ML: several cascades
+template <bool ML>
+TN_DEVICE bool point_occupied(const MarchGrid& g, const MarchStep& st, float t, float x, float y, float z) {
+    Cascade c{0};
+    if constexpr (ML)
+        c = cascade_of(g.n_levels, g.inv_res, max(max(abs_bits(x), abs_bits(y)), abs_bits(z)),
+                       step_dt(st, t) * g.level_scale);
+    const float s = ML ? c.inv_scale() : 1.0f;
+    const uint32_t xu = min((uint32_t)fmaxf((x * s + 0.5f) * g.res_f, 0.0f), g.lim);
+    const uint32_t yu = min((uint32_t)fmaxf((y * s + 0.5f) * g.res_f, 0.0f), g.lim);
+    const uint32_t zu = min((uint32_t)fmaxf((z * s + 0.5f) * g.res_f, 0.0f), g.lim);
+    return ((g.bits[morton3d(xu, yu, zu)] >> (ML ? c.level() : 0)) & 1u) != 0u;
+}
+
+// distance to the next cell boundary along one axis: gc the coordinate in
+// cells, h = copysign(0.5, d), id = 1 / d, k the cell's side
+TN_DEVICE float axis_distance(float gc, float h, float id, float k) {
+    return k * ((floorf(h + gc + 0.5f) - gc) * id);
+}
+
+// max(lo, minimum of v over the quad), a NaN (a ray along a cell face) left out
+// as fminf and fmaxf do. In assembly because fminf of a lane-permuted value
+// costs a move and a quieting max besides; the two wait states that a DPP read
+// needs after a vector write are part of it.
+TN_DEVICE float quad_min_above(float v, float lo) {
+    float a, b;
+    asm("s_nop 1\n\tv_min_f32_dpp %0, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf" : "=&v"(a) : "v"(v));
+    asm("s_nop 1\n\tv_min_f32_dpp %0, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\tv_max_f32 %0, %2, %0"
+        : "=&v"(b)
+        : "v"(a), "s"(lo));
+    return b;
+}
+TN_DEVICE uint32_t quad_max(uint32_t v) {
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true));     // lanes 1 0 3 2
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));  // lanes 2 3 0 1
+}
+
+// index of the group's first lane with a set bit of `ballot`, or G (8 or 16)
+template <int G>
+TN_DEVICE uint32_t group_first(uint64_t ballot) {
     const uint32_t lane = __lane_id();
-    float tj = t;
-    if (dt_min == dt_max) {
-        for (uint32_t k = 0; k < 63; ++k) {
-            const float tn = tj + dt_min;
-            tj = lane > k ? tn : tj;
-        }
-    } else {
-        for (uint32_t k = 0; k < 63; ++k) {
-            const float tn = tj + get_dt(tj, cone, dt_min, dt_max);
-            tj = lane > k ? tn : tj;
-        }
-    }
-    t_lane = tj;
-    const float x = r.ox + tj * r.dx, y = r.oy + tj * r.dy, z = r.oz + tj * r.dz;
-    const bool within = lane < budget && tj < t_max && bbox_contains(bbox, x, y, z);
-    bool good = within;
-    if (within) {
-        const float dtj = get_dt(tj, cone, dt_min, dt_max);
-        const int lvl = grid_level_at(g.n_levels, g.inv_res, x, y, z, dtj * g.level_scale);
-        const uint32_t m = voxel_morton_index(g.res_f, g.lim, lvl, x, y, z);
-        good = ((g.bits[m] >> lvl) & 1u) != 0u;
-    }
-    const uint64_t bad = __ballot(!good);
-    const uint64_t empty = __ballot(within && !good);
-    const uint32_t f = bad == 0ull ? 64u : (uint32_t)__builtin_ctzll(bad);
-    empty_stop = f < 64u && ((empty >> f) & 1ull) != 0ull;
-    return f;
+    const uint32_t half = lane < 32u ? (uint32_t)ballot : (uint32_t)(ballot >> 32);
+    return (uint32_t)__builtin_ctz((half >> (lane & 31u & ~(uint32_t)(G - 1))) | (1u << G));
+}
+// v of the group's lane j
+template <int G>
+TN_DEVICE float group_get(float v, uint32_t j) {
+    return __shfl(v, (int)((__lane_id() & ~(uint32_t)(G - 1)) + j), 64);
 }
 
-// DDA skip steps from t, whose cell is empty, until the point is outside the
-// box, at or beyond t_max, or in an occupied cell (the reference's loop takes
-// the same steps, testing each point in turn); returns that point's t.
-TN_DEVICE float skip_empty(const MarchGrid& g, const tn_bbox_t& bbox, const MarchRay& r, float t, float t_max,
-                           float cone, float dt_min, float dt_max, float idx, float idy, float idz, WaveCache& wc) {
-    float x = r.ox + t * r.dx, y = r.oy + t * r.dy, z = r.oz + t * r.dz;
-    int lvl = grid_level_at(g.n_levels, g.inv_res, x, y, z, get_dt(t, cone, dt_min, dt_max) * g.level_scale);
-    for (;;) {
-        t += dt_to_next_voxel(g.res_f, g.inv_res, x, y, z, r.dx, r.dy, r.dz, idx, idy, idz, dt_min, lvl);
-        if (!(t < t_max)) return t;
-        x = r.ox + t * r.dx;
-        y = r.oy + t * r.dy;
-        z = r.oz + t * r.dz;
-        if (!bbox_contains(bbox, x, y, z)) return t;
-        lvl = grid_level_at(g.n_levels, g.inv_res, x, y, z, get_dt(t, cone, dt_min, dt_max) * g.level_scale);
-        if (wave_occupied(g, lvl, t, x, y, z, r.dx, r.dy, r.dz, wc)) return t;
+// One ray per group, all 64 / G of a wave at once. Emits through `emit(n, t)`
+// (lane-wise: sample n of the lane's ray at t). COUNT: stops at t_max, at
+// the box and at max_n samples; otherwise (the generate pass) takes max_n
+// samples, and one outside the box, which the count pass cannot have counted,
+// would be emitted without advancing. Returns the ray's sample count.
+template <int G, bool ML, bool COUNT, typename Emit>
+TN_DEVICE uint32_t march_group(bool active, const MarchRay& r, float t, float t_max, uint32_t max_n,
+                               const tn_bbox_t& bbox, const MarchGrid& g, const MarchStep& st, Emit emit) {
+    const uint32_t lane = __lane_id(), j = lane & (uint32_t)(G - 1), axis = lane & 3u;
+    const float oa = axis == 0 ? r.ox : axis == 1 ? r.oy : r.oz;
+    const float da = axis == 0 ? r.dx : axis == 1 ? r.dy : r.dz;
+    const float ida = 1.0f / da, ha = 0.5f * copysignf(1.0f, da);
+    uint32_t n = 0;
+    bool done = !active, skip = false;
+    while (__ballot(!done) != 0ull) {
+        if (__ballot(!done && !skip) != 0ull) {
+            // a run: lane j's t after j more samples
+            float tj = t;
+            if (st.dt_min == st.dt_max) {
+#pragma unroll
+                for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k) tj = j > k ? tj + st.dt_min : tj;
+            } else {
+#pragma unroll
+                for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k)
+                    tj = j > k ? tj + step_dt(st, tj) : tj;
+            }
+            const float x = r.ox + tj * r.dx, y = r.oy + tj * r.dy, z = r.oz + tj * r.dz;
+            const bool inside = bbox_contains(bbox, x, y, z);
+            const bool within = !done && !skip && j < max_n - n && (!COUNT || tj < t_max) && inside;
+            const bool good = within && point_occupied<ML>(g, st, tj, x, y, z);
+            const uint32_t f = group_first<G>(__ballot(!good));
+            const uint32_t e = group_first<G>(__ballot(within && !good));
+            const float tn = tj + step_dt(st, tj);
+            const float t_f = group_get<G>(f < (uint32_t)G ? tj : tn, f < (uint32_t)G ? f : (uint32_t)G - 1u);
+            if (!done && !skip) {
+                if (j < f) emit(n + j, tj);
+                n += f;
+                t = t_f;
+                skip = f < (uint32_t)G && e == f;  // the run ended at an empty cell
+                if (f < (uint32_t)G && !skip) {
+                    if (!COUNT)
+                        for (uint32_t k = n + j; k < max_n; k += (uint32_t)G) emit(k, t);
+                    done = true;
+                }
+            }
+        }
+        if (__ballot(!done && skip) != 0ull) {
+            // a skip from an empty cell: lane j's t after j + 1 steps
+            float tc = t, tj = t;
+#pragma unroll
+            for (uint32_t k = 0; k < (uint32_t)G; ++k) {
+                const float p = oa + tc * da;
+                float s = 1.0f, cell = g.inv_res;
+                if constexpr (ML) {
+                    const Cascade c = cascade_of(g.n_levels, g.inv_res, quad_max(abs_bits(p)),
+                                                 step_dt(st, tc) * g.level_scale);
+                    s = c.inv_scale();
+                    cell = c.scaled(g.inv_res);
+                }
+                const float gc = (p * s + 0.5f) * g.res_f;
+                const float d = quad_min_above(axis_distance(gc, ha, ida, cell), st.dt_min);
+                tc += div_up(d, st.dt_min, st.inv_dt_min) * st.dt_min;
+                tj = j == k ? tc : tj;
+            }
+            const float x = r.ox + tj * r.dx, y = r.oy + tj * r.dy, z = r.oz + tj * r.dz;
+            const bool within = !done && skip && (!COUNT || tj < t_max) && bbox_contains(bbox, x, y, z);
+            const bool occupied = within && point_occupied<ML>(g, st, tj, x, y, z);
+            const uint32_t f = group_first<G>(__ballot(!within || occupied));
+            const float t_f = group_get<G>(tj, min(f, (uint32_t)G - 1u));
+            if (!done && skip) {
+                t = t_f;
+                skip = f == (uint32_t)G;  // otherwise the run's tests decide at t
+            }
+        }
     }
-}
-
-// t after the run of f steps: lane f's t_f, or one more step after lane 63's
-TN_DEVICE float after_run(uint32_t f, float t_lane, float cone, float dt_min, float dt_max) {
-    if (f < 64u) return __shfl(t_lane, (int)f, 64);
-    const float t63 = __shfl(t_lane, 63, 64);
-    return t63 + get_dt(t63, cone, dt_min, dt_max);
+    return n;
 }
 
 constexpr int kMarchWaves = 4;  // waves per workgroup
 // The marching kernels are launched on at most TN_TUNE_MARCH_MAX_BLOCKS
-// workgroups (2048 by default: a larger grid leaves a large scene's render
-// passes under four rays per wave, in the wave-per-ray mode: 8192 took its
-// 1080p frame from 81 to 199 ms) and stride
-// over the live rays, one ray per wave at a time: the ray count lives on the
-// device, and a grid sized for the largest batch would launch a wave per
-// possible ray, nearly all of which exit at once yet occupy the dispatcher
-// beside the network kernels.
+// workgroups and stride over the live rays: the ray count lives on the device,
+// and a grid sized for the largest batch would launch a wave per possible ray,
+// nearly all of which exit at once yet occupy the dispatcher beside the
+// network kernels.
 inline unsigned march_blocks(uint32_t n_rays_max) {
-    return std::min(blocks_for(n_rays_max, kMarchWaves), (unsigned)tune_value(TN_TUNE_MARCH_MAX_BLOCKS));
+    return std::min(blocks_for((uint64_t)n_rays_max * 16, 64 * kMarchWaves), (unsigned)tune_value(TN_TUNE_MARCH_MAX_BLOCKS));
 }
 
-TN_DEVICE void march_count_ray(uint32_t i, uint32_t B, const tn_bbox_t& bbox, const MarchGrid& g, float cone,
-                               float dt_min, float dt_max, uint32_t max_steps, const float* __restrict__ dir,
-                               const float* __restrict__ ray_tmax, uint8_t* __restrict__ ray_alive,
-                               const float* __restrict__ ori, const float* __restrict__ ray_t,
-                               uint32_t* __restrict__ n_steps) {
-    const bool lane0 = __lane_id() == 0;
-    if (!ray_alive[i]) {
-        if (lane0) n_steps[i] = 0;
-        return;
-    }
-    const MarchRay r = {ori[i], ori[i + B], ori[i + 2 * B], dir[i], dir[i + B], dir[i + 2 * B]};
-    const float idx = 1.0f / r.dx, idy = 1.0f / r.dy, idz = 1.0f / r.dz;
-    uint32_t n = 0;
-    float t = ray_t[i];
-    const float t_max = ray_tmax[i];
-    WaveCache wc;
-    while (t < t_max && n < max_steps) {
-        const float x = r.ox + t * r.dx, y = r.oy + t * r.dy, z = r.oz + t * r.dz;
-        if (!bbox_contains(bbox, x, y, z)) break;
-        float t_lane;
-        bool empty;
-        const uint32_t f = occupied_run(g, bbox, r, t, t_max, max_steps - n, cone, dt_min, dt_max, t_lane, empty);
-        if (f != 0u) {
-            t = after_run(f, t_lane, cone, dt_min, dt_max);
-            n += f;
-        }
-        // f == 0: lane 0 is inside, below t_max and within budget, so its cell is empty
-        if (f == 0u || empty) t = skip_empty(g, bbox, r, t, t_max, cone, dt_min, dt_max, idx, idy, idz, wc);
-    }
-    if (lane0) {
-        if (n == 0) ray_alive[i] = 0;
-        n_steps[i] = n;
-    }
+// A group of 16 halves the tests per step and so a ray's latency, one of 8 the
+// waves that a large pass needs. Measured, count pass in us with groups of 16
+// and of 8 (unit box with 8 blobs; 16-unit box with 5 cascades and 128 small
+// blobs): 4,096 rays 51 / 85 and 133 / 166, 16,384 rays 45 / 45 and 150 / 167,
+// 32,768 rays 57 / 45 and 224 / 179, 131,072 rays 120 / 78 and 466 / 304.
+// Groups of 4 took 80 and 310 there and 146 and 237 at 4,096, groups of 32 and
+// 64 were slower at every size, and a ray per lane took 96 and 327 at 131,072.
+constexpr uint32_t kGroup16Rays = 24576;
+
+TN_DEVICE MarchRay load_ray(bool active, uint32_t i, uint32_t B, const float* __restrict__ ori,
+                            const float* __restrict__ dir) {
+    return active ? MarchRay{ori[i], ori[i + B], ori[i + 2 * B], dir[i], dir[i + B], dir[i + 2 * B]}
+                  : MarchRay{0.0f, 0.0f, 0.0f, 1.0f, 1.0f, 1.0f};
 }
 
-TN_DEVICE float lane_f(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
-TN_DEVICE uint32_t lane_u(uint32_t v, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); }
-
-// Many rays per wave (a render pass or a sparse scene): lanes [0, K) own rays
-// first + lane. Each lane takes its ray through empty cells by the serial DDA
-// itself (reading its cells' bits), so the long skips of rays through mostly
-// empty space run side by side; a ray that reaches an occupied cell is then
-// taken by the whole wave for its occupied runs (one ray at a time, as in
-// march_count_ray), after which its lane resumes. Every ray follows the same
-// recurrence as march_count_ray, step for step.
-struct LaneRayState {
-    MarchRay r;
-    float idx, idy, idz, t, t_max;
-    uint32_t n;
-    bool done, ready;
+struct MarchCountArgs {
+    uint32_t n_rays, B, max_steps;
+    const float *dir, *tmax, *ori, *t;
+    uint8_t* alive;
+    uint32_t* n_steps;
 };
 
-TN_DEVICE void lane_skip_step(const MarchGrid& g, const tn_bbox_t& bbox, float cone, float dt_min, float dt_max,
-                              uint32_t max_steps, LaneRayState& q) {
-    if (!(q.t < q.t_max && q.n < max_steps)) {
-        q.done = true;
-        return;
-    }
-    const float x = q.r.ox + q.t * q.r.dx, y = q.r.oy + q.t * q.r.dy, z = q.r.oz + q.t * q.r.dz;
-    if (!bbox_contains(bbox, x, y, z)) {
-        q.done = true;
-        return;
-    }
-    const int lvl = grid_level_at(g.n_levels, g.inv_res, x, y, z, get_dt(q.t, cone, dt_min, dt_max) * g.level_scale);
-    if ((g.bits[voxel_morton_index(g.res_f, g.lim, lvl, x, y, z)] >> lvl) & 1u)
-        q.ready = true;
-    else
-        q.t += dt_to_next_voxel(g.res_f, g.inv_res, x, y, z, q.r.dx, q.r.dy, q.r.dz, q.idx, q.idy, q.idz, dt_min, lvl);
-}
-
-TN_DEVICE LaneRayState lane_ray_state(bool active, uint32_t i, uint32_t B, const float* __restrict__ ori,
-                                      const float* __restrict__ dir, const float* __restrict__ ray_t, float t_max) {
-    LaneRayState q;
-    q.r = active ? MarchRay{ori[i], ori[i + B], ori[i + 2 * B], dir[i], dir[i + B], dir[i + 2 * B]}
-                 : MarchRay{0.0f, 0.0f, 0.0f, 1.0f, 1.0f, 1.0f};
-    q.idx = 1.0f / q.r.dx;
-    q.idy = 1.0f / q.r.dy;
-    q.idz = 1.0f / q.r.dz;
-    q.t = active ? ray_t[i] : 0.0f;
-    q.t_max = t_max;
-    q.n = 0;
-    q.done = !active;
-    q.ready = false;
-    return q;
-}
-
-TN_DEVICE MarchRay lane_ray(const MarchRay& r, int l) {
-    return MarchRay{lane_f(r.ox, l), lane_f(r.oy, l), lane_f(r.oz, l), lane_f(r.dx, l), lane_f(r.dy, l),
-                    lane_f(r.dz, l)};
-}
-
-TN_DEVICE void march_count_lanes(uint32_t first, uint32_t K, uint32_t n_rays, uint32_t B, const tn_bbox_t& bbox,
-                                 const MarchGrid& g, float cone, float dt_min, float dt_max, uint32_t max_steps,
-                                 const float* __restrict__ dir, const float* __restrict__ ray_tmax,
-                                 uint8_t* __restrict__ ray_alive, const float* __restrict__ ori,
-                                 const float* __restrict__ ray_t, uint32_t* __restrict__ n_steps) {
-    const uint32_t lane = __lane_id();
-    const uint32_t i = first + lane;
-    const bool own = lane < K && i < n_rays;
-    const bool active = own && ray_alive[i] != 0;
-    LaneRayState q = lane_ray_state(active, i, B, ori, dir, ray_t, active ? ray_tmax[i] : 0.0f);
-    while (__ballot(!q.done) != 0ull) {
-        if (!q.done && !q.ready) lane_skip_step(g, bbox, cone, dt_min, dt_max, max_steps, q);
-        uint64_t rb = __ballot(q.ready);
-        while (rb != 0ull) {
-            const int L = __builtin_ctzll(rb);
-            rb &= rb - 1ull;
-            const MarchRay r = lane_ray(q.r, L);
-            float t = lane_f(q.t, L);
-            const float t_max = lane_f(q.t_max, L);
-            uint32_t n = lane_u(q.n, L);
-            for (;;) {  // the point at t is occupied and within the limits, so the first run takes a step
-                float t_lane;
-                bool empty;
-                const uint32_t f = occupied_run(g, bbox, r, t, t_max, max_steps - n, cone, dt_min, dt_max, t_lane, empty);
-                if (f == 0u) break;
-                t = after_run(f, t_lane, cone, dt_min, dt_max);
-                n += f;
-                if (f < 64u || !(t < t_max && n < max_steps)) break;
-            }
-            if ((int)lane == L) {
-                q.t = t;
-                q.n = n;
-                q.ready = false;  // the lane's next step re-tests the point where the run stopped
-            }
+template <int G, bool ML>
+TN_DEVICE void march_count_rays(const MarchCountArgs& a, const tn_bbox_t& bbox, const MarchGrid& g,
+                                const MarchStep& st) {
+    const uint32_t n_threads = gridDim.x * blockDim.x, tid = blockIdx.x * blockDim.x + threadIdx.x;
+    // whole waves: every lane of a wave takes part in the group operations
+    for (uint32_t w = tid & ~63u; w / G < a.n_rays; w += n_threads) {
+        const uint32_t i = (w + (tid & 63u)) / G;
+        const bool own = i < a.n_rays;
+        const bool active = own && a.alive[i] != 0;
+        const MarchRay r = load_ray(active, i, a.B, a.ori, a.dir);
+        const uint32_t n = march_group<G, ML, true>(active, r, active ? a.t[i] : 0.0f, active ? a.tmax[i] : 0.0f,
+                                                  a.max_steps, bbox, g, st, [](uint32_t, float) {});
+        if (own && (tid & (uint32_t)(G - 1)) == 0) {
+            if (active && n == 0) a.alive[i] = 0;
+            a.n_steps[i] = n;
         }
     }
-    if (own) {
-        if (!active) {
-            n_steps[i] = 0;
-        } else {
-            if (q.n == 0) ray_alive[i] = 0;
-            n_steps[i] = q.n;
-        }
-    }
-}
-
-// Rays per wave from which lanes take rays through empty space themselves;
-// below it a wave marches one ray at a time (march_count_ray), skipping with
-// its wave cache, which is faster per ray.
-constexpr uint32_t kLaneRaysMin = 4;
-
-TN_DEVICE uint32_t rays_per_wave(uint32_t n_rays, uint32_t n_waves) {
-    const uint32_t k = (n_rays + n_waves - 1) / n_waves;
-    return k < kLaneRaysMin ? 1u : min(k, 64u);
 }
 
 __global__ void __launch_bounds__(64 * kMarchWaves)
@@ -312,18 +288,15 @@ march_count_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ d_n_rays, u
                    const float* __restrict__ dir, const float* __restrict__ ray_tmax, uint8_t* __restrict__ ray_alive,
                    const float* __restrict__ ori, const float* __restrict__ ray_t, uint32_t* __restrict__ n_steps) {
     const uint32_t n_rays = d_n_rays ? min(*d_n_rays, n_rays_max) : n_rays_max;
-    const uint32_t n_waves = gridDim.x * kMarchWaves;
-    const uint32_t wave = blockIdx.x * kMarchWaves + (threadIdx.x >> 6);
     const MarchGrid g = make_grid(grid);
-    const uint32_t K = rays_per_wave(n_rays, n_waves);
-    if (K == 1) {
-        for (uint32_t i = wave; i < n_rays; i += n_waves)
-            march_count_ray(i, B, bbox, g, cone, dt_min, dt_max, max_steps, dir, ray_tmax, ray_alive, ori, ray_t,
-                            n_steps);
+    const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
+    const MarchCountArgs a = {n_rays, B, max_steps, dir, ray_tmax, ori, ray_t, ray_alive, n_steps};
+    if (grid.n_levels == 1) {
+        if (n_rays <= kGroup16Rays) march_count_rays<16, false>(a, bbox, g, st);
+        else march_count_rays<8, false>(a, bbox, g, st);
     } else {
-        for (uint32_t first = wave * K; first < n_rays; first += n_waves * K)
-            march_count_lanes(first, K, n_rays, B, bbox, g, cone, dt_min, dt_max, max_steps, dir, ray_tmax, ray_alive,
-                              ori, ray_t, n_steps);
+        if (n_rays <= kGroup16Rays) march_count_rays<16, true>(a, bbox, g, st);
+        else march_count_rays<8, true>(a, bbox, g, st);
     }
 }
 
@@ -449,108 +422,29 @@ __global__ void scan_write_select_kernel(uint32_t n, const uint32_t* __restrict_
     }
 }
 
-TN_DEVICE void march_generate_ray(uint32_t i, uint32_t B, const tn_bbox_t& bbox, const MarchGrid& g, float dt_min,
-                                  float dt_max, float cone, const float* __restrict__ ori,
-                                  const float* __restrict__ dir, const float* __restrict__ ray_t,
-                                  const uint32_t* __restrict__ ray_offset, const uint32_t* __restrict__ n_ray_steps,
-                                  uint32_t* __restrict__ out_ray, float* __restrict__ out_t) {
-    const uint32_t lane = __lane_id();
-    const uint32_t n_steps = n_ray_steps[i];
-    const uint32_t off = ray_offset[i];
-    const MarchRay r = {ori[i], ori[i + B], ori[i + 2 * B], dir[i], dir[i + B], dir[i + 2 * B]};
-    const float idx = 1.0f / r.dx, idy = 1.0f / r.dy, idz = 1.0f / r.dz;
-    float t = ray_t[i];
-    uint32_t n = 0;
-    WaveCache wc;
-    while (n < n_steps) {
-        const float x = r.ox + t * r.dx, y = r.oy + t * r.dy, z = r.oz + t * r.dz;
-        if (!bbox_contains(bbox, x, y, z)) {
-            // the count pass stops at the box boundary, so every counted
-            // sample is inside; one outside would be emitted without advancing
-            if (lane == 0) {
-                out_t[off + n] = t;
-                out_ray[off + n] = i;
-            }
-            ++n;
-            continue;
-        }
-        float t_lane;
-        bool empty;
-        const uint32_t f = occupied_run(g, bbox, r, t, INFINITY, n_steps - n, cone, dt_min, dt_max, t_lane, empty);
-        if (f != 0u) {
-            if (lane < f) {  // one coalesced row of samples
-                out_t[off + n + lane] = t_lane;
-                out_ray[off + n + lane] = i;
-            }
-            t = after_run(f, t_lane, cone, dt_min, dt_max);
-            n += f;
-        }
-        if (f == 0u || empty) t = skip_empty(g, bbox, r, t, INFINITY, cone, dt_min, dt_max, idx, idy, idz, wc);
-    }
-}
+struct MarchGenerateArgs {
+    uint32_t n_rays, B;
+    const float *ori, *dir, *t;
+    const uint32_t *offset, *n_steps;
+    const uint8_t* alive;
+    uint32_t* out_ray;
+    float* out_t;
+};
 
-// march_generate_ray for rays first + lane, lanes [0, K) (see march_count_lanes)
-TN_DEVICE void march_generate_lanes(uint32_t first, uint32_t K, uint32_t n_rays, uint32_t B, const tn_bbox_t& bbox,
-                                    const MarchGrid& g, float dt_min, float dt_max, float cone,
-                                    const float* __restrict__ ori, const float* __restrict__ dir,
-                                    const float* __restrict__ ray_t, const uint32_t* __restrict__ ray_offset,
-                                    const uint8_t* __restrict__ ray_alive, const uint32_t* __restrict__ n_ray_steps,
-                                    uint32_t* __restrict__ out_ray, float* __restrict__ out_t) {
-    const uint32_t lane = __lane_id();
-    const uint32_t i = first + lane;
-    const bool active = lane < K && i < n_rays && ray_alive[i] != 0;
-    const uint32_t ns = active ? n_ray_steps[i] : 0u;
-    const uint32_t off = active ? ray_offset[i] : 0u;
-    LaneRayState q = lane_ray_state(active, i, B, ori, dir, ray_t, INFINITY);
-    while (__ballot(!q.done) != 0ull) {
-        if (!q.done && !q.ready) {
-            if (!(q.n < ns)) {
-                q.done = true;
-            } else {
-                const float x = q.r.ox + q.t * q.r.dx, y = q.r.oy + q.t * q.r.dy, z = q.r.oz + q.t * q.r.dz;
-                if (!bbox_contains(bbox, x, y, z)) {
-                    // the count pass stops at the box boundary, so every counted
-                    // sample is inside; one outside would be emitted without advancing
-                    out_t[off + q.n] = q.t;
-                    out_ray[off + q.n] = i;
-                    ++q.n;
-                } else {
-                    const int lvl = grid_level_at(g.n_levels, g.inv_res, x, y, z, get_dt(q.t, cone, dt_min, dt_max) * g.level_scale);
-                    if ((g.bits[voxel_morton_index(g.res_f, g.lim, lvl, x, y, z)] >> lvl) & 1u)
-                        q.ready = true;
-                    else
-                        q.t += dt_to_next_voxel(g.res_f, g.inv_res, x, y, z, q.r.dx, q.r.dy, q.r.dz, q.idx, q.idy,
-                                                q.idz, dt_min, lvl);
-                }
-            }
-        }
-        uint64_t rb = __ballot(q.ready);
-        while (rb != 0ull) {
-            const int L = __builtin_ctzll(rb);
-            rb &= rb - 1ull;
-            const MarchRay r = lane_ray(q.r, L);
-            float t = lane_f(q.t, L);
-            uint32_t n = lane_u(q.n, L);
-            const uint32_t nsL = lane_u(ns, L), offL = lane_u(off, L), iL = lane_u(i, L);
-            for (;;) {
-                float t_lane;
-                bool empty;
-                const uint32_t f = occupied_run(g, bbox, r, t, INFINITY, nsL - n, cone, dt_min, dt_max, t_lane, empty);
-                if (f == 0u) break;
-                if (lane < f) {  // one coalesced row of samples
-                    out_t[offL + n + lane] = t_lane;
-                    out_ray[offL + n + lane] = iL;
-                }
-                t = after_run(f, t_lane, cone, dt_min, dt_max);
-                n += f;
-                if (f < 64u || n >= nsL) break;
-            }
-            if ((int)lane == L) {
-                q.t = t;
-                q.n = n;
-                q.ready = false;
-            }
-        }
+template <int G, bool ML>
+TN_DEVICE void march_generate_rays(const MarchGenerateArgs& a, const tn_bbox_t& bbox, const MarchGrid& g,
+                                   const MarchStep& st) {
+    const uint32_t n_threads = gridDim.x * blockDim.x, tid = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t w = tid & ~63u; w / G < a.n_rays; w += n_threads) {
+        const uint32_t i = (w + (tid & 63u)) / G;
+        const bool active = i < a.n_rays && a.alive[i] != 0;
+        const MarchRay r = load_ray(active, i, a.B, a.ori, a.dir);
+        const uint32_t off = active ? a.offset[i] : 0u;
+        march_group<G, ML, false>(active, r, active ? a.t[i] : 0.0f, INFINITY, active ? a.n_steps[i] : 0u, bbox, g, st,
+                                [&](uint32_t n, float t) {
+                                    a.out_t[off + n] = t;
+                                    a.out_ray[off + n] = i;
+                                });
     }
 }
 
@@ -562,20 +456,15 @@ march_generate_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ info, ui
                       const uint32_t* __restrict__ n_ray_steps, uint32_t* __restrict__ out_ray,
                       float* __restrict__ out_t) {
     const uint32_t n_rays = min(info[0], n_rays_max);
-    const uint32_t n_waves = gridDim.x * kMarchWaves;
-    const uint32_t wave = blockIdx.x * kMarchWaves + (threadIdx.x >> 6);
     const MarchGrid g = make_grid(grid);
-    const uint32_t K = rays_per_wave(n_rays, n_waves);
-    if (K == 1) {
-        for (uint32_t i = wave; i < n_rays; i += n_waves) {
-            if (ray_alive[i])
-                march_generate_ray(i, B, bbox, g, dt_min, dt_max, cone, ori, dir, ray_t, ray_offset, n_ray_steps,
-                                   out_ray, out_t);
-        }
+    const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
+    const MarchGenerateArgs a = {n_rays, B, ori, dir, ray_t, ray_offset, n_ray_steps, ray_alive, out_ray, out_t};
+    if (grid.n_levels == 1) {
+        if (n_rays <= kGroup16Rays) march_generate_rays<16, false>(a, bbox, g, st);
+        else march_generate_rays<8, false>(a, bbox, g, st);
     } else {
-        for (uint32_t first = wave * K; first < n_rays; first += n_waves * K)
-            march_generate_lanes(first, K, n_rays, B, bbox, g, dt_min, dt_max, cone, ori, dir, ray_t, ray_offset,
-                                 ray_alive, n_ray_steps, out_ray, out_t);
+        if (n_rays <= kGroup16Rays) march_generate_rays<16, true>(a, bbox, g, st);
+        else march_generate_rays<8, true>(a, bbox, g, st);
     }
 }
 
