@@ -34,29 +34,59 @@ struct HashCorners {
     uint32_t gx, gy, gz;  // the cell (its lowest corner)
 };
 
-TN_DEVICE void hash_corners(const tn_hashgrid_t& g, int l, float px, float py, float pz, HashCorners& hc) {
+// Level-relative entries of the eight corners of cell (gx, gy, gz); corner c
+// adds (c & 1, c / 2 & 1, c / 4). The level is the same for a whole workgroup,
+// so whether it is dense is one scalar branch. Dense: the corners lie at fixed
+// distances from the first, and only a cell whose last corner passes the
+// level's end (positions at or beyond the box's far faces) wraps around.
+// Hashed: the neighbour's product is the cell's plus the prime, so two
+// multiplications serve all corners.
+TN_DEVICE void hash_indices(const tn_hashgrid_t& g, int l, uint32_t gx, uint32_t gy, uint32_t gz, uint32_t (&id)[8]) {
+    const uint32_t size = g.level_size[l];
+    if (g.level_dense[l] != 0) {
+        const uint32_t r = g.resolution[l], r2 = r * r, first = gx + gy * r + gz * r2;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) id[c] = first + ((c & 1) ? 1u : 0u) + ((c & 2) ? r : 0u) + ((c & 4) ? r2 : 0u);
+        if (first >= size - (1u + r + r2)) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) id[c] %= size;
+        }
+    } else {  // level sizes are powers of two here
+        const uint32_t y0 = gy * 2654435761u, y1 = y0 + 2654435761u, z0 = gz * 805459861u, z1 = z0 + 805459861u;
+        const uint32_t m = size - 1u;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) id[c] = ((gx + (c & 1)) ^ ((c & 2) ? y1 : y0) ^ ((c & 4) ? z1 : z0)) & m;
+    }
+}
+
+// the cell of a position at level l and the position within it
+TN_DEVICE void hash_cell(const tn_hashgrid_t& g, int l, float px, float py, float pz, uint32_t& gx, uint32_t& gy,
+                         uint32_t& gz, float& fx, float& fy, float& fz) {
     const float s = g.scale[l];
     const float x = px * s + 0.5f, y = py * s + 0.5f, z = pz * s + 0.5f;
     const float fx0 = floorf(x), fy0 = floorf(y), fz0 = floorf(z);
-    const float fx = x - fx0, fy = y - fy0, fz = z - fz0;
-    const uint32_t gx = (uint32_t)(int32_t)fx0, gy = (uint32_t)(int32_t)fy0, gz = (uint32_t)(int32_t)fz0;
-    hc.gx = gx;
-    hc.gy = gy;
-    hc.gz = gz;
-    const uint32_t size = g.level_size[l];
-    const uint32_t off = g.level_offset[l];
-    const bool dense = g.level_dense[l] != 0;
-    const uint32_t r = g.resolution[l];
+    fx = x - fx0;
+    fy = y - fy0;
+    fz = z - fz0;
+    gx = (uint32_t)(int32_t)fx0;
+    gy = (uint32_t)(int32_t)fy0;
+    gz = (uint32_t)(int32_t)fz0;
+}
+
+TN_DEVICE void hash_weights(float fx, float fy, float fz, float (&w)[8]) {
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const uint32_t cx = c & 1, cy = (c >> 1) & 1, cz = (c >> 2) & 1;
-        const uint32_t X = gx + cx, Y = gy + cy, Z = gz + cz;
-        uint32_t id = dense ? (X + Y * r + Z * r * r) : ((X * 1u) ^ (Y * 2654435761u) ^ (Z * 805459861u));
-        // level sizes are multiples of 8; hashed levels are powers of two
-        id = dense ? id % size : (id & (size - 1u));
-        hc.idx[c] = off + id;
-        hc.w[c] = (cx ? fx : 1.0f - fx) * (cy ? fy : 1.0f - fy) * (cz ? fz : 1.0f - fz);
-    }
+    for (int c = 0; c < 8; ++c)
+        w[c] = ((c & 1) ? fx : 1.0f - fx) * ((c & 2) ? fy : 1.0f - fy) * ((c & 4) ? fz : 1.0f - fz);
+}
+
+TN_DEVICE void hash_corners(const tn_hashgrid_t& g, int l, float px, float py, float pz, HashCorners& hc) {
+    float fx, fy, fz;
+    hash_cell(g, l, px, py, pz, hc.gx, hc.gy, hc.gz, fx, fy, fz);
+    hash_indices(g, l, hc.gx, hc.gy, hc.gz, hc.idx);
+    hash_weights(fx, fy, fz, hc.w);
+    const uint32_t off = g.level_offset[l];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) hc.idx[c] += off;
 }
 
 template <typename T>
@@ -126,12 +156,12 @@ struct Gather<float> {
 // sets the hash's lowest bit -- so one load of the aligned entry pair
 // holding the lower corner also yields the upper one; the upper corner is
 // loaded on its own only where it lies elsewhere. Same values, and the
-// trilinear sums keep their order. `table` spans `bytes` (< 2^32). The
+// trilinear sums keep their order. `table` (a level's) spans `bytes`. The
 // pairs pass through an empty asm statement once every load is issued:
 // without it the compiler narrows each pair load to the half it sees used
 // and loads the other corner separately again (eight loads).
 template <typename TT>
-TN_DEVICE void gather_corners(const TT* __restrict__ table, uint32_t bytes, const HashCorners& hc,
+TN_DEVICE void gather_corners(const TT* __restrict__ table, uint32_t bytes, const uint32_t (&id)[8],
                               typename Pair<TT>::V (&v)[8]) {
     using V = typename Pair<TT>::V;
     using W = typename Gather<TT>::W;
@@ -140,19 +170,35 @@ TN_DEVICE void gather_corners(const TT* __restrict__ table, uint32_t bytes, cons
     V up[4];
     bool own[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) w[q] = Gather<TT>::pair(r, hc.idx[2 * q]);
+    for (int q = 0; q < 4; ++q) w[q] = Gather<TT>::pair(r, id[2 * q]);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        own[q] = hc.idx[2 * q + 1] != (hc.idx[2 * q] ^ 1u);
-        up[q] = Gather<TT>::one(r, hc.idx[2 * q + 1], own[q]);
+        own[q] = id[2 * q + 1] != (id[2 * q] ^ 1u);
+        up[q] = Gather<TT>::one(r, id[2 * q + 1], own[q]);
     }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         asm volatile("" : "+v"(w[q]));
         const V even = Gather<TT>::even(w[q]), odd = Gather<TT>::odd(w[q]);
-        const bool odd0 = (hc.idx[2 * q] & 1u) != 0u;
+        const bool odd0 = (id[2 * q] & 1u) != 0u;
         v[2 * q] = odd0 ? odd : even;
         v[2 * q + 1] = own[q] ? up[q] : (odd0 ? even : odd);
+    }
+}
+
+// The trilinear sums of the two features, corners in order. fp16 features (an
+// fp16 network's inference) take fused multiply-adds straight from the fp16
+// entries (v_fma_mix_f32, 16 instructions in place of 48); fp32 features, which
+// training runs on, keep the product and the sum rounded one after the other.
+template <typename TT, typename TO>
+TN_DEVICE void hash_interpolate(const float (&w)[8], const typename Pair<TT>::V (&v)[8], float& f0, float& f1) {
+    f0 = 0.0f;
+    f1 = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const float a = Pair<TT>::a(v[c]), b = Pair<TT>::b(v[c]);
+        f0 = sizeof(TO) == 2 ? __builtin_fmaf(w[c], a, f0) : f0 + w[c] * a;
+        f1 = sizeof(TO) == 2 ? __builtin_fmaf(w[c], b, f1) : f1 + w[c] * b;
     }
 }
 
@@ -166,18 +212,15 @@ __global__ void __launch_bounds__(256) hashgrid_fwd_kernel(uint32_t n_max, const
     const int l = l0 + (int)blockIdx.y;
     const uint32_t n = info ? min(info[1], n_max) : n_max;
     if (i >= n) return;
-    HashCorners hc;
-    hash_corners(g, l, pos[i], pos[i + B], pos[i + 2 * (uint64_t)B], hc);
-    // the table's entries (every corner index lies below: levels wrap their indices)
-    const uint32_t n_entries = g.level_offset[g.n_levels - 1] + g.level_size[g.n_levels - 1];
+    uint32_t gx, gy, gz, id[8];
+    float fx, fy, fz, w[8];
+    hash_cell(g, l, pos[i], pos[i + B], pos[i + 2 * (uint64_t)B], gx, gy, gz, fx, fy, fz);
+    hash_indices(g, l, gx, gy, gz, id);
     typename Pair<TT>::V v[8];
-    gather_corners<TT>(table, n_entries * (uint32_t)(2 * sizeof(TT)), hc, v);
-    float f0 = 0.0f, f1 = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        f0 += hc.w[c] * Pair<TT>::a(v[c]);
-        f1 += hc.w[c] * Pair<TT>::b(v[c]);
-    }
+    gather_corners<TT>(table + 2 * (uint64_t)g.level_offset[l], g.level_size[l] * (uint32_t)(2 * sizeof(TT)), id, v);
+    hash_weights(fx, fy, fz, w);
+    float f0, f1;
+    hash_interpolate<TT, TO>(w, v, f0, f1);
     out[(uint64_t)(2 * l) * OB + i] = (TO)f0;
     out[(uint64_t)(2 * l + 1) * OB + i] = (TO)f1;
 }
@@ -207,13 +250,11 @@ __global__ void __launch_bounds__(kHfLdsThreads) hashgrid_fwd_lds_kernel(
         for (int l = 0; l < Ls; ++l) {
             HashCorners hc;
             hash_corners(g, l, px, py, pz, hc);
-            float f0 = 0.0f, f1 = 0.0f;
+            typename Pair<TT>::V v[8];
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const typename Pair<TT>::V v = st[hc.idx[c]];
-                f0 += hc.w[c] * Pair<TT>::a(v);
-                f1 += hc.w[c] * Pair<TT>::b(v);
-            }
+            for (int c = 0; c < 8; ++c) v[c] = st[hc.idx[c]];
+            float f0, f1;
+            hash_interpolate<TT, TO>(hc.w, v, f0, f1);
             out[(uint64_t)(2 * l) * OB + i] = (TO)f0;
             out[(uint64_t)(2 * l + 1) * OB + i] = (TO)f1;
         }
