@@ -10,8 +10,7 @@
 // modulo the level size. The table is entry-major: entry e's F features are
 // contiguous. Features are written feature-major, out[(l*F+f)*stride + i].
 //
-// Launch shape. Forward: one thread per (sample, level), blockIdx.y = level,
-// so the blocks in flight gather from one level's table at a time. Backward:
+// Launch shape. Forward: hashgrid_fwd_kernel. Backward without a workspace:
 // two threads per (sample, level), one per feature, in a 1-D grid whose
 // block b serves level b % L and sample chunk b / L; workgroups go to the 8
 // XCDs round-robin, so with L = 16 each XCD scatters into two levels'
@@ -161,30 +160,33 @@ struct Gather<float> {
 // without it the compiler narrows each pair load to the half it sees used
 // and loads the other corner separately again (eight loads).
 template <typename TT>
-TN_DEVICE void gather_corners(const TT* __restrict__ table, uint32_t bytes, const uint32_t (&id)[8],
-                              typename Pair<TT>::V (&v)[8]) {
+struct Corners {
     using V = typename Pair<TT>::V;
-    using W = typename Gather<TT>::W;
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<TT*>(table), 0, (int)bytes, 0x00020000);
-    W w[4];
+    typename Gather<TT>::W w[4];
     V up[4];
-    bool own[4];
+    bool own[4], odd[4];
+
+    TN_DEVICE void load(const TT* __restrict__ table, uint32_t bytes, const uint32_t (&id)[8]) {
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<TT*>(table), 0, (int)bytes, 0x00020000);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) w[q] = Gather<TT>::pair(r, id[2 * q]);
+        for (int q = 0; q < 4; ++q) w[q] = Gather<TT>::pair(r, id[2 * q]);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        own[q] = id[2 * q + 1] != (id[2 * q] ^ 1u);
-        up[q] = Gather<TT>::one(r, id[2 * q + 1], own[q]);
+        for (int q = 0; q < 4; ++q) {
+            own[q] = id[2 * q + 1] != (id[2 * q] ^ 1u);
+            odd[q] = (id[2 * q] & 1u) != 0u;
+            up[q] = Gather<TT>::one(r, id[2 * q + 1], own[q]);
+        }
     }
+    TN_DEVICE void get(V (&v)[8]) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        asm volatile("" : "+v"(w[q]));
-        const V even = Gather<TT>::even(w[q]), odd = Gather<TT>::odd(w[q]);
-        const bool odd0 = (id[2 * q] & 1u) != 0u;
-        v[2 * q] = odd0 ? odd : even;
-        v[2 * q + 1] = own[q] ? up[q] : (odd0 ? even : odd);
+        for (int q = 0; q < 4; ++q) {
+            asm volatile("" : "+v"(w[q]));
+            const V lo = Gather<TT>::even(w[q]), hi = Gather<TT>::odd(w[q]);
+            v[2 * q] = odd[q] ? hi : lo;
+            v[2 * q + 1] = own[q] ? up[q] : (odd[q] ? lo : hi);
+        }
     }
-}
+};
 
 // The trilinear sums of the two features, corners in order. fp16 features (an
 // fp16 network's inference) take fused multiply-adds straight from the fp16
@@ -202,27 +204,50 @@ TN_DEVICE void hash_interpolate(const float (&w)[8], const typename Pair<TT>::V 
     }
 }
 
-// Levels [l0, l0 + gridDim.y) gathered from global memory.
+// Levels [l0, L) gathered from global memory, two per thread: the y-th finest
+// and the y-th coarsest. What bounds the fine levels is the rate of the
+// XCD's L2 (every corner row of every sample is a line of its own: 264 G
+// lines/s over the chip, 2.3 cycles per line and CU), what bounds the coarse
+// ones is instructions; in one thread the one hides behind the other, and the
+// position is read once for both (262,144 samples 55.6 -> 50.0 us, 4 M
+// samples to fp16 features 673 -> 568 us against one level per thread with
+// levels in turn). Block b takes pair b / chunks, or with
+// `by_xcd` pair b % pairs: workgroups go to the 8 XCDs in turn, so with 16
+// levels each XCD then works on two levels' tables only and reads 3 MB of the
+// table instead of all 24.
 template <typename TT, typename TO>
 __global__ void __launch_bounds__(256) hashgrid_fwd_kernel(uint32_t n_max, const uint32_t* __restrict__ info,
                                                            uint32_t B, uint32_t OB, tn_hashgrid_t g,
                                                            const float* __restrict__ pos, const TT* __restrict__ table,
-                                                           TO* __restrict__ out, int l0) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int l = l0 + (int)blockIdx.y;
+                                                           TO* __restrict__ out, int l0, uint32_t chunks, int by_xcd) {
+    const uint32_t pairs = ((uint32_t)(g.n_levels - l0) + 1u) / 2u;
+    const uint32_t y = by_xcd ? blockIdx.x % pairs : blockIdx.x / chunks;
+    const uint32_t i = (by_xcd ? blockIdx.x / pairs : blockIdx.x % chunks) * blockDim.x + threadIdx.x;
+    const int l[2] = {g.n_levels - 1 - (int)y, l0 + (int)y};
     const uint32_t n = info ? min(info[1], n_max) : n_max;
     if (i >= n) return;
-    uint32_t gx, gy, gz, id[8];
-    float fx, fy, fz, w[8];
-    hash_cell(g, l, pos[i], pos[i + B], pos[i + 2 * (uint64_t)B], gx, gy, gz, fx, fy, fz);
-    hash_indices(g, l, gx, gy, gz, id);
-    typename Pair<TT>::V v[8];
-    gather_corners<TT>(table + 2 * (uint64_t)g.level_offset[l], g.level_size[l] * (uint32_t)(2 * sizeof(TT)), id, v);
-    hash_weights(fx, fy, fz, w);
-    float f0, f1;
-    hash_interpolate<TT, TO>(w, v, f0, f1);
-    out[(uint64_t)(2 * l) * OB + i] = (TO)f0;
-    out[(uint64_t)(2 * l + 1) * OB + i] = (TO)f1;
+    const float px = pos[i], py = pos[i + B], pz = pos[i + 2 * (uint64_t)B];
+    float fx[2], fy[2], fz[2];
+    Corners<TT> c[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        uint32_t gx, gy, gz, id[8];
+        hash_cell(g, l[k], px, py, pz, gx, gy, gz, fx[k], fy[k], fz[k]);
+        hash_indices(g, l[k], gx, gy, gz, id);
+        c[k].load(table + 2 * (uint64_t)g.level_offset[l[k]], g.level_size[l[k]] * (uint32_t)(2 * sizeof(TT)), id);
+    }
+#pragma unroll
+    for (int k = 1; k >= 0; --k) {  // the coarse level's entries arrive first
+        if (k == 1 && l[0] == l[1]) continue;  // the middle of an odd number of levels
+        float w[8];
+        typename Pair<TT>::V v[8];
+        hash_weights(fx[k], fy[k], fz[k], w);
+        c[k].get(v);
+        float f0, f1;
+        hash_interpolate<TT, TO>(w, v, f0, f1);
+        out[(uint64_t)(2 * l[k]) * OB + i] = (TO)f0;
+        out[(uint64_t)(2 * l[k] + 1) * OB + i] = (TO)f1;
+    }
 }
 
 // The coarse dense levels [0, Ls) from a copy of their tables in LDS. Their
@@ -260,6 +285,13 @@ __global__ void __launch_bounds__(kHfLdsThreads) hashgrid_fwd_lds_kernel(
         }
     }
 }
+
+// Samples up to which the encoding gives each XCD two levels (hashgrid_fwd_kernel).
+// fp16 features, us, all XCDs on a pair of levels at a time / a pair per XCD:
+// 16,384 samples 7.3 / 6.9, 65,536 19.4 / 15.3, 262,144 48.0 / 50.9, 4 M 568 /
+// 735: beyond about 200,000 samples reading a table eight times costs less
+// than waiting for the XCD with the finest level.
+constexpr uint32_t kHfByXcdSamples = 1u << 17;
 
 // Levels staged in LDS: the longest prefix of dense levels, at most `want`,
 // whose entries (entry_bytes each) fit kHfLdsBytes; 0 when the table is not
@@ -1374,19 +1406,20 @@ extern "C" int tn_hashgrid_forward(int table_dtype, int feat_dtype, uint32_t n_m
                 static_cast<float*>(features), Ls, stage);
         }
     }
-    const dim3 blocks(blocks_for(n_max, tb), grid.n_levels - Ls);
+    const unsigned chunks = blocks_for(n_max, tb), blocks = chunks * (unsigned)((grid.n_levels - Ls + 1) / 2);
+    const int by_xcd = n_max <= kHfByXcdSamples ? 1 : 0;
     if (table_dtype == 0)
         hashgrid_fwd_kernel<float, float><<<blocks, tb, 0, stream>>>(n_max, info, stride, out_stride, grid, pos,
                                                                       static_cast<const float*>(table),
-                                                                      static_cast<float*>(features), Ls);
+                                                                      static_cast<float*>(features), Ls, chunks, by_xcd);
     else if (feat_dtype == 1)
         hashgrid_fwd_kernel<_Float16, _Float16><<<blocks, tb, 0, stream>>>(
             n_max, info, stride, out_stride, grid, pos, static_cast<const _Float16*>(table),
-            static_cast<_Float16*>(features), Ls);
+            static_cast<_Float16*>(features), Ls, chunks, by_xcd);
     else
         hashgrid_fwd_kernel<_Float16, float><<<blocks, tb, 0, stream>>>(n_max, info, stride, out_stride, grid, pos,
                                                                          static_cast<const _Float16*>(table),
-                                                                         static_cast<float*>(features), Ls);
+                                                                         static_cast<float*>(features), Ls, chunks, by_xcd);
     TN_CHECK_LAUNCH();
     return TN_OK;
 }
