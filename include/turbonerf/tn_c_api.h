@@ -254,6 +254,17 @@ int tn_hashgrid_backward_binned(int dfeat_dtype, uint32_t n_max, const uint32_t*
     uint32_t dfeat_stride, tn_hashgrid_t grid, const float* pos, const void* dfeat, float* dtable,
     void* workspace, size_t workspace_bytes, tn_stream_t stream);
 
+/* The same sort with every contribution kept in fp32 (10-byte records instead
+ * of 8): the accuracy of tn_hashgrid_backward, and a result that does not
+ * depend on the order of the sums. Same replacement (reference
+ * src/core/nerf-network.cu:760). The workspace (256-byte aligned,
+ * tn_hashgrid_backward_sorted_bytes, 0 = layout beyond the bin limits) is
+ * scratch; without it the atomic kernel runs. dtable is 8-byte aligned. */
+size_t tn_hashgrid_backward_sorted_bytes(uint32_t n_max, tn_hashgrid_t grid);
+int tn_hashgrid_backward_sorted(int dfeat_dtype, uint32_t n_max, const uint32_t* info, uint32_t stride,
+    uint32_t dfeat_stride, tn_hashgrid_t grid, const float* pos, const void* dfeat, float* dtable,
+    void* workspace, size_t workspace_bytes, tn_stream_t stream);
+
 /* tn_hashgrid_backward_binned in two calls (same result bit for bit), for a
  * caller that has the positions before the gradients (the reference's
  * trainer does: the batch's sample positions at trainer.cu:184-216, the

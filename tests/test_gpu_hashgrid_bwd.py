@@ -421,3 +421,50 @@ def test_binned_vs_fp64_central_differences(cuda):
         worst = max(worst, e)
         assert e < 1e-5, (l, e)
     print(f"[hash bwd fd] {n} samples on 64 rays, worst level rel err {worst:.2e}", flush=True)
+
+
+@pytest.mark.parametrize("n,log2_T", [(1, 12), (300, 19), (10_000, 12), (30_000, 19), (70_001, 21)])
+def test_sorted_fp32_records(cuda, n, log2_T):
+    """The sort with fp32 records (through the autograd layer's rule, on both
+    sides of it, and called directly) against float64: no further off than
+    the atomic scatter-add by more than the fixed-point rounding, added to a
+    non-zero table, the same bits from run to run, and a non-finite gradient
+    reaching the entries it belongs to."""
+    import torch
+
+    from turbonerf_amd import _capi, ops
+
+    g = ops.hashgrid_layout(log2_T=log2_T)
+    rng = np.random.default_rng(n)
+    pos = _rays(rng, max(1, n // 100), 100, 0.0011)[:, :n]
+    n = pos.shape[1]
+    dfeat = (rng.normal(size=(32, n)) * 10.0 ** rng.uniform(-4, 2, (32, 1))).astype(np.float32)
+    base = rng.normal(size=g.n_params).astype(np.float32)
+    ref = _oracle_bwd(g, pos, dfeat)
+    p, d = torch.from_numpy(np.ascontiguousarray(pos)).cuda(), torch.from_numpy(dfeat).cuda()
+    print(f"[hashgrid sorted] n {n} log2_T {log2_T}", flush=True)
+    nb = _capi.query("tn_hashgrid_backward_sorted_bytes", n, g)
+    assert nb > 0
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+
+    def direct(d):
+        t = torch.zeros(g.n_params, device="cuda")
+        _capi.call("tn_hashgrid_backward_sorted", 0, n, None, n, n, g, p.data_ptr(), d.data_ptr(), t.data_ptr(),
+                   ws.data_ptr(), nb, _capi.stream_ptr())
+        return t
+
+    atomic = torch.zeros(g.n_params, device="cuda")
+    ops.hashgrid_backward(g, n, p, n, d, atomic)
+    t = direct(d)
+    e_s, e_a = norm_rel(t.cpu().numpy(), ref), norm_rel(atomic.cpu().numpy(), ref)
+    print(f"[hashgrid sorted] error {e_s:.2e}, atomic {e_a:.2e}", flush=True)
+    assert e_s <= e_a + 1e-7  # fp32 sums of runs, then exact sums rounded once
+    assert torch.equal(t, direct(d))
+    acc = torch.from_numpy(base).cuda()
+    ops.hashgrid_backward_sorted(g, n, p, n, d, acc)
+    assert norm_rel(acc.cpu().numpy() - base.astype(np.float64), ref) <= 1e-6 + 1e-7 * np.linalg.norm(base) / np.linalg.norm(ref)
+    bad = d.clone()
+    bad[5, n // 2] = float("inf")
+    ti, ta = direct(bad).cpu().numpy(), torch.zeros(g.n_params, device="cuda")
+    ops.hashgrid_backward(g, n, p, n, bad, ta)
+    assert np.array_equal(np.isfinite(ti), np.isfinite(ta.cpu().numpy()))

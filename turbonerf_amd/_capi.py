@@ -171,6 +171,8 @@ _SIGS: dict[str, tuple] = {
     "tn_hashgrid_backward": (C.c_int, [C.c_int, u32, vp, u32, u32, HashGrid, vp, vp, vp, vp]),
     "tn_hashgrid_backward_workspace_bytes": (C.c_size_t, [u32, HashGrid]),
     "tn_hashgrid_backward_binned": (C.c_int, [C.c_int, u32, vp, u32, u32, HashGrid, vp, vp, vp, vp, C.c_size_t, vp]),
+    "tn_hashgrid_backward_sorted_bytes": (C.c_size_t, [u32, HashGrid]),
+    "tn_hashgrid_backward_sorted": (C.c_int, [C.c_int, u32, vp, u32, u32, HashGrid, vp, vp, vp, vp, C.c_size_t, vp]),
     "tn_hashgrid_backward_plan_bytes": (C.c_size_t, [u32, HashGrid]),
     "tn_hashgrid_backward_work_bytes": (C.c_size_t, [u32, HashGrid]),
     "tn_hashgrid_backward_plan": (C.c_int, [u32, vp, u32, HashGrid, vp, vp, C.c_size_t, vp]),

@@ -57,7 +57,7 @@ class HashGridEncoding(torch.autograd.Function):
         g = _contig(grad_feat)
         if g.dtype not in (torch.float32, torch.float16):
             g = g.float()
-        ops.hashgrid_backward(ctx.grid, n, pos, n, g, dtable)
+        ops.hashgrid_backward_sorted(ctx.grid, n, pos, n, g, dtable)
         return dtable.to(ctx.table_dtype), None, None
 
 

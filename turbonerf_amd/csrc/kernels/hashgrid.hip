@@ -391,7 +391,7 @@ __global__ void __launch_bounds__(256) hashgrid_bwd_kernel(uint32_t n_max, const
 // records, the scale 2^S with S = 62 - E - ceil(log2(m + 1)) cannot overflow,
 // and the sum of the records is exact up to the rounding of each value to a
 // multiple of 2^-S (relative 2^-38 of the bin's largest value or better);
-// each record carries its value to 17 significant bits (HbRecord). Blocks of count and
+// each record carries its value to 17 significant bits (HbRec8) or whole (HbRec10). Blocks of count and
 // scatter work on one level each: block b serves level b % L and the
 // contiguous 256-sample chunks [j, j + 1) * chunk_blocks, j = b / L, so the
 // records of a range of samples can be scattered on their own (the slots of
@@ -417,16 +417,16 @@ struct HbPlan {
     uint64_t cap;         // record capacity: n_max * L * 8
 };
 
-// A record is one contribution to both features of one entry of a bin, in 8
-// bytes: each value rounded to 17 significant bits (relative error at most
-// 2^-18, far below the fp16 gradient accumulation of the reference) and the
-// bin-relative 12-bit entry index in the freed low mantissa bits, its bits
-// 0..5 in the first value's and 6..11 in the second's. (The scatter's write
-// and the accumulation's read of the records bound both passes; 12-byte
-// records took 1.5 times as long.)
-struct HbRecord {
-    uint32_t a, b;
-};
+// A record is one contribution to both features of one entry of a bin. The
+// trainer's are 8 bytes (HbRec8): each value rounded to 17 significant bits
+// (relative error at most 2^-18, far below the fp16 gradient accumulation of
+// the reference) and the bin-relative 12-bit entry index in the freed low
+// mantissa bits, its bits 0..5 in the first value's and 6..11 in the second's.
+// (The scatter's write and the accumulation's read of the records bound both
+// passes; 12-byte records took 1.5 times as long.) Callers that ask for fp32
+// contributions get HbRec10: both values as they are and the entry in 16 bits,
+// in arrays of their own. All passes, plan included, on 262,144 samples along
+// rays: 172 us with HbRec8, 221 us with HbRec10; 754 us by atomics.
 
 // v rounded to 17 significant bits (half away from zero; a carry may raise the
 // exponent, up to inf), low 6 bits cleared; inf and NaN keep their pattern
@@ -435,10 +435,30 @@ TN_DEVICE uint32_t hb_round17(float v) {
     if ((u & 0x7F800000u) == 0x7F800000u) return u & ~63u;
     return (u + 32u) & ~63u;
 }
-TN_DEVICE HbRecord hb_pack(uint32_t e, uint32_t r0, uint32_t r1) { return HbRecord{r0 | (e & 63u), r1 | (e >> 6)}; }
-TN_DEVICE uint32_t hb_entry(const HbRecord& r) { return (r.a & 63u) | ((r.b & 63u) << 6); }
-TN_DEVICE float hb_v0(const HbRecord& r) { return __uint_as_float(r.a & ~63u); }
-TN_DEVICE float hb_v1(const HbRecord& r) { return __uint_as_float(r.b & ~63u); }
+
+struct HbRec8 {
+    static constexpr bool kEntryArray = false;
+    static constexpr size_t kBytes = 8;
+    TN_DEVICE static uint32_t value(float v) { return hb_round17(v); }
+    TN_DEVICE static uint2 pack(uint32_t e, uint32_t r0, uint32_t r1) { return make_uint2(r0 | (e & 63u), r1 | (e >> 6)); }
+    TN_DEVICE static uint32_t entry(uint2 r, uint32_t) { return (r.x & 63u) | ((r.y & 63u) << 6); }
+    TN_DEVICE static float v0(uint2 r) { return __uint_as_float(r.x & ~63u); }
+    TN_DEVICE static float v1(uint2 r) { return __uint_as_float(r.y & ~63u); }
+};
+struct HbRec10 {
+    static constexpr bool kEntryArray = true;
+    static constexpr size_t kBytes = 10;
+    TN_DEVICE static uint32_t value(float v) { return __float_as_uint(v); }
+    TN_DEVICE static uint2 pack(uint32_t, uint32_t r0, uint32_t r1) { return make_uint2(r0, r1); }
+    TN_DEVICE static uint32_t entry(uint2, uint32_t e) { return e; }
+    TN_DEVICE static float v0(uint2 r) { return __uint_as_float(r.x); }
+    TN_DEVICE static float v1(uint2 r) { return __uint_as_float(r.y); }
+};
+// the records of a work area: `cap` values, then (HbRec10) as many entries
+struct HbRecords {
+    uint2* val;
+    uint16_t* ent;
+};
 
 // One sample per lane, level l: the eight corner contributions of both
 // features, with runs of consecutive lanes on one entry summed into the run's
@@ -470,13 +490,78 @@ TN_DEVICE void seg_step16(float (&a0)[8], float (&a1)[8], int key) {
     }
 }
 
-TN_DEVICE void seg_sum16(float (&a0)[8], float (&a1)[8], int key) {
-    seg_step16<0x111, 0xF>(a0, a1, key);
-    seg_step16<0x112, 0xF>(a0, a1, key);
-    seg_step16<0x114, 0xF>(a0, a1, key);
-    seg_step16<0x118, 0xF>(a0, a1, key);
-    seg_step16<0x142, 0xA>(a0, a1, key);
-    seg_step16<0x143, 0xC>(a0, a1, key);
+// The same step for finite values of less than 2^100: take becomes a factor
+// of 1 or 0 of a fused multiply-add whose product operand is the shifted
+// value, one instruction per value (exact: the factor is 1 or 0). Lanes whose
+// source is outside the row or in a row not selected are not written. The two
+// wait states before a DPP read of a fresh register are part of the block.
+#define TN_SEG_FMAC(CTRL, ROWS)                                                                                  \
+    asm("s_nop 1\n\t"                                                                                            \
+        "v_fmac_f32_dpp %0, %0, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %1, %1, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %2, %2, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %3, %3, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %4, %4, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %5, %5, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %6, %6, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %7, %7, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %8, %8, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %9, %9, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                                \
+        "v_fmac_f32_dpp %10, %10, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                              \
+        "v_fmac_f32_dpp %11, %11, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                              \
+        "v_fmac_f32_dpp %12, %12, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                              \
+        "v_fmac_f32_dpp %13, %13, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                              \
+        "v_fmac_f32_dpp %14, %14, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf\n\t"                              \
+        "v_fmac_f32_dpp %15, %15, %16 " CTRL " row_mask:" ROWS " bank_mask:0xf"                                  \
+        : "+v"(a0[0]), "+v"(a0[1]), "+v"(a0[2]), "+v"(a0[3]), "+v"(a0[4]), "+v"(a0[5]), "+v"(a0[6]),             \
+          "+v"(a0[7]), "+v"(a1[0]), "+v"(a1[1]), "+v"(a1[2]), "+v"(a1[3]), "+v"(a1[4]), "+v"(a1[5]),             \
+          "+v"(a1[6]), "+v"(a1[7])                                                                               \
+        : "v"(f))
+
+template <int CTRL, int ROWS>
+TN_DEVICE float seg_factor(int key) {
+    return __builtin_amdgcn_update_dpp(0, key, CTRL, ROWS, 0xF, false) == key ? 1.0f : 0.0f;
+}
+
+// Segmented sums over the runs of `heads` (bit i: lane i starts a run). The
+// scatter is bound by its vector instructions, and these sums were 222 of 625
+// per wave and level; with these, and one LDS counter and maximum for the two
+// x neighbours, it went from 87 to 71 us at 262,144 samples. A step
+// that no run is long enough for, or that crosses into rows no run crosses
+// into, is left out: on fine levels runs are of two or three samples.
+TN_DEVICE void seg_sum16(float (&a0)[8], float (&a1)[8], int key, uint64_t heads, bool small) {
+    if (!small) {
+        seg_step16<0x111, 0xF>(a0, a1, key);
+        seg_step16<0x112, 0xF>(a0, a1, key);
+        seg_step16<0x114, 0xF>(a0, a1, key);
+        seg_step16<0x118, 0xF>(a0, a1, key);
+        seg_step16<0x142, 0xA>(a0, a1, key);
+        seg_step16<0x143, 0xC>(a0, a1, key);
+        return;
+    }
+    const uint64_t n1 = ~heads, n2 = n1 & (n1 >> 1), n4 = n2 & (n2 >> 2), n8 = n4 & (n4 >> 4);
+    float f = seg_factor<0x111, 0xF>(key);
+    TN_SEG_FMAC("row_shr:1", "0xf");
+    if (n2 != 0ull) {
+        f = seg_factor<0x112, 0xF>(key);
+        TN_SEG_FMAC("row_shr:2", "0xf");
+    }
+    if (n4 != 0ull) {
+        f = seg_factor<0x114, 0xF>(key);
+        TN_SEG_FMAC("row_shr:4", "0xf");
+    }
+    if (n8 != 0ull) {
+        f = seg_factor<0x118, 0xF>(key);
+        TN_SEG_FMAC("row_shr:8", "0xf");
+    }
+    if ((n1 & ((1ull << 16) | (1ull << 48))) != 0ull) {
+        f = seg_factor<0x142, 0xA>(key);
+        TN_SEG_FMAC("row_bcast:15", "0xa");
+    }
+    if ((n1 & (1ull << 32)) != 0ull) {
+        f = seg_factor<0x143, 0xC>(key);
+        TN_SEG_FMAC("row_bcast:31", "0xc");
+    }
 }
 
 // Corner entries and weights of an active sample i at level l, and the mask
@@ -561,7 +646,9 @@ TN_DEVICE void hb_corners(const tn_hashgrid_t& g, int l, bool active, const HbIn
     }
     if (hm != ~0ull) {
         const uint64_t le = lane == 63 ? ~0ull : ((1ull << (lane + 1)) - 1ull);
-        seg_sum16(a0, a1, __builtin_popcountll(hm & le));
+        constexpr float kSmall = 1.2676506e30f;  // 2^100: sums of a wave's values stay finite
+        const bool large = !(fabsf(v.g0) < kSmall) || !(fabsf(v.g1) < kSmall);
+        seg_sum16(a0, a1, __builtin_popcountll(hm & le), hm, __ballot(large) == 0ull);
     }
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
@@ -603,7 +690,12 @@ __global__ void __launch_bounds__(256) hashgrid_bwd_count_kernel(uint32_t n_max,
         hb_cells(g, l, v.x, v.y, v.z, active, c8, hm);
         if (hb_emits(active, hm)) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) atomicAdd(&hist[(c8.idx[k] - g.level_offset[l]) >> kHbBinLog], 1u);
+            for (int k = 0; k < 8; k += 2) {  // the neighbours in x, nearly always in one bin
+                const uint32_t b0 = (c8.idx[k] - g.level_offset[l]) >> kHbBinLog;
+                const uint32_t b1 = (c8.idx[k + 1] - g.level_offset[l]) >> kHbBinLog;
+                atomicAdd(&hist[b0], b0 == b1 ? 2u : 1u);
+                if (b0 != b1) atomicAdd(&hist[b1], 1u);
+            }
         }
     }
     __syncthreads();
@@ -732,11 +824,11 @@ __global__ void __launch_bounds__(1024) hashgrid_bwd_scan_kernel(HbPlan p, const
 constexpr uint32_t kHbScatterThreads = 256;
 constexpr uint32_t kHbChunkRecords = 8 * kHbScatterThreads;
 static_assert(kHbMaxLevelBins <= 2 * kHbScatterThreads, "two bins per thread in the chunk scan");
-template <typename TG>
+template <typename TG, class Rec>
 __global__ void __launch_bounds__(kHbScatterThreads) hashgrid_bwd_scatter_kernel(
     uint32_t n_max, const uint32_t* __restrict__ info, uint32_t B, uint32_t GB, tn_hashgrid_t g, HbPlan p,
     const float* __restrict__ pos, const TG* __restrict__ dfeat, const uint32_t* __restrict__ offsets,
-    const uint32_t* __restrict__ start, uint32_t* __restrict__ binmax, HbRecord* __restrict__ rec, uint32_t l0,
+    const uint32_t* __restrict__ start, uint32_t* __restrict__ binmax, HbRecords rec, uint32_t l0,
     uint32_t Lg, uint32_t j0) {
     // cur: the bin's next global slot; cnt: the chunk's records per bin;
     // lstart: the chunk's first LDS place of the bin; gdel: global slot minus
@@ -745,6 +837,7 @@ __global__ void __launch_bounds__(kHbScatterThreads) hashgrid_bwd_scatter_kernel
     __shared__ uint32_t lstart[kHbMaxLevelBins], gdel[kHbMaxLevelBins];
     __shared__ uint2 srec[kHbChunkRecords];
     __shared__ uint32_t sslot[kHbChunkRecords];
+    __shared__ uint16_t sent[Rec::kEntryArray ? kHbChunkRecords : 1];
     __shared__ uint32_t wtot[kHbScatterThreads / 64];
     const uint32_t L = (uint32_t)g.n_levels;
     // this launch covers levels [l0, l0 + Lg) and count blocks j >= j0;
@@ -772,13 +865,26 @@ __global__ void __launch_bounds__(kHbScatterThreads) hashgrid_bwd_scatter_kernel
         uint32_t bin[8], rank[8], r0[8], r1[8];
         if (hc.emit) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                bin[k] = (hc.idx[k] - off) >> kHbBinLog;
-                rank[k] = atomicAdd(&cnt[bin[k]], 1u);
-                r0[k] = hb_round17(hc.a0[k]);
-                r1[k] = hb_round17(hc.a1[k]);
-                const uint32_t m = max(r0[k] & 0x7FFFFFFFu, r1[k] & 0x7FFFFFFFu);  // of the rounded values
-                if (m != 0u) atomicMax(&bmax[bin[k]], m);
+            for (int k = 0; k < 8; k += 2) {
+                // the neighbours in x, nearly always in one bin: one rank and
+                // one maximum for both
+                uint32_t m[2];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    bin[k + h] = (hc.idx[k + h] - off) >> kHbBinLog;
+                    r0[k + h] = Rec::value(hc.a0[k + h]);
+                    r1[k + h] = Rec::value(hc.a1[k + h]);
+                    m[h] = max(r0[k + h] & 0x7FFFFFFFu, r1[k + h] & 0x7FFFFFFFu);  // of the recorded values
+                }
+                const bool one = bin[k] == bin[k + 1];
+                rank[k] = atomicAdd(&cnt[bin[k]], one ? 2u : 1u);
+                rank[k + 1] = rank[k] + 1u;
+                const uint32_t m0 = one ? max(m[0], m[1]) : m[0];
+                if (m0 != 0u) atomicMax(&bmax[bin[k]], m0);
+                if (!one) {
+                    rank[k + 1] = atomicAdd(&cnt[bin[k + 1]], 1u);
+                    if (m[1] != 0u) atomicMax(&bmax[bin[k + 1]], m[1]);
+                }
             }
         }
         __syncthreads();
@@ -817,17 +923,20 @@ __global__ void __launch_bounds__(kHbScatterThreads) hashgrid_bwd_scatter_kernel
         if (hc.emit) {
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                const uint32_t q = lstart[bin[k]] + rank[k];
-                const HbRecord r = hb_pack((hc.idx[k] - off) & (kHbBinEntries - 1u), r0[k], r1[k]);
-                srec[q] = make_uint2(r.a, r.b);
+                const uint32_t q = lstart[bin[k]] + rank[k], e = (hc.idx[k] - off) & (kHbBinEntries - 1u);
+                srec[q] = Rec::pack(e, r0[k], r1[k]);
                 sslot[q] = q + gdel[bin[k]];
+                if constexpr (Rec::kEntryArray) sent[q] = (uint16_t)e;
             }
         }
         __syncthreads();
         for (uint32_t q = tid; q < total; q += kHbScatterThreads) {
             const uint32_t slot = sslot[q];
             const uint2 r = srec[q];
-            if (slot < p.cap) reinterpret_cast<uint2*>(rec)[slot] = r;  // rec is 8-byte aligned
+            if (slot < p.cap) {
+                rec.val[slot] = r;
+                if constexpr (Rec::kEntryArray) rec.ent[slot] = sent[q];
+            }
         }
     }
     __syncthreads();
@@ -1004,12 +1113,13 @@ TN_DEVICE int hb_scale(uint32_t bits, uint64_t m) {
 // so the result does not depend on the order the blocks run in. A bin
 // holding a non-finite value sums in float and adds into dtable atomically
 // instead, so inf and NaN reach the table.
+template <class Rec>
 __global__ void __launch_bounds__(512) hashgrid_bwd_accumulate_kernel(tn_hashgrid_t g, HbPlan p,
                                                                       const uint32_t* __restrict__ start,
                                                                       const uint32_t* __restrict__ chunk_start,
                                                                       const uint32_t* __restrict__ binmax,
                                                                       const uint32_t* __restrict__ slot_base,
-                                                                      const HbRecord* __restrict__ rec,
+                                                                      HbRecords rec,
                                                                       unsigned long long* __restrict__ slots,
                                                                       float* __restrict__ dtable, uint32_t k_lo,
                                                                       uint32_t k_hi, HbAdam adam) {
@@ -1038,24 +1148,27 @@ __global__ void __launch_bounds__(512) hashgrid_bwd_accumulate_kernel(tn_hashgri
     float* accf = reinterpret_cast<float*>(acc);
     constexpr int kRecUnroll = 8;  // records in flight per lane
     for (uint64_t r = r0 + threadIdx.x; r < r1; r += kRecUnroll * blockDim.x) {
-        HbRecord q[kRecUnroll];
+        uint2 q[kRecUnroll];
+        uint32_t qe[kRecUnroll];
         bool in[kRecUnroll];
 #pragma unroll
         for (int u = 0; u < kRecUnroll; ++u) {
             const uint64_t rr = r + (uint64_t)u * blockDim.x;
             in[u] = rr < r1;
-            q[u] = in[u] ? rec[rr] : HbRecord{0u, 0u};
+            q[u] = in[u] ? rec.val[rr] : make_uint2(0u, 0u);
+            qe[u] = 0u;
+            if constexpr (Rec::kEntryArray) qe[u] = in[u] ? rec.ent[rr] : 0u;
         }
 #pragma unroll
         for (int u = 0; u < kRecUnroll; ++u) {
-            const uint32_t e = hb_entry(q[u]);
+            const uint32_t e = Rec::entry(q[u], qe[u]);
             if (!in[u] || e >= ne) continue;
             if (finite) {
-                atomicAdd(&acc[2 * e], (unsigned long long)hb_fixed(hb_v0(q[u]), S));
-                atomicAdd(&acc[2 * e + 1], (unsigned long long)hb_fixed(hb_v1(q[u]), S));
+                atomicAdd(&acc[2 * e], (unsigned long long)hb_fixed(Rec::v0(q[u]), S));
+                atomicAdd(&acc[2 * e + 1], (unsigned long long)hb_fixed(Rec::v1(q[u]), S));
             } else {
-                atomicAdd(&accf[2 * e], hb_v0(q[u]));
-                atomicAdd(&accf[2 * e + 1], hb_v1(q[u]));
+                atomicAdd(&accf[2 * e], Rec::v0(q[u]));
+                atomicAdd(&accf[2 * e + 1], Rec::v1(q[u]));
             }
         }
     }
@@ -1225,7 +1338,7 @@ struct HbPlanArea {
 struct HbWorkArea {
     uint32_t* binmax;
     unsigned long long* slots;
-    HbRecord* rec;
+    HbRecords rec;
 };
 
 inline size_t hb_align(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1258,19 +1371,25 @@ inline size_t hb_plan_area(const HbPlan& p, void* base, HbPlanArea* pa) {
 }
 
 // work-area bytes, and the carve-up when `base` is given
+template <class Rec = HbRec8>
 inline size_t hb_work_area(const HbPlan& p, void* base, HbWorkArea* wa) {
     HbCarver c{static_cast<unsigned char*>(base)};
     HbWorkArea a;
     a.binmax = reinterpret_cast<uint32_t*>(c.take((size_t)p.n_bins * p.level_blocks * sizeof(uint32_t)));
     a.slots = reinterpret_cast<unsigned long long*>(
         c.take((size_t)p.split_slots * 2 * kHbBinEntries * sizeof(unsigned long long)));
-    a.rec = reinterpret_cast<HbRecord*>(c.take((size_t)p.cap * sizeof(HbRecord)));
+    a.rec.val = reinterpret_cast<uint2*>(c.take((size_t)p.cap * sizeof(uint2)));
+    a.rec.ent = nullptr;
+    if (Rec::kEntryArray) a.rec.ent = reinterpret_cast<uint16_t*>(c.take((size_t)p.cap * sizeof(uint16_t)));
     if (wa) *wa = a;
     return c.off;
 }
 
 // both parts in one buffer (the plan first)
-inline size_t hb_workspace(const HbPlan& p) { return hb_plan_area(p, nullptr, nullptr) + hb_work_area(p, nullptr, nullptr); }
+template <class Rec = HbRec8>
+inline size_t hb_workspace(const HbPlan& p) {
+    return hb_plan_area(p, nullptr, nullptr) + hb_work_area<Rec>(p, nullptr, nullptr);
+}
 
 // (1)-(2b): the plan from the positions
 inline void hashgrid_backward_plan(uint32_t n_max, const uint32_t* info, uint32_t B, const tn_hashgrid_t& g,
@@ -1283,16 +1402,17 @@ inline void hashgrid_backward_plan(uint32_t n_max, const uint32_t* info, uint32_
 }
 
 // (3) for levels [l0, l0 + Lg) and the samples of count blocks [j0, j1)
-template <typename TG>
+template <typename TG, class Rec>
 void hb_scatter(uint32_t n_max, const uint32_t* info, uint32_t B, uint32_t GB, const tn_hashgrid_t& g, const HbPlan& p,
                 const float* pos, const TG* dfeat, const HbPlanArea& pa, const HbWorkArea& wa, uint32_t l0,
                 uint32_t Lg, uint32_t j0, uint32_t j1, hipStream_t stream) {
     if (j1 > j0)
-        hashgrid_bwd_scatter_kernel<TG><<<(j1 - j0) * Lg, kHbScatterThreads, 0, stream>>>(
+        hashgrid_bwd_scatter_kernel<TG, Rec><<<(j1 - j0) * Lg, kHbScatterThreads, 0, stream>>>(
             n_max, info, B, GB, g, p, pos, dfeat, pa.offsets, pa.start, wa.binmax, wa.rec, l0, Lg, j0);
 }
 
 // (4) for levels [l0, l0 + Lg), every record of them scattered
+template <class Rec>
 inline void hb_accumulate(uint32_t n_max, const tn_hashgrid_t& g, const HbPlan& p, float* dtable,
                           const HbPlanArea& pa, const HbWorkArea& wa, uint32_t l0, uint32_t Lg, const HbAdam& adam,
                           hipStream_t stream) {
@@ -1301,7 +1421,7 @@ inline void hb_accumulate(uint32_t n_max, const tn_hashgrid_t& g, const HbPlan& 
     // chunks of the group's bins: at most one per bin plus one per kHbChunk records
     const uint64_t cap_g = (uint64_t)n_max * Lg * 8;
     const uint32_t acc_blocks = (uint32_t)((k_hi - k_lo) + (cap_g + kHbChunk - 1) / kHbChunk);
-    hashgrid_bwd_accumulate_kernel<<<acc_blocks, 512, 0, stream>>>(g, p, pa.start, pa.chunk_start, wa.binmax,
+    hashgrid_bwd_accumulate_kernel<Rec><<<acc_blocks, 512, 0, stream>>>(g, p, pa.start, pa.chunk_start, wa.binmax,
                                                                    pa.slot_base, wa.rec, wa.slots, dtable, k_lo, k_hi,
                                                                    adam);
 }
@@ -1314,7 +1434,7 @@ inline void hb_finish(const tn_hashgrid_t& g, const HbPlan& p, float* dtable, co
 }
 
 // (3)-(5): records, sums and the table update, from the plan and the gradients
-template <typename TG>
+template <typename TG, class Rec = HbRec8>
 void hashgrid_backward_planned(uint32_t n_max, const uint32_t* info, uint32_t B, uint32_t GB, const tn_hashgrid_t& g,
                                const HbPlan& p, const float* pos, const TG* dfeat, float* dtable,
                                const HbPlanArea& pa, const HbWorkArea& wa, hipStream_t stream,
@@ -1326,8 +1446,8 @@ void hashgrid_backward_planned(uint32_t n_max, const uint32_t* info, uint32_t B,
     const uint32_t per = (L + G - 1) / G;
     for (uint32_t l0 = 0; l0 < L; l0 += per) {
         const uint32_t Lg = std::min(per, L - l0);
-        hb_scatter<TG>(n_max, info, B, GB, g, p, pos, dfeat, pa, wa, l0, Lg, 0, p.level_blocks, stream);
-        hb_accumulate(n_max, g, p, dtable, pa, wa, l0, Lg, adam, stream);
+        hb_scatter<TG, Rec>(n_max, info, B, GB, g, p, pos, dfeat, pa, wa, l0, Lg, 0, p.level_blocks, stream);
+        hb_accumulate<Rec>(n_max, g, p, dtable, pa, wa, l0, Lg, adam, stream);
     }
     hb_finish(g, p, dtable, pa, wa, adam, stream);
 }
@@ -1484,6 +1604,43 @@ extern "C" int tn_hashgrid_backward_binned(int dfeat_dtype, uint32_t n_max, cons
     return TN_OK;
 }
 
+// The scatter-add of tn_hashgrid_backward through the same sort with fp32
+// records (each contribution whole, as the atomic kernel adds it), for callers
+// that want its accuracy without its cost; the result does not depend on the
+// order of the sums. A missing or short workspace, or a layout beyond the bin
+// limits, takes the atomic kernel.
+extern "C" size_t tn_hashgrid_backward_sorted_bytes(uint32_t n_max, tn_hashgrid_t grid) {
+    HbPlan p;
+    if (!hb_layout_ok(grid) || n_max == 0 || !hb_plan(grid, n_max, kHbBlocksPerLevel, p)) return 0;
+    return hb_workspace<HbRec10>(p);
+}
+
+extern "C" int tn_hashgrid_backward_sorted(int dfeat_dtype, uint32_t n_max, const uint32_t* info, uint32_t stride,
+                                           uint32_t dfeat_stride, tn_hashgrid_t grid, const float* pos,
+                                           const void* dfeat, float* dtable, void* workspace, size_t workspace_bytes,
+                                           hipStream_t stream) {
+    TN_CHECK_ARG(pos && dfeat && dtable && n_max <= stride && n_max <= dfeat_stride && hb_layout_ok(grid));
+    TN_CHECK_ARG(dfeat_dtype == 0 || dfeat_dtype == 1);
+    if (n_max == 0) return TN_OK;
+    HbPlan p;
+    if (!workspace || !hb_plan(grid, n_max, kHbBlocksPerLevel, p) || workspace_bytes < hb_workspace<HbRec10>(p))
+        return tn_hashgrid_backward(dfeat_dtype, n_max, info, stride, dfeat_stride, grid, pos, dfeat, dtable, stream);
+    TN_CHECK_ARG((reinterpret_cast<uintptr_t>(workspace) & 255) == 0 && (reinterpret_cast<uintptr_t>(dtable) & 7) == 0);
+    HbPlanArea pa;
+    HbWorkArea wa;
+    const size_t plan_bytes = hb_plan_area(p, workspace, &pa);
+    hb_work_area<HbRec10>(p, static_cast<unsigned char*>(workspace) + plan_bytes, &wa);
+    hashgrid_backward_plan(n_max, info, stride, grid, p, pos, pa, stream);
+    if (dfeat_dtype == 0)
+        hashgrid_backward_planned<float, HbRec10>(n_max, info, stride, dfeat_stride, grid, p, pos,
+                                                  static_cast<const float*>(dfeat), dtable, pa, wa, stream);
+    else
+        hashgrid_backward_planned<_Float16, HbRec10>(n_max, info, stride, dfeat_stride, grid, p, pos,
+                                                     static_cast<const _Float16*>(dfeat), dtable, pa, wa, stream);
+    TN_CHECK_LAUNCH();
+    return TN_OK;
+}
+
 // tn_hashgrid_backward_binned in two calls, for callers that know the
 // positions before the gradients: the plan (record counts and offsets per
 // bin, from the positions alone) into `plan`, then the gradient passes into
@@ -1619,10 +1776,10 @@ extern "C" int tn_hashgrid_backward_scatter(int dfeat_dtype, uint32_t n_max, con
     hb_work_area(p, work, &wa);
     const uint32_t L = (uint32_t)grid.n_levels;
     if (dfeat_dtype == 0)
-        hb_scatter<float>(n_max, info, stride, dfeat_stride, grid, p, pos, static_cast<const float*>(dfeat), pa, wa,
+        hb_scatter<float, HbRec8>(n_max, info, stride, dfeat_stride, grid, p, pos, static_cast<const float*>(dfeat), pa, wa,
                           0, L, j0, j1, stream);
     else
-        hb_scatter<_Float16>(n_max, info, stride, dfeat_stride, grid, p, pos, static_cast<const _Float16*>(dfeat),
+        hb_scatter<_Float16, HbRec8>(n_max, info, stride, dfeat_stride, grid, p, pos, static_cast<const _Float16*>(dfeat),
                              pa, wa, 0, L, j0, j1, stream);
     TN_CHECK_LAUNCH();
     return TN_OK;
@@ -1641,7 +1798,7 @@ static int hb_accumulate_all(uint32_t n_max, tn_hashgrid_t grid, float* dtable, 
     HbWorkArea wa;
     hb_plan_area(p, const_cast<void*>(plan), &pa);
     hb_work_area(p, work, &wa);
-    hb_accumulate(n_max, grid, p, dtable, pa, wa, 0, (uint32_t)grid.n_levels, adam, stream);
+    hb_accumulate<HbRec8>(n_max, grid, p, dtable, pa, wa, 0, (uint32_t)grid.n_levels, adam, stream);
     hb_finish(grid, p, dtable, pa, wa, adam, stream);
     TN_CHECK_LAUNCH();
     return TN_OK;
