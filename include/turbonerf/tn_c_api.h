@@ -110,6 +110,12 @@ int tn_accumulate_samples(const uint32_t* info, unsigned long long* total, tn_st
  * over the whole batch (src/core/nerf-network.cu:223-317). */
 int tn_batch_tail(const uint32_t* info, uint32_t first, uint32_t* tail_info, tn_stream_t stream);
 
+/* The descriptor of a batch whose counts the host knows: n_rays rays,
+ * n_samples samples, status 0 (written on the stream, with no copy from host
+ * memory; the reference passes its host-side counts as kernel arguments,
+ * src/core/nerf-network.cu:223-317). */
+int tn_batch_info(uint32_t n_rays, uint32_t n_samples, uint32_t* info, tn_stream_t stream);
+
 /* Next step's ray count from this step's samples per ray (device-side
  * replacement of reference src/core/trainer.cu:133-140). */
 int tn_estimate_rays(const uint32_t* info, uint32_t max_samples, uint32_t cap, uint32_t min_rays,

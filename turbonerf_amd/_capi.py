@@ -148,6 +148,7 @@ _SIGS: dict[str, tuple] = {
                                     vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]),
     "tn_estimate_rays": (C.c_int, [vp, u32, u32, u32, vp, vp]),
     "tn_accumulate_samples": (C.c_int, [vp, vp, vp]),
+    "tn_batch_info": (C.c_int, [u32, u32, vp, vp]),
     "tn_batch_tail": (C.c_int, [vp, u32, vp, vp]),
     "tn_composite_scratch_bytes": (sz, [u32, u32]),
     "tn_composite_train": (C.c_int, [C.c_int, vp, u32, u32, u32, f32, C.c_int, f32, vp, vp, vp, vp, vp, vp, vp, vp,

@@ -81,7 +81,7 @@ class NerfMLP(torch.autograd.Function):
         if grad_rgb is None:
             grad_rgb = torch.zeros(3, n, dtype=net.dtype, device=net.device)
         ones = torch.ones(n, dtype=torch.float32, device=net.device)  # t >= 1: no distance scaling
-        grad_net = torch.zeros(net.numel(), dtype=torch.float32, device=net.device)
+        grad_net = torch.empty(net.numel(), dtype=torch.float32, device=net.device)  # stored whole
         dfeat = ops.mlp_backward(net, 0, n, feat, n, dir01, n, ones, _contig(grad_rgb.to(net.dtype)),
                                  _contig(grad_dens.float()), 1.0, grad_net)
         return grad_net.to(net.dtype), dfeat.view(32, n), None
@@ -96,7 +96,7 @@ class CompositeLoss(torch.autograd.Function):
         steps, offsets, bg, target = _contig(steps), _contig(offsets), _contig(bg), _contig(target)
         n_rays = steps.numel()
         S = density.numel()
-        info = torch.tensor([n_rays, S, 0, 0], dtype=torch.int32, device=density.device)
+        info = ops.batch_info(n_rays, S)
         loss, dLd, dLc = ops.composite_train(info, n_rays, n_rays, S, steps, offsets, bg, target, density,
                                              color, dt, grad_scale=1.0, min_T=min_T)
         ctx.save_for_backward(dLd, dLc)
@@ -120,7 +120,7 @@ class DistortionLoss(torch.autograd.Function):
         n_rays = steps.numel()
         S = density.numel()
         code = {torch.float32: 0, torch.float16: 1}[density.dtype]
-        info = torch.tensor([n_rays, S, 0, 0], dtype=torch.int32, device=density.device)
+        info = ops.batch_info(n_rays, S)
         loss = torch.zeros(n_rays, dtype=torch.float32, device=density.device)
         grad = torch.zeros(S, dtype=torch.float32, device=density.device)
         nb = query("tn_distortion_scratch_bytes", n_rays, S)

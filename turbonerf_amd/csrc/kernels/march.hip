@@ -537,9 +537,23 @@ __global__ void batch_tail_kernel(const uint32_t* __restrict__ info, uint32_t fi
     tail[3] = info[3];
 }
 
+__global__ void batch_info_kernel(uint32_t n_rays, uint32_t n_samples, uint32_t* __restrict__ info) {
+    info[0] = n_rays;
+    info[1] = n_samples;
+    info[2] = 0u;
+    info[3] = n_rays;
+}
+
 }  // namespace tn
 
 using namespace tn;
+
+extern "C" int tn_batch_info(uint32_t n_rays, uint32_t n_samples, uint32_t* info, hipStream_t stream) {
+    TN_CHECK_ARG(info);
+    batch_info_kernel<<<1, 1, 0, stream>>>(n_rays, n_samples, info);
+    TN_CHECK_LAUNCH();
+    return TN_OK;
+}
 
 // total[0] += info[1] on the device (running count of trained samples)
 extern "C" int tn_accumulate_samples(const uint32_t* info, unsigned long long* total, hipStream_t stream) {

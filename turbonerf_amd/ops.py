@@ -125,17 +125,31 @@ def march_generate(rays: Rays, samples: Samples, n_rays_max: int, info: torch.Te
 _DTYPE_CODE = {torch.float32: 0, torch.float16: 1}
 
 
+def _out(n: int, written: bool, dtype) -> torch.Tensor:
+    """An output buffer: zero-filled unless the call writes every element."""
+    return (torch.empty if written else torch.zeros)(n, dtype=dtype, device="cuda")
+
+
+def batch_info(n_rays: int, n_samples: int) -> torch.Tensor:
+    """Batch descriptor of counts that the host knows."""
+    info = torch.empty(4, dtype=torch.int32, device="cuda")
+    call("tn_batch_info", n_rays, n_samples, ptr(info), stream_ptr())
+    return info
+
+
 def composite_train(info: torch.Tensor, n_rays_max: int, stride: int, sample_stride: int, steps: torch.Tensor,
                     offs: torch.Tensor, bg: torch.Tensor, target: torch.Tensor, density: torch.Tensor,
                     color: torch.Tensor, dt: torch.Tensor, grad_scale: float = 1.0, min_T: float = 1e-4,
-                    fp64_accumulate: bool = False, scale_by_rays: bool = False):
-    """Returns (loss[4*stride], dL_ddensity[sample_stride], dL_dcolor[3*sample_stride])."""
+                    fp64_accumulate: bool = False, scale_by_rays: bool = False, whole: bool = False):
+    """Returns (loss[4*stride], dL_ddensity[sample_stride], dL_dcolor[3*sample_stride]).
+    whole: info counts every ray and sample of the buffers, so that nothing
+    beyond the batch is left to be zero."""
     code = 2 if fp64_accumulate else _DTYPE_CODE[density.dtype]
     if fp64_accumulate and density.dtype != torch.float32:
         raise ValueError("fp64 accumulation takes fp32 inputs")
-    loss = torch.zeros(4 * stride, dtype=torch.float32, device="cuda")
-    dLd = torch.zeros(sample_stride, dtype=torch.float32, device="cuda")
-    dLc = torch.zeros(3 * sample_stride, dtype=density.dtype, device="cuda")
+    loss = _out(4 * stride, whole, torch.float32)
+    dLd = _out(sample_stride, whole, torch.float32)
+    dLc = _out(3 * sample_stride, whole, density.dtype)
     nb = query("tn_composite_scratch_bytes", n_rays_max, sample_stride)
     scratch = torch.empty(nb // 4, dtype=torch.float32, device="cuda")
     call("tn_composite_train", code, ptr(info), n_rays_max, stride, sample_stride, grad_scale, int(scale_by_rays), min_T,
@@ -226,7 +240,7 @@ def hashgrid_forward(grid: _capi.HashGrid, n: int, pos: torch.Tensor, stride: in
     MLP kernels take fp32 features in both precisions)."""
     feat_dtype = torch.float32 if feat_dtype is None else feat_dtype
     out_stride = stride if out_stride is None else out_stride
-    out = torch.zeros(2 * grid.n_levels * out_stride, dtype=feat_dtype, device="cuda")
+    out = _out(2 * grid.n_levels * out_stride, info is None and n == out_stride, feat_dtype)
     call("tn_hashgrid_forward", _PREC[table.dtype], _PREC[feat_dtype], n, ptr(info), stride, out_stride, grid,
          ptr(pos), ptr(table), ptr(out), stream_ptr())
     return out
@@ -320,8 +334,9 @@ def mlp_forward(params: torch.Tensor, net_offset: int, n: int, feat: torch.Tenso
     f16 = feat.dtype == torch.float16
     if (feat.dtype != torch.float32 and not (f16 and prec == 1)) or feat.numel() < 32 * feat_stride:
         raise ValueError("the MLP kernels take fp32 features [32][feat_stride] (fp16 for an fp16 network)")
-    dens = torch.zeros(stride, dtype=params.dtype, device="cuda")
-    rgb = torch.zeros(3 * stride, dtype=params.dtype, device="cuda") if color else None
+    written = info is None and n == stride
+    dens = _out(stride, written, params.dtype)
+    rgb = _out(3 * stride, written, params.dtype) if color else None
     call("tn_mlp_inference", prec, int(f16), n, ptr(info), stride, feat_stride, stride, ptr(params), net_offset,
          ptr(feat), ptr(dir), int(color), ptr(dens), ptr(rgb), _app_ref(app), stream_ptr())
     return dens, rgb
@@ -359,7 +374,7 @@ def mlp_backward(params: torch.Tensor, net_offset: int, n: int, feat: torch.Tens
         raise ValueError("the MLP kernels take fp32 features [32][feat_stride]")
     if dL_drgb.dtype != params.dtype:
         raise ValueError("dL_drgb is in the network precision")
-    dfeat = torch.zeros(32 * feat_stride, dtype=torch.float32, device="cuda")
+    dfeat = _out(32 * feat_stride, info is None and n == feat_stride, torch.float32)
     nb = query("tn_mlp_backward_workspace_bytes", n)
     ws = torch.empty(max(nb, 4), dtype=torch.uint8, device="cuda")
     call("tn_mlp_backward", prec, n, ptr(info), stride, feat_stride, ptr(params), net_offset, ptr(feat), ptr(dir),
