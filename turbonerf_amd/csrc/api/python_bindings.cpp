@@ -369,10 +369,9 @@ PYBIND11_MODULE(PyTurboNeRF, m) {
                 float thr) { tc.set_occupancy_from_density(d.data(), thr); },
              py::arg("density"), py::arg("threshold"))
         .def("get_params",
-             [](const NeRFTrainingController& tc) {
-                 auto v = tc.get_params();
-                 py::array_t<float> a(v.size());
-                 std::memcpy(a.mutable_data(), v.data(), v.size() * sizeof(float));
+             [](NeRFTrainingController& tc) {
+                 py::array_t<float> a(tc.n_params());
+                 tc.read_params(a.mutable_data());
                  return a;
              })
         .def("set_params",

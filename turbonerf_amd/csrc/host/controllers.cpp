@@ -279,6 +279,12 @@ std::vector<float> NeRFTrainingController::get_params() const {
     return h;
 }
 
+void NeRFTrainingController::read_params(float* dst) {
+    const DeviceBuffer<float>& p = proxy->nerfs[0].params.params_fp;
+    // training work ends with the device stream waiting for it
+    reader_.read(dst, p.data(), p.bytes(), DeviceManager::stream());
+}
+
 void NeRFTrainingController::set_params(const std::vector<float>& h) {
     NeRF& nerf = proxy->nerfs[0];
     if (h.size() != nerf.params.params_fp.size()) throw std::runtime_error("set_params: size mismatch");

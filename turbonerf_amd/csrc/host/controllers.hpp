@@ -128,6 +128,9 @@ struct NeRFTrainingController {
     void set_occupancy_from_density(const float* density_host, float threshold);
     // raw parameter access (fp32 master weights), for tests and snapshots
     std::vector<float> get_params() const;
+    size_t n_params() const { return proxy->nerfs[0].params.params_fp.size(); }
+    // get_params() into a caller's array of n_params()
+    void read_params(float* dst);
     void set_params(const std::vector<float>& p);
 
     // per-phase HIP-event timing of enqueued steps (name -> ms, launches)
@@ -155,6 +158,7 @@ private:
     uint64_t generation_ = 0;  // proxy->generation when setup_data() ran
     Trainer trainer_;
     hipEvent_t ev_in_ = nullptr, ev_out_ = nullptr;
+    HostReader reader_;
     void sync_settings();
     // Training runs on the trainer's own streams; begin_work orders it after
     // the work already on the device stream (uploads, parameter writes),

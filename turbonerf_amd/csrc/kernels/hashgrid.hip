@@ -526,7 +526,7 @@ TN_DEVICE float seg_factor(int key) {
 // Segmented sums over the runs of `heads` (bit i: lane i starts a run). The
 // scatter is bound by its vector instructions, and these sums were 222 of 625
 // per wave and level; with these, and one LDS counter and maximum for the two
-// x neighbours, it went from 87 to 71 us at 262,144 samples. A step
+// x neighbours, it went from 87 to 81 us at 262,144 samples. A step
 // that no run is long enough for, or that crosses into rows no run crosses
 // into, is left out: on fine levels runs are of two or three samples.
 TN_DEVICE void seg_sum16(float (&a0)[8], float (&a1)[8], int key, uint64_t heads, bool small) {
