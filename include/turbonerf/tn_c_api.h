@@ -55,6 +55,21 @@ int tn_init_training_rays(uint32_t n_rays_max, const uint32_t* d_n_rays, uint32_
     float* ori, float* dir, float* ray_t, float* ray_tmax, uint8_t* ray_alive,
     tn_stream_t stream);
 
+/* A training batch's rays in one launch, for a caller that keeps the ray count
+ * and the uniform stream's position on the device: ray i < *d_n_rays draws
+ * elements i, i + stride, i + 2 stride and i + 3 stride of tn_fill_uniform's
+ * stream at *d_offset into random[4][stride] (the rest is left as it is;
+ * *d_offset is not advanced, tn_batch_select does that), is formed as
+ * tn_init_training_rays forms it from the first, split evenly over the
+ * images, and dropped as tn_deactivate_rays drops it by the second when both
+ * bounds are below 1. Replaces the same reference kernels. */
+int tn_training_rays(uint32_t n_rays_max, const uint32_t* d_n_rays, uint32_t stride, uint32_t n_images,
+    uint32_t n_pixels_per_image, int32_t img_w, int32_t img_h, const tn_bbox_t* bbox,
+    const tn_camera_t* cameras, const uint8_t* images, uint64_t seed, const unsigned long long* d_offset,
+    float alpha_threshold, float selection_probability, float* random, float* pix_rgba,
+    uint32_t* ray_img_id, float* ori, float* dir, float* ray_t, float* ray_tmax, uint8_t* ray_alive,
+    tn_stream_t stream);
+
 /* Replaces deactivate_rays_with_alpha_threshold_kernel
  * (reference src/utils/training-batch-kernels.cuh:189-208). */
 int tn_deactivate_rays(uint32_t n_rays_max, const uint32_t* d_n_rays, uint32_t stride,
@@ -85,6 +100,14 @@ int tn_scan_select(int mode, uint32_t n_rays, const uint32_t* d_n_rays, const ui
     uint32_t max_samples,
     uint32_t* ray_offset, uint32_t* info, void* workspace, size_t workspace_bytes,
     tn_stream_t stream);
+
+/* tn_scan_select (mode 0) of a training batch, tn_estimate_rays for the next
+ * one and the uniform stream's advance (*d_offset += advance; null: none) in
+ * one launch of one workgroup; d_n_rays and n_rays_next may be the same.
+ * Replaces the same reference code. */
+int tn_batch_select(uint32_t n_rays_max, const uint32_t* d_n_rays, const uint32_t* n_steps, uint32_t max_samples,
+    uint32_t* ray_offset, uint32_t* info, uint32_t cap, uint32_t min_rays, uint32_t* n_rays_next,
+    unsigned long long* d_offset, uint64_t advance, tn_stream_t stream);
 
 /* Re-march and write compacted per-sample SoA buffers (stride sample_stride;
  * ray buffers have stride `stride`). Replaces

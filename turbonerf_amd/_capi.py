@@ -139,6 +139,9 @@ _SIGS: dict[str, tuple] = {
     "tn_fill_uniform_dev": (C.c_int, [u64, u64, vp, vp, vp]),
     "tn_init_training_rays": (C.c_int, [u32, vp, u32, u32, u32, i32, i32, f32, vp, vp, vp, vp, vp, vp, vp,
                                         vp, vp, vp, vp, vp]),
+    "tn_training_rays": (C.c_int, [u32, vp, u32, u32, u32, i32, i32, vp, vp, vp, u64, vp, f32, f32, vp, vp, vp, vp,
+                                   vp, vp, vp, vp, vp]),
+    "tn_batch_select": (C.c_int, [u32, vp, vp, u32, vp, vp, u32, u32, vp, vp, u64, vp]),
     "tn_deactivate_rays": (C.c_int, [u32, vp, u32, f32, f32, vp, vp, vp, vp]),
     "tn_march_count": (C.c_int, [u32, vp, u32, BBox, OccupancyGrid, f32, f32, f32, u32, vp, vp, vp, vp, vp,
                                  vp, vp]),

@@ -399,14 +399,13 @@ void TrainingWorkspace::enlarge(uint32_t B, uint32_t R) {
     sample_m_norm.resize(B);
     sample_dt_norm.resize(B);
     info.resize(4);
-    scan_ws.resize(std::max<size_t>(tn_scan_workspace_bytes(R), 4));
 }
 
 size_t TrainingWorkspace::bytes() const {
     return random_float.bytes() + pix_rgba.bytes() + ray_origin.bytes() + ray_dir.bytes() + ray_t.bytes() +
            ray_t_max.bytes() + ray_img_id.bytes() + ray_step.bytes() + ray_offset.bytes() + ray_alive.bytes() +
            sample_img_id.bytes() + sample_t.bytes() + sample_pos.bytes() + sample_dir.bytes() + sample_dt.bytes() +
-           sample_m_norm.bytes() + sample_dt_norm.bytes() + scan_ws.bytes() + hash_plan.bytes();
+           sample_m_norm.bytes() + sample_dt_norm.bytes() + hash_plan.bytes();
 }
 
 void TrainingWorkspace::free_allocations() { *this = TrainingWorkspace(); }
@@ -477,20 +476,15 @@ void Trainer::generate_next_training_batch(Context& ctx, TrainingWorkspace& ws, 
         // seeded uniforms: slice 0 picks pixels, slices 1-3 are the background
         // colour (reference trainer.cu:45-50,332); rays are generated for the
         // device-side estimate of how many fill the batch and split evenly
-        // over the images by that count (-1 below)
+        // over the images by that count
         ScopedPhase ph(tm, "rays", s);
-        TN_TRY(tn_fill_uniform_dev(4 * (uint64_t)R, ctx.rng_seed, ctx.d_rng.data(), ws.random_float.data(), ts));
-        TN_TRY(tn_init_training_rays(R, ctx.n_rays_next.data(), R, dw.n_images, dw.n_pixels_per_image,
-                                     dw.image_dims.x, dw.image_dims.y, -1.0f,
-                                     reinterpret_cast<const tn_bbox_t*>(dw.bbox.data()),
-                                     reinterpret_cast<const tn_camera_t*>(dw.cameras.data()), dw.images.data(),
-                                     ws.random_float.data(), ws.pix_rgba.data(), ws.ray_img_id.data(),
-                                     ws.ray_origin.data(), ws.ray_dir.data(), ws.ray_t.data(), ws.ray_t_max.data(),
-                                     ws.ray_alive.data(), ts));
-        if (ctx.alpha_selection_threshold < 1.0f && ctx.alpha_selection_probability < 1.0f)
-            TN_TRY(tn_deactivate_rays(R, ctx.n_rays_next.data(), R, ctx.alpha_selection_threshold,
-                                      ctx.alpha_selection_probability, ws.pix_rgba.data(), ws.random_float.data() + R,
-                                      ws.ray_alive.data(), ts));
+        TN_TRY(tn_training_rays(R, ctx.n_rays_next.data(), R, dw.n_images, dw.n_pixels_per_image, dw.image_dims.x,
+                                dw.image_dims.y, reinterpret_cast<const tn_bbox_t*>(dw.bbox.data()),
+                                reinterpret_cast<const tn_camera_t*>(dw.cameras.data()), dw.images.data(),
+                                ctx.rng_seed, ctx.d_rng.data(), ctx.alpha_selection_threshold,
+                                ctx.alpha_selection_probability, ws.random_float.data(), ws.pix_rgba.data(),
+                                ws.ray_img_id.data(), ws.ray_origin.data(), ws.ray_dir.data(), ws.ray_t.data(),
+                                ws.ray_t_max.data(), ws.ray_alive.data(), ts));
     }
     const float dt_min = ctx.min_step_size;
     const float dt_max = ds.bounding_box.size() * dt_min;
@@ -504,8 +498,8 @@ void Trainer::generate_next_training_batch(Context& ctx, TrainingWorkspace& ws, 
     }
     {
         ScopedPhase ph(tm, "scan_select", s);
-        TN_TRY(tn_scan_select(0, R, ctx.n_rays_next.data(), ws.ray_step.data(), B, ws.ray_offset.data(),
-                              ws.info.data(), ws.scan_ws.data(), ws.scan_ws.size(), ts));
+        TN_TRY(tn_batch_select(R, ctx.n_rays_next.data(), ws.ray_step.data(), B, ws.ray_offset.data(),
+                               ws.info.data(), R, 64, ctx.n_rays_next.data(), ctx.d_rng.data(), 4 * (uint64_t)R, ts));
     }
     {
         ScopedPhase ph(tm, "march_generate", s);
@@ -515,7 +509,6 @@ void Trainer::generate_next_training_batch(Context& ctx, TrainingWorkspace& ws, 
                                  ws.ray_step.data(), ws.sample_img_id.data(), ws.sample_t.data(), ws.sample_pos.data(),
                                  ws.sample_dir.data(), ws.sample_dt.data(), ws.sample_m_norm.data(),
                                  ws.sample_dt_norm.data(), ts));
-        TN_TRY(tn_estimate_rays(ws.info.data(), B, R, 64, ctx.n_rays_next.data(), ts));
     }
     {
         // the hash-grid backward's plan needs only the positions: formed here,

@@ -240,7 +240,6 @@ struct TrainingWorkspace {
     DeviceBuffer<uint32_t> sample_img_id;
     DeviceBuffer<float> sample_t, sample_pos, sample_dir, sample_dt, sample_m_norm, sample_dt_norm;
     DeviceBuffer<uint32_t> info;
-    DeviceBuffer<uint8_t> scan_ws;
     // the hash-grid backward's plan for this batch (record counts and offsets
     // per bin, from the sample positions), formed with the batch
     DeviceBuffer<uint8_t> hash_plan;

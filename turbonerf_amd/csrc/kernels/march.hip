@@ -511,9 +511,8 @@ __global__ void march_expand_kernel(uint32_t n_rays_max, uint32_t SB_max, const 
 // step's samples-per-ray rate, with 1/8 headroom so the prefix selection
 // usually has rays to spare (replaces the reference's host-side estimate,
 // trainer.cu:133-140).
-__global__ void estimate_rays_kernel(const uint32_t* __restrict__ info, uint32_t max_samples, uint32_t cap,
-                                     uint32_t min_rays, uint32_t* __restrict__ n_rays_next) {
-    const uint32_t n_rays = info[0], n_samples = info[1];
+TN_DEVICE uint32_t estimate_rays(uint32_t n_rays, uint32_t n_samples, uint32_t max_samples, uint32_t cap,
+                                 uint32_t min_rays) {
     uint32_t est = cap;
     if (n_samples > 0 && n_rays > 0) {
         const double per = (double)n_rays / (double)n_samples;
@@ -522,7 +521,84 @@ __global__ void estimate_rays_kernel(const uint32_t* __restrict__ info, uint32_t
     }
     if (est < min_rays) est = min_rays;
     if (est > cap) est = cap;
-    *n_rays_next = est;
+    return est;
+}
+
+__global__ void estimate_rays_kernel(const uint32_t* __restrict__ info, uint32_t max_samples, uint32_t cap,
+                                     uint32_t min_rays, uint32_t* __restrict__ n_rays_next) {
+    *n_rays_next = estimate_rays(info[0], info[1], max_samples, cap, min_rays);
+}
+
+// A training batch's selection in one launch of one workgroup: the exclusive
+// scan of the rays' step counts, the reference's selection (mode 0 of
+// scan_write_select_kernel), the next batch's ray count and the advance of the
+// uniform stream. A batch has some thousands of rays, so a launch costs more
+// than the scan: three scan launches, the estimate and the counter took 5 us
+// each; more rays than one round of the workgroup (16,384) take 3 us more per
+// round.
+constexpr int kSelectThreads = 1024;
+__global__ void __launch_bounds__(kSelectThreads)
+batch_select_kernel(uint32_t n_max, const uint32_t* d_n, const uint32_t* __restrict__ vals, uint32_t max_samples,
+                    uint32_t* __restrict__ offsets, uint32_t* __restrict__ info, uint32_t cap, uint32_t min_rays,
+                    uint32_t* n_rays_next, unsigned long long* __restrict__ rng, unsigned long long rng_advance) {
+    __shared__ uint32_t wsum[kSelectThreads / 64];
+    __shared__ uint32_t kept[2];
+    const uint32_t n = min(*d_n, n_max), lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+    if (threadIdx.x < 2) kept[threadIdx.x] = 0u;
+    uint64_t carry = 0;  // samples of the rounds before
+    for (uint32_t base = 0; base < n; base += kSelectThreads * kScanItems) {
+        const uint32_t j0 = base + threadIdx.x * kScanItems;
+        uint32_t v[kScanItems], s = 0;
+#pragma unroll
+        for (int k = 0; k < kScanItems; ++k) {
+            v[k] = j0 + k < n ? vals[j0 + k] : 0u;
+            s += v[k];
+        }
+        uint32_t inc = s;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(inc, d, 64);
+            if (lane >= (uint32_t)d) inc += o;
+        }
+        __syncthreads();  // wsum is free, kept cleared
+        if (lane == 63) wsum[wid] = inc;
+        __syncthreads();
+        uint64_t run = carry + inc - s;
+        uint32_t total = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kSelectThreads / 64; ++w) {
+            const uint32_t x = wsum[w];
+            run += w < wid ? x : 0u;
+            total += x;
+        }
+#pragma unroll
+        for (int k = 0; k < kScanItems; ++k) {
+            const uint32_t j = j0 + k;
+            if (j >= n) break;
+            const uint32_t off = (uint32_t)min(run, (uint64_t)0xFFFFFFFFu);
+            offsets[j] = off;
+            const uint64_t next = run + v[k];
+            // exactly one ray is the last with offset < max_samples; the rays before it are kept
+            if (off < max_samples && (j + 1 == n || next >= max_samples)) {
+                kept[0] = j;
+                kept[1] = off;
+            }
+            run = next;
+        }
+        carry += total;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t nr = kept[0], ns = kept[1];
+        if (n > 0) {
+            info[0] = nr;
+            info[1] = ns;
+            info[2] = nr == 0 ? (uint32_t)TN_ERR_NO_RAYS : (ns == 0 ? (uint32_t)TN_ERR_NO_SAMPLES : 0u);
+        }
+        info[3] = n;
+        *n_rays_next = estimate_rays(info[0], info[1], max_samples, cap, min_rays);
+        if (rng) *rng += rng_advance;
+    }
 }
 
 __global__ void accumulate_samples_kernel(const uint32_t* __restrict__ info, unsigned long long* __restrict__ total) {
@@ -626,6 +702,18 @@ extern "C" int tn_march_generate(uint32_t n_rays_max, const uint32_t* info, uint
     march_expand_kernel<<<blocks_for(sample_stride, 256), 256, 0, stream>>>(
         n_rays_max, sample_stride, info, stride, sample_stride, inv_aabb, dt_min, dt_max, cone_angle, ray_img_id, ori,
         dir, ray_t, ray_offset, n_ray_steps, out_img_id, out_t, out_pos, out_dir, out_dt, out_m_norm, out_dt_norm);
+    TN_CHECK_LAUNCH();
+    return TN_OK;
+}
+
+extern "C" int tn_batch_select(uint32_t n_rays_max, const uint32_t* d_n_rays, const uint32_t* n_steps,
+                               uint32_t max_samples, uint32_t* ray_offset, uint32_t* info, uint32_t cap,
+                               uint32_t min_rays, uint32_t* n_rays_next, unsigned long long* d_offset,
+                               uint64_t advance, hipStream_t stream) {
+    TN_CHECK_ARG(d_n_rays && n_steps && ray_offset && info && n_rays_next && n_rays_max > 0 && max_samples > 0 && cap > 0);
+    batch_select_kernel<<<1, kSelectThreads, 0, stream>>>(n_rays_max, d_n_rays, n_steps, max_samples, ray_offset, info,
+                                                          cap, min_rays, n_rays_next, d_offset,
+                                                          (unsigned long long)advance);
     TN_CHECK_LAUNCH();
     return TN_OK;
 }
