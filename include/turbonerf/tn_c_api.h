@@ -120,6 +120,26 @@ int tn_march_generate(uint32_t n_rays_max, const uint32_t* info, uint32_t stride
     const uint32_t* n_ray_steps, uint32_t* out_img_id, float* out_t, float* out_pos,
     float* out_dir, float* out_dt, float* out_m_norm, float* out_dt_norm, tn_stream_t stream);
 
+/* The two marching passes for a caller that keeps a workspace between them
+ * (tn_march_runs_bytes for the ray capacity, 128-byte aligned): the count pass
+ * leaves each ray's runs of samples there, and the generate pass forms the
+ * samples from them without marching through empty cells again, in one
+ * launch, the same bit for bit. Between the calls the rays, the grid and the
+ * settings stay as they are. out_img_id, out_t, out_m_norm and out_dt_norm
+ * may be null (a render reads none of them; ray_img_id too, without
+ * out_img_id). Same replacements as tn_march_count and tn_march_generate. */
+size_t tn_march_runs_bytes(uint32_t n_rays_max);
+int tn_march_count_runs(uint32_t n_rays_max, const uint32_t* d_n_rays, uint32_t stride,
+    tn_bbox_t bbox, tn_occupancy_grid_t grid, float cone_angle, float dt_min, float dt_max,
+    uint32_t max_steps, const float* dir, const float* ray_tmax, uint8_t* ray_alive,
+    const float* ori, const float* ray_t, uint32_t* n_steps, void* runs, size_t runs_bytes, tn_stream_t stream);
+int tn_march_generate_runs(uint32_t n_rays_max, const uint32_t* info, uint32_t stride,
+    uint32_t sample_stride, tn_bbox_t bbox, float inv_aabb, tn_occupancy_grid_t grid, float dt_min, float dt_max,
+    float cone_angle, const uint32_t* ray_img_id, const float* ori, const float* dir,
+    const float* ray_t, const uint32_t* ray_offset, const uint8_t* ray_alive,
+    const uint32_t* n_ray_steps, const void* runs, size_t runs_bytes, uint32_t* out_img_id, float* out_t,
+    float* out_pos, float* out_dir, float* out_dt, float* out_m_norm, float* out_dt_norm, tn_stream_t stream);
+
 /* total[0] += info[1] on the device: a running count of trained samples that
  * needs no host synchronisation (no reference counterpart; the reference
  * reads n_samples back every step, src/core/trainer.cu:169-179). */

@@ -149,6 +149,11 @@ _SIGS: dict[str, tuple] = {
     "tn_scan_select": (C.c_int, [C.c_int, u32, vp, vp, u32, vp, vp, vp, sz, vp]),
     "tn_march_generate": (C.c_int, [u32, vp, u32, u32, BBox, f32, OccupancyGrid, f32, f32, f32, vp, vp, vp, vp, vp,
                                     vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]),
+    "tn_march_runs_bytes": (sz, [u32]),
+    "tn_march_count_runs": (C.c_int, [u32, vp, u32, BBox, OccupancyGrid, f32, f32, f32, u32, vp, vp, vp, vp, vp,
+                                      vp, vp, sz, vp]),
+    "tn_march_generate_runs": (C.c_int, [u32, vp, u32, u32, BBox, f32, OccupancyGrid, f32, f32, f32, vp, vp, vp, vp,
+                                         vp, vp, vp, vp, sz, vp, vp, vp, vp, vp, vp, vp, vp]),
     "tn_estimate_rays": (C.c_int, [vp, u32, u32, u32, vp, vp]),
     "tn_accumulate_samples": (C.c_int, [vp, vp, vp]),
     "tn_batch_info": (C.c_int, [u32, u32, vp, vp]),

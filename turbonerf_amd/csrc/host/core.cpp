@@ -391,6 +391,7 @@ void TrainingWorkspace::enlarge(uint32_t B, uint32_t R) {
     ray_step.resize(R);
     ray_offset.resize(R);
     ray_alive.resize(R);
+    ray_runs.resize(tn_march_runs_bytes(R));
     sample_img_id.resize(B);
     sample_t.resize(B);
     sample_pos.resize(3 * (size_t)B);
@@ -404,7 +405,8 @@ void TrainingWorkspace::enlarge(uint32_t B, uint32_t R) {
 size_t TrainingWorkspace::bytes() const {
     return random_float.bytes() + pix_rgba.bytes() + ray_origin.bytes() + ray_dir.bytes() + ray_t.bytes() +
            ray_t_max.bytes() + ray_img_id.bytes() + ray_step.bytes() + ray_offset.bytes() + ray_alive.bytes() +
-           sample_img_id.bytes() + sample_t.bytes() + sample_pos.bytes() + sample_dir.bytes() + sample_dt.bytes() +
+           ray_runs.bytes() + sample_img_id.bytes() + sample_t.bytes() + sample_pos.bytes() + sample_dir.bytes() +
+           sample_dt.bytes() +
            sample_m_norm.bytes() + sample_dt_norm.bytes() + hash_plan.bytes();
 }
 
@@ -492,9 +494,10 @@ void Trainer::generate_next_training_batch(Context& ctx, TrainingWorkspace& ws, 
     const tn_occupancy_grid_t grid = nerf.occupancy_grid.view();
     {
         ScopedPhase ph(tm, "march_count", s);
-        TN_TRY(tn_march_count(R, ctx.n_rays_next.data(), R, bbox, grid, NeRFConstants::cone_angle, dt_min, dt_max,
-                              0xFFFFFFFFu, ws.ray_dir.data(), ws.ray_t_max.data(), ws.ray_alive.data(),
-                              ws.ray_origin.data(), ws.ray_t.data(), ws.ray_step.data(), ts));
+        TN_TRY(tn_march_count_runs(R, ctx.n_rays_next.data(), R, bbox, grid, NeRFConstants::cone_angle, dt_min,
+                                   dt_max, 0xFFFFFFFFu, ws.ray_dir.data(), ws.ray_t_max.data(), ws.ray_alive.data(),
+                                   ws.ray_origin.data(), ws.ray_t.data(), ws.ray_step.data(), ws.ray_runs.data(),
+                                   ws.ray_runs.size(), ts));
     }
     {
         ScopedPhase ph(tm, "scan_select", s);
@@ -503,12 +506,13 @@ void Trainer::generate_next_training_batch(Context& ctx, TrainingWorkspace& ws, 
     }
     {
         ScopedPhase ph(tm, "march_generate", s);
-        TN_TRY(tn_march_generate(R, ws.info.data(), R, B, bbox, 1.0f / ds.bounding_box.size(), grid, dt_min, dt_max,
-                                 NeRFConstants::cone_angle, ws.ray_img_id.data(), ws.ray_origin.data(),
-                                 ws.ray_dir.data(), ws.ray_t.data(), ws.ray_offset.data(), ws.ray_alive.data(),
-                                 ws.ray_step.data(), ws.sample_img_id.data(), ws.sample_t.data(), ws.sample_pos.data(),
-                                 ws.sample_dir.data(), ws.sample_dt.data(), ws.sample_m_norm.data(),
-                                 ws.sample_dt_norm.data(), ts));
+        TN_TRY(tn_march_generate_runs(R, ws.info.data(), R, B, bbox, 1.0f / ds.bounding_box.size(), grid, dt_min,
+                                      dt_max, NeRFConstants::cone_angle, ws.ray_img_id.data(), ws.ray_origin.data(),
+                                      ws.ray_dir.data(), ws.ray_t.data(), ws.ray_offset.data(), ws.ray_alive.data(),
+                                      ws.ray_step.data(), ws.ray_runs.data(), ws.ray_runs.size(),
+                                      ws.sample_img_id.data(), ws.sample_t.data(), ws.sample_pos.data(),
+                                      ws.sample_dir.data(), ws.sample_dt.data(), ws.sample_m_norm.data(),
+                                      ws.sample_dt_norm.data(), ts));
     }
     {
         // the hash-grid backward's plan needs only the positions: formed here,

@@ -236,7 +236,7 @@ struct TrainingWorkspace {
     DeviceBuffer<float> random_float;
     DeviceBuffer<float> pix_rgba, ray_origin, ray_dir, ray_t, ray_t_max;
     DeviceBuffer<uint32_t> ray_img_id, ray_step, ray_offset;
-    DeviceBuffer<uint8_t> ray_alive;
+    DeviceBuffer<uint8_t> ray_alive, ray_runs;
     DeviceBuffer<uint32_t> sample_img_id;
     DeviceBuffer<float> sample_t, sample_pos, sample_dir, sample_dt, sample_m_norm, sample_dt_norm;
     DeviceBuffer<uint32_t> info;

@@ -30,15 +30,12 @@ void RenderingWorkspace::enlarge(uint32_t rays, uint32_t samples, size_t e) {
     offset.resize(rays);
     info.resize(4);
     alive.resize(rays);
+    runs.resize(tn_march_runs_bytes(rays));
     scan_ws.resize(std::max<size_t>(tn_scan_workspace_bytes(rays), 4));
     to_local.resize(12 * sizeof(float));
-    s_img.resize(samples);
-    s_t.resize(samples);
     s_pos.resize(3 * (size_t)samples);
     s_dir.resize(3 * (size_t)samples);
     s_dt.resize(samples);
-    s_m.resize(samples);
-    s_dtn.resize(samples);
     features.resize(32 * (size_t)samples * 4);  // fp32 in both precisions
     density.resize((size_t)samples * e);
     color.resize(3 * (size_t)samples * e);
@@ -79,16 +76,18 @@ uint64_t Renderer::render_pixels(hipStream_t s, const RenderRequest& req, const 
             m = std::min(m, (uint32_t)std::clamp(1.05 * (double)S / samples_per_ray, 256.0, (double)R));
         TN_TRY(tn_render_rays(m, p, R, cam, bbox, to_local, ws.ray_ori.data(), ws.ray_dir.data(), ws.ray_t.data(),
                               ws.ray_tmax.data(), ws.pixel.data(), ws.alive.data(), ts));
-        TN_TRY(tn_march_count(m, nullptr, R, bbox, grid, NeRFConstants::cone_angle, dt_min, dt_max,
-                              st.max_samples_per_ray, ws.ray_dir.data(), ws.ray_tmax.data(), ws.alive.data(),
-                              ws.ray_ori.data(), ws.ray_t.data(), ws.n_steps.data(), ts));
+        TN_TRY(tn_march_count_runs(m, nullptr, R, bbox, grid, NeRFConstants::cone_angle, dt_min, dt_max,
+                                   st.max_samples_per_ray, ws.ray_dir.data(), ws.ray_tmax.data(), ws.alive.data(),
+                                   ws.ray_ori.data(), ws.ray_t.data(), ws.n_steps.data(), ws.runs.data(),
+                                   ws.runs.size(), ts));
         TN_TRY(tn_scan_select(1, m, nullptr, ws.n_steps.data(), S, ws.offset.data(), ws.info.data(), ws.scan_ws.data(),
                               ws.scan_ws.size(), ts));
-        TN_TRY(tn_march_generate(m, ws.info.data(), R, S, bbox, 1.0f / aabb, grid, dt_min, dt_max,
-                                 NeRFConstants::cone_angle, ws.pixel.data(), ws.ray_ori.data(), ws.ray_dir.data(),
-                                 ws.ray_t.data(), ws.offset.data(), ws.alive.data(), ws.n_steps.data(), ws.s_img.data(),
-                                 ws.s_t.data(), ws.s_pos.data(), ws.s_dir.data(), ws.s_dt.data(), ws.s_m.data(),
-                                 ws.s_dtn.data(), ts));
+        // (image ids, t and the normalised steps are for training only)
+        TN_TRY(tn_march_generate_runs(m, ws.info.data(), R, S, bbox, 1.0f / aabb, grid, dt_min, dt_max,
+                                      NeRFConstants::cone_angle, nullptr, ws.ray_ori.data(), ws.ray_dir.data(),
+                                      ws.ray_t.data(), ws.offset.data(), ws.alive.data(), ws.n_steps.data(),
+                                      ws.runs.data(), ws.runs.size(), nullptr, nullptr, ws.s_pos.data(),
+                                      ws.s_dir.data(), ws.s_dt.data(), nullptr, nullptr, ts));
         if (nerf.analytic_blobs.size()) {
             // synthetic scene: sigma and colour of the blob field
             TN_TRY(tn_blob_eval(ws.info.data(), S, S, aabb, nerf.analytic_blobs.data(),

@@ -137,9 +137,8 @@ struct RenderingWorkspace {
     uint32_t ray_capacity = 0, sample_capacity = 0;
     DeviceBuffer<float> ray_ori, ray_dir, ray_t, ray_tmax, rgba, image;
     DeviceBuffer<uint32_t> pixel, n_steps, offset, info;
-    DeviceBuffer<uint8_t> alive, scan_ws, to_local;
-    DeviceBuffer<uint32_t> s_img;
-    DeviceBuffer<float> s_t, s_pos, s_dir, s_dt, s_m, s_dtn;
+    DeviceBuffer<uint8_t> alive, scan_ws, to_local, runs;
+    DeviceBuffer<float> s_pos, s_dir, s_dt;
     DeviceBuffer<uint8_t> features, density, color;
     // several NeRFs (fixed-step world samples shared by all NeRFs)
     DeviceBuffer<float> m_trans, m_pos, m_dt, m_net_pos, m_net_dir, m_net_dt, m_c_pos, m_c_dir, m_rgba;

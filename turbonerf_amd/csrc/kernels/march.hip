@@ -157,16 +157,21 @@ TN_DEVICE float group_get(float v, uint32_t j) {
 // (lane-wise: sample n of the lane's ray at t). COUNT: stops at t_max, at
 // the box and at max_n samples; otherwise (the generate pass) takes max_n
 // samples, and one outside the box, which the count pass cannot have counted,
-// would be emitted without advancing. Returns the ray's sample count.
-template <int G, bool ML, bool COUNT, typename Emit>
+// would be emitted without advancing. Each run of samples without a skip in
+// between goes to `log` (its first t and sample, and the t after its last), in
+// pieces of at most G. Returns the ray's sample count.
+struct NoLog {
+    TN_DEVICE void run(bool, float, uint32_t, float) {}
+};
+template <int G, bool ML, bool COUNT, typename Emit, typename Log>
 TN_DEVICE uint32_t march_group(bool active, const MarchRay& r, float t, float t_max, uint32_t max_n,
-                               const tn_bbox_t& bbox, const MarchGrid& g, const MarchStep& st, Emit emit) {
+                               const tn_bbox_t& bbox, const MarchGrid& g, const MarchStep& st, Emit emit, Log& log) {
     const uint32_t lane = __lane_id(), j = lane & (uint32_t)(G - 1), axis = lane & 3u;
     const float oa = axis == 0 ? r.ox : axis == 1 ? r.oy : r.oz;
     const float da = axis == 0 ? r.dx : axis == 1 ? r.dy : r.dz;
     const float ida = 1.0f / da, ha = 0.5f * copysignf(1.0f, da);
     uint32_t n = 0;
-    bool done = !active, skip = false;
+    bool done = !active, skip = false, open = false;  // open: the last block's run goes on
     while (__ballot(!done) != 0ull) {
         if (__ballot(!done && !skip) != 0ull) {
             // a run: lane j's t after j more samples
@@ -189,6 +194,8 @@ TN_DEVICE uint32_t march_group(bool active, const MarchRay& r, float t, float t_
             const float t_f = group_get<G>(f < (uint32_t)G ? tj : tn, f < (uint32_t)G ? f : (uint32_t)G - 1u);
             if (!done && !skip) {
                 if (j < f) emit(n + j, tj);
+                if (f != 0u) log.run(!open, t, n, t_f);
+                open = f == (uint32_t)G;
                 n += f;
                 t = t_f;
                 skip = f < (uint32_t)G && e == f;  // the run ended at an empty cell
@@ -256,11 +263,35 @@ TN_DEVICE MarchRay load_ray(bool active, uint32_t i, uint32_t B, const float* __
                   : MarchRay{0.0f, 0.0f, 0.0f, 1.0f, 1.0f, 1.0f};
 }
 
+// What the count pass leaves of a ray for the generate pass (16 records of 8
+// bytes, one 128-byte line per ray): record 0 the number of runs and the t
+// after the last sample, records 1 to 15 each run's first t and sample. Within
+// a run the t's follow from its first one alone, so the generate pass neither
+// skips through empty cells nor looks up occupancy again. A ray of more runs
+// (their number is still counted) is marched a second time.
+constexpr uint32_t kRunRecords = 16;
+struct RunLog {
+    uint2* rec;  // the ray's records; null in all lanes but the group's first
+    uint32_t n = 0;
+    float t_end = 0.0f;
+    TN_DEVICE void run(bool first, float t, uint32_t sample, float t_after) {
+        if (first) {
+            ++n;
+            if (rec && n < kRunRecords) rec[n] = make_uint2(__float_as_uint(t), sample);
+        }
+        t_end = t_after;
+    }
+    TN_DEVICE void close() {
+        if (rec) rec[0] = make_uint2(n, __float_as_uint(t_end));
+    }
+};
+
 struct MarchCountArgs {
     uint32_t n_rays, B, max_steps;
     const float *dir, *tmax, *ori, *t;
     uint8_t* alive;
     uint32_t* n_steps;
+    uint2* runs;  // null: none wanted
 };
 
 template <int G, bool ML>
@@ -270,12 +301,14 @@ TN_DEVICE void march_count_rays(const MarchCountArgs& a, const tn_bbox_t& bbox, 
     // whole waves: every lane of a wave takes part in the group operations
     for (uint32_t w = tid & ~63u; w / G < a.n_rays; w += n_threads) {
         const uint32_t i = (w + (tid & 63u)) / G;
-        const bool own = i < a.n_rays;
+        const bool own = i < a.n_rays, first = (tid & (uint32_t)(G - 1)) == 0;
         const bool active = own && a.alive[i] != 0;
         const MarchRay r = load_ray(active, i, a.B, a.ori, a.dir);
+        RunLog log{a.runs && active && first ? a.runs + (uint64_t)i * kRunRecords : nullptr};
         const uint32_t n = march_group<G, ML, true>(active, r, active ? a.t[i] : 0.0f, active ? a.tmax[i] : 0.0f,
-                                                  a.max_steps, bbox, g, st, [](uint32_t, float) {});
-        if (own && (tid & (uint32_t)(G - 1)) == 0) {
+                                                    a.max_steps, bbox, g, st, [](uint32_t, float) {}, log);
+        log.close();
+        if (own && first) {
             if (active && n == 0) a.alive[i] = 0;
             a.n_steps[i] = n;
         }
@@ -286,11 +319,12 @@ __global__ void __launch_bounds__(64 * kMarchWaves)
 march_count_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ d_n_rays, uint32_t B, tn_bbox_t bbox,
                    tn_occupancy_grid_t grid, float cone, float dt_min, float dt_max, uint32_t max_steps,
                    const float* __restrict__ dir, const float* __restrict__ ray_tmax, uint8_t* __restrict__ ray_alive,
-                   const float* __restrict__ ori, const float* __restrict__ ray_t, uint32_t* __restrict__ n_steps) {
+                   const float* __restrict__ ori, const float* __restrict__ ray_t, uint32_t* __restrict__ n_steps,
+                   uint2* __restrict__ runs) {
     const uint32_t n_rays = d_n_rays ? min(*d_n_rays, n_rays_max) : n_rays_max;
     const MarchGrid g = make_grid(grid);
     const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
-    const MarchCountArgs a = {n_rays, B, max_steps, dir, ray_tmax, ori, ray_t, ray_alive, n_steps};
+    const MarchCountArgs a = {n_rays, B, max_steps, dir, ray_tmax, ori, ray_t, ray_alive, n_steps, runs};
     if (grid.n_levels == 1) {
         if (n_rays <= kGroup16Rays) march_count_rays<16, false>(a, bbox, g, st);
         else march_count_rays<8, false>(a, bbox, g, st);
@@ -440,11 +474,13 @@ TN_DEVICE void march_generate_rays(const MarchGenerateArgs& a, const tn_bbox_t& 
         const bool active = i < a.n_rays && a.alive[i] != 0;
         const MarchRay r = load_ray(active, i, a.B, a.ori, a.dir);
         const uint32_t off = active ? a.offset[i] : 0u;
+        NoLog log;
         march_group<G, ML, false>(active, r, active ? a.t[i] : 0.0f, INFINITY, active ? a.n_steps[i] : 0u, bbox, g, st,
-                                [&](uint32_t n, float t) {
-                                    a.out_t[off + n] = t;
-                                    a.out_ray[off + n] = i;
-                                });
+                                  [&](uint32_t n, float t) {
+                                      a.out_t[off + n] = t;
+                                      a.out_ray[off + n] = i;
+                                  },
+                                  log);
     }
 }
 
@@ -505,6 +541,123 @@ __global__ void march_expand_kernel(uint32_t n_rays_max, uint32_t SB_max, const 
     out_dir[sid + 2 * SB] = 0.5f * dir[r + 2 * B] + 0.5f;
     out_m_norm[sid] = fminf(fmaxf(((t + 0.5f * dt) - t_min) / t_span, 0.0f), 1.0f);
     out_dt_norm[sid] = dt / t_span;
+}
+
+// Where a sample's words go; the normalised steps, t and image ids may be null
+// (a render reads none).
+struct SampleOut {
+    uint32_t* __restrict__ img_id;
+    float *__restrict__ t, *__restrict__ pos, *__restrict__ dir, *__restrict__ dt, *__restrict__ m_norm,
+        *__restrict__ dt_norm;
+    uint32_t SB;
+};
+
+// Sample sid at t of a ray that starts at t_min and whose last sample's step
+// ends at t_end (march_expand_kernel's expressions)
+TN_DEVICE void write_sample(const SampleOut& o, uint32_t sid, float t, const MarchRay& r, float t_min, float t_end,
+                            uint32_t img, float inv_aabb, const MarchStep& st) {
+    if (sid >= o.SB) return;
+    const float dt = step_dt(st, t);
+    const float x = r.ox + t * r.dx, y = r.oy + t * r.dy, z = r.oz + t * r.dz;
+    const float t_span = fmaxf(t_end - t_min, 1e-6f);
+    if (o.img_id) o.img_id[sid] = img;
+    if (o.t) o.t[sid] = t;
+    o.dt[sid] = inv_aabb * dt;
+    o.pos[sid] = fminf(fmaxf(x * inv_aabb + 0.5f, 0.0f), 1.0f);
+    o.pos[sid + o.SB] = fminf(fmaxf(y * inv_aabb + 0.5f, 0.0f), 1.0f);
+    o.pos[sid + 2 * (uint64_t)o.SB] = fminf(fmaxf(z * inv_aabb + 0.5f, 0.0f), 1.0f);
+    o.dir[sid] = 0.5f * r.dx + 0.5f;
+    o.dir[sid + o.SB] = 0.5f * r.dy + 0.5f;
+    o.dir[sid + 2 * (uint64_t)o.SB] = 0.5f * r.dz + 0.5f;
+    if (o.m_norm) o.m_norm[sid] = fminf(fmaxf(((t + 0.5f * dt) - t_min) / t_span, 0.0f), 1.0f);
+    if (o.dt_norm) o.dt_norm[sid] = dt / t_span;
+}
+
+// The generate pass from the count pass's runs: 16 lanes per ray form 16 t's of
+// a run at a time and write the samples' words at once, in rows of 16. Bound
+// by the serial chain of 15 step sizes per 16 samples and the 36 or 52 bytes
+// per sample; 8 lanes per ray would halve the rows, 64 quadruple the chain.
+// Against marching again and expanding in a second launch, per pass: 23 us
+// (was 36 + 4) for a training step of 1,900 rays, 24 (was 39 + 10) for 20,000
+// rendered rays, 32 (was 39 + 25) for 130,000 rays and 4.2 M samples, 43 (was
+// 168 + 14) in a scene of 16 units, where most steps are skips. The count
+// pass's 128 bytes per ray cost it 1 to 2 us.
+template <bool ML>
+TN_DEVICE void march_generate_from_runs(uint32_t n_rays, uint32_t B, const tn_bbox_t& bbox, const MarchGrid& g,
+                                        const MarchStep& st, float inv_aabb, const float* __restrict__ ori,
+                                        const float* __restrict__ dir, const float* __restrict__ ray_t,
+                                        const uint32_t* __restrict__ ray_offset, const uint8_t* __restrict__ ray_alive,
+                                        const uint32_t* __restrict__ n_ray_steps,
+                                        const uint32_t* __restrict__ ray_img_id, const uint2* __restrict__ runs,
+                                        const SampleOut& o) {
+    constexpr int G = 16;
+    const uint32_t n_threads = gridDim.x * blockDim.x, tid = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t j = tid & (uint32_t)(G - 1);
+    for (uint32_t w = tid & ~63u; w / G < n_rays; w += n_threads) {
+        const uint32_t i = (w + (tid & 63u)) / G;
+        const bool active = i < n_rays && ray_alive[i] != 0;
+        const MarchRay r = load_ray(active, i, B, ori, dir);
+        const uint32_t off = active ? ray_offset[i] : 0u, ns = active ? n_ray_steps[i] : 0u;
+        const uint32_t img = active && o.img_id ? ray_img_id[i] : 0u;
+        const float t_min = active ? ray_t[i] : 0.0f;
+        const uint2 rec = active ? runs[(uint64_t)i * kRunRecords + j] : make_uint2(0u, 0u);
+        const float rec_t = __uint_as_float(rec.x), rec_n = __uint_as_float(rec.y);
+        const uint32_t nr = __float_as_uint(group_get<G>(rec_t, 0));
+        const float t_end = group_get<G>(rec_n, 0);
+        const bool again = nr >= kRunRecords;  // more runs than records
+        auto emit = [&](uint32_t n, float t) { write_sample(o, off + n, t, r, t_min, t_end, img, inv_aabb, st); };
+        uint32_t q = 0, n = 0, n1 = 0;  // run, next sample, the run's end
+        float t = 0.0f;
+        bool done = !active || again;
+        while (__ballot(!done) != 0ull) {
+            // (all lanes: the group reads its records across lanes)
+            const bool next = n == n1;
+            const uint32_t q1 = next ? q + 1 : q;
+            const float t_q = group_get<G>(rec_t, min(q1, (uint32_t)G - 1u));
+            const uint32_t n_q = __float_as_uint(group_get<G>(rec_n, min(q1 + 1u, (uint32_t)G - 1u)));
+            if (next) {
+                q = q1;
+                t = t_q;
+                n1 = q < nr ? n_q : ns;
+            }
+            float tj = t;
+            if (st.dt_min == st.dt_max) {
+#pragma unroll
+                for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k) tj = j > k ? tj + st.dt_min : tj;
+            } else {
+#pragma unroll
+                for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k) tj = j > k ? tj + step_dt(st, tj) : tj;
+            }
+            const uint32_t f = min((uint32_t)G, n1 - n);
+            if (!done && j < f) emit(n + j, tj);
+            const float t16 = group_get<G>(tj + step_dt(st, tj), (uint32_t)G - 1u);
+            n += f;
+            t = t16;  // used only when the run goes on past 16 samples
+            done = done || n >= ns || (n == n1 && q >= nr);
+        }
+        if (__ballot(active && again) != 0ull) {
+            NoLog log;
+            march_group<G, ML, false>(active && again, r, t_min, INFINITY, ns, bbox, g, st, emit, log);
+        }
+    }
+}
+
+__global__ void __launch_bounds__(64 * kMarchWaves)
+march_generate_runs_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ info, uint32_t B, tn_bbox_t bbox,
+                           float inv_aabb, tn_occupancy_grid_t grid, float dt_min, float dt_max, float cone,
+                           const uint32_t* __restrict__ ray_img_id, const float* __restrict__ ori,
+                           const float* __restrict__ dir, const float* __restrict__ ray_t,
+                           const uint32_t* __restrict__ ray_offset, const uint8_t* __restrict__ ray_alive,
+                           const uint32_t* __restrict__ n_ray_steps, const uint2* __restrict__ runs, SampleOut o) {
+    const uint32_t n_rays = min(info[0], n_rays_max);
+    const MarchGrid g = make_grid(grid);
+    const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
+    if (grid.n_levels == 1)
+        march_generate_from_runs<false>(n_rays, B, bbox, g, st, inv_aabb, ori, dir, ray_t, ray_offset, ray_alive,
+                                        n_ray_steps, ray_img_id, runs, o);
+    else
+        march_generate_from_runs<true>(n_rays, B, bbox, g, st, inv_aabb, ori, dir, ray_t, ray_offset, ray_alive,
+                                       n_ray_steps, ray_img_id, runs, o);
 }
 
 // Next step's ray count: the rays that would fill the sample budget at this
@@ -646,20 +799,41 @@ extern "C" int tn_batch_tail(const uint32_t* info, uint32_t first, uint32_t* tai
     return TN_OK;
 }
 
-extern "C" int tn_march_count(uint32_t n_rays_max, const uint32_t* d_n_rays, uint32_t stride,
-                              tn_bbox_t bbox, tn_occupancy_grid_t grid, float cone_angle, float dt_min,
-                              float dt_max, uint32_t max_steps, const float* dir, const float* ray_tmax,
-                              uint8_t* ray_alive, const float* ori, const float* ray_t, uint32_t* n_steps,
-                              hipStream_t stream) {
+static int march_count(uint32_t n_rays_max, const uint32_t* d_n_rays, uint32_t stride, tn_bbox_t bbox,
+                       tn_occupancy_grid_t grid, float cone_angle, float dt_min, float dt_max, uint32_t max_steps,
+                       const float* dir, const float* ray_tmax, uint8_t* ray_alive, const float* ori,
+                       const float* ray_t, uint32_t* n_steps, void* runs, hipStream_t stream) {
     TN_CHECK_ARG(dir && ray_tmax && ray_alive && ori && ray_t && n_steps && grid.bitfield);
     TN_CHECK_ARG(n_rays_max <= stride && grid.n_levels >= 1 && grid.n_levels <= 8);
     TN_CHECK_ARG(grid.resolution >= 2 && grid.resolution <= 1024 && dt_min > 0.0f && dt_max >= dt_min);
     if (n_rays_max == 0) return TN_OK;
     march_count_kernel<<<march_blocks(n_rays_max), 64 * kMarchWaves, 0, stream>>>(
         n_rays_max, d_n_rays, stride, bbox, grid, cone_angle, dt_min, dt_max, max_steps, dir, ray_tmax,
-        ray_alive, ori, ray_t, n_steps);
+        ray_alive, ori, ray_t, n_steps, static_cast<uint2*>(runs));
     TN_CHECK_LAUNCH();
     return TN_OK;
+}
+
+extern "C" int tn_march_count(uint32_t n_rays_max, const uint32_t* d_n_rays, uint32_t stride,
+                              tn_bbox_t bbox, tn_occupancy_grid_t grid, float cone_angle, float dt_min,
+                              float dt_max, uint32_t max_steps, const float* dir, const float* ray_tmax,
+                              uint8_t* ray_alive, const float* ori, const float* ray_t, uint32_t* n_steps,
+                              hipStream_t stream) {
+    return march_count(n_rays_max, d_n_rays, stride, bbox, grid, cone_angle, dt_min, dt_max, max_steps, dir, ray_tmax,
+                       ray_alive, ori, ray_t, n_steps, nullptr, stream);
+}
+
+extern "C" size_t tn_march_runs_bytes(uint32_t n_rays_max) { return (size_t)n_rays_max * kRunRecords * sizeof(uint2); }
+
+extern "C" int tn_march_count_runs(uint32_t n_rays_max, const uint32_t* d_n_rays, uint32_t stride, tn_bbox_t bbox,
+                                   tn_occupancy_grid_t grid, float cone_angle, float dt_min, float dt_max,
+                                   uint32_t max_steps, const float* dir, const float* ray_tmax, uint8_t* ray_alive,
+                                   const float* ori, const float* ray_t, uint32_t* n_steps, void* runs,
+                                   size_t runs_bytes, hipStream_t stream) {
+    TN_CHECK_ARG(runs && (reinterpret_cast<uintptr_t>(runs) & 127) == 0);
+    if (runs_bytes < tn_march_runs_bytes(n_rays_max)) return TN_ERR_OUT_OF_MEMORY;
+    return march_count(n_rays_max, d_n_rays, stride, bbox, grid, cone_angle, dt_min, dt_max, max_steps, dir, ray_tmax,
+                       ray_alive, ori, ray_t, n_steps, runs, stream);
 }
 
 extern "C" size_t tn_scan_workspace_bytes(uint32_t n) {
@@ -702,6 +876,28 @@ extern "C" int tn_march_generate(uint32_t n_rays_max, const uint32_t* info, uint
     march_expand_kernel<<<blocks_for(sample_stride, 256), 256, 0, stream>>>(
         n_rays_max, sample_stride, info, stride, sample_stride, inv_aabb, dt_min, dt_max, cone_angle, ray_img_id, ori,
         dir, ray_t, ray_offset, n_ray_steps, out_img_id, out_t, out_pos, out_dir, out_dt, out_m_norm, out_dt_norm);
+    TN_CHECK_LAUNCH();
+    return TN_OK;
+}
+
+extern "C" int tn_march_generate_runs(uint32_t n_rays_max, const uint32_t* info, uint32_t stride,
+                                      uint32_t sample_stride, tn_bbox_t bbox, float inv_aabb,
+                                      tn_occupancy_grid_t grid, float dt_min, float dt_max, float cone_angle,
+                                      const uint32_t* ray_img_id, const float* ori, const float* dir,
+                                      const float* ray_t, const uint32_t* ray_offset, const uint8_t* ray_alive,
+                                      const uint32_t* n_ray_steps, const void* runs, size_t runs_bytes,
+                                      uint32_t* out_img_id, float* out_t, float* out_pos, float* out_dir,
+                                      float* out_dt, float* out_m_norm, float* out_dt_norm, hipStream_t stream) {
+    TN_CHECK_ARG(ori && dir && ray_t && ray_offset && ray_alive && n_ray_steps && out_pos && out_dir && out_dt &&
+                 grid.bitfield && (!out_img_id || ray_img_id));
+    TN_CHECK_ARG(n_rays_max <= stride && grid.n_levels >= 1 && grid.n_levels <= 8 && dt_min > 0.0f && dt_max >= dt_min);
+    TN_CHECK_ARG(info != nullptr && sample_stride > 0 && runs && (reinterpret_cast<uintptr_t>(runs) & 127) == 0);
+    if (runs_bytes < tn_march_runs_bytes(n_rays_max)) return TN_ERR_OUT_OF_MEMORY;
+    if (n_rays_max == 0) return TN_OK;
+    march_generate_runs_kernel<<<march_blocks(n_rays_max), 64 * kMarchWaves, 0, stream>>>(
+        n_rays_max, info, stride, bbox, inv_aabb, grid, dt_min, dt_max, cone_angle, ray_img_id, ori, dir, ray_t,
+        ray_offset, ray_alive, n_ray_steps, static_cast<const uint2*>(runs),
+        SampleOut{out_img_id, out_t, out_pos, out_dir, out_dt, out_m_norm, out_dt_norm, sample_stride});
     TN_CHECK_LAUNCH();
     return TN_OK;
 }
