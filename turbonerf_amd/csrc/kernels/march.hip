@@ -13,24 +13,66 @@
 
 namespace tn {
 
+// Level k of the grid spans 2^k box units, and a point's level (grid_level_at)
+// is the first with 2^k / 2 > |coordinate| and 2^k inv_res > dt. That only adds
+// k to exponents, so levels are held as the exponent field of a float,
+// kLevel0 + k << 23, and what is scaled by 2^k or 2^-k follows from it by one
+// integer addition.
+constexpr uint32_t kExponent = 0xFF800000u;  // sign and exponent
+constexpr int kLevel0 = 0x3E800000;          // 0.25: a coordinate in [0.5, 1) is level 1's
+
 struct MarchGrid {
     const uint8_t* bits;
-    int n_levels;
+    int top;         // the highest level
     float res_f;
     float inv_res;
+    float half_res;
     uint32_t lim;
     float level_scale;  // the cascade is chosen from dt * level_scale
+    int dt_bias;        // bits of (dt * level_scale) - dt_bias: the level that dt asks for, rounded down to an exponent
+    int res_bias;       // res_bias - level: bits of res 2^-k
+    int cell_bias;      // cell_bias + level: bits of 2^k / res
 };
 
 TN_DEVICE MarchGrid make_grid(const tn_occupancy_grid_t& g) {
     MarchGrid m;
     m.bits = g.bitfield;
-    m.n_levels = g.n_levels;
+    m.top = kLevel0 + ((g.n_levels - 1) << 23);
     m.res_f = (float)g.resolution;
     m.inv_res = 1.0f / m.res_f;
+    m.half_res = 0.5f * m.res_f;
     m.lim = (uint32_t)g.resolution - 1u;
     m.level_scale = g.level_dt_scale > 0.0f ? g.level_dt_scale : 1.0f;
+    m.dt_bias = __float_as_int(m.inv_res) - (1 << 23) - kLevel0;
+    m.res_bias = __float_as_int(m.res_f) + kLevel0;
+    m.cell_bias = __float_as_int(m.inv_res) - kLevel0;
     return m;
+}
+
+// What a marching kernel is compiled for. SEVERAL cascades; POW2: the
+// resolution is a power of two, so that (x 2^-k + 1/2) res is one fused
+// multiply-add with the same rounding; DT: a step may be longer than a cell of
+// level 0 and so decide the level (training in a large box; a render's steps
+// are normalised by the scene size and never are).
+template <bool SEVERAL_, bool POW2_, bool DT_>
+struct GridForm {
+    static constexpr bool SEVERAL = SEVERAL_, POW2 = POW2_, DT = DT_;
+};
+// fn with the form for a launch on `grid`
+template <typename Fn>
+inline void with_grid_form(const tn_occupancy_grid_t& grid, float dt_max, Fn fn) {
+    const bool pow2 = (grid.resolution & (grid.resolution - 1)) == 0;
+    const float level_scale = grid.level_dt_scale > 0.0f ? grid.level_dt_scale : 1.0f;
+    if (grid.n_levels == 1) {
+        if (pow2) fn(GridForm<false, true, false>{});
+        else fn(GridForm<false, false, false>{});
+    } else if (!pow2) {
+        fn(GridForm<true, false, true>{});
+    } else if (dt_max * level_scale < 1.0f / (float)grid.resolution) {
+        fn(GridForm<true, true, false>{});
+    } else {
+        fn(GridForm<true, true, true>{});
+    }
 }
 
 // Marching follows the reference's serial recurrence exactly (contraction
@@ -52,11 +94,19 @@ TN_DEVICE MarchGrid make_grid(const tn_occupancy_grid_t& g) {
 //    across the quad, which leaves about a third of the instructions;
 //  * the step's division by dt_min, rounded upwards, is by a constant: its
 //    reciprocal is formed once (div_up);
-//  * the cascade of a point is formed from exponents, without a loop.
-// A skip step is 24 vector instructions in one cascade and 36 in several. A
-// wave per ray that looked every skip step's cell up in turn took 214 us to
+//  * the cascade of a point is formed from exponents, without a loop, and
+//    where the resolution is a power of two or a step cannot decide the
+//    cascade, the kernels are compiled without what that takes (GridForm);
+//  * the groups of a wave that run and those that skip share a block's test.
+// A skip step is 20 vector instructions in one cascade and 28 or 34 in several;
+// a test about 80 and one load. Few rays are bound by the latency of the
+// chain and of that load, many rays by instruction issue: 65,000 rays through
+// a 16-unit scene issued vector instructions in nine cycles of ten.
+// A wave per ray that looked every skip step's cell up in turn took 214 us to
 // count and 116 us to generate a batch of 4,369 rays through a unit box with
-// 8 blobs, and 120 us to count 53 rays; this takes 51, 47 and 42 us.
+// 8 blobs, and 120 us to count 53 rays; this takes 49, 40 and 39 us. A render
+// pass of 65,000 rays in the 16-unit scene takes 290 us to count (380 with 24
+// and 36 instructions per skip step and a test for runs and skips each).
 // G is 16 for up to kGroup16Rays rays and 8 for more (see there).
 struct MarchStep {
     float cone, dt_min, dt_max, inv_dt_min;
@@ -75,52 +125,76 @@ struct MarchRay {
 TN_DEVICE float div_up(float a, float b, float y) {
     const float q0 = a * y;
     const float q = __builtin_fmaf(__builtin_fmaf(-q0, b, a), y, q0);
-    return __uint_as_float(__float_as_uint(q) + (__builtin_fmaf(-q, b, a) > 0.0f ? 1u : 0u));
+    const uint32_t below = __float_as_uint(__builtin_fmaf(q, b, -a)) >> 31;  // q b < a
+    return __uint_as_float(__float_as_uint(q) + below);
 }
 
-// The cascade (grid_level_at) of a point whose largest |coordinate| has the
-// bits m, from the step dt that decides it: level k covers the point when
-// 2^k / 2 > |coordinate| and 2^k inv_res > dt. 2^k only adds k to the exponent,
-// so the first such k follows from the difference of the bit patterns, rounded
-// up to a whole exponent; `bits` is k << 23, which added to a float's pattern
-// multiplies it by 2^k (no zeros or overflows here: n_levels <= 8).
-struct Cascade {
-    int bits;
-    TN_DEVICE int level() const { return bits >> 23; }
-    TN_DEVICE float inv_scale() const { return __uint_as_float(0x3F800000u - (uint32_t)bits); }  // 2^-k
-    TN_DEVICE float scaled(float v) const { return __uint_as_float(__float_as_uint(v) + (uint32_t)bits); }
-};
-constexpr int kExponentOne = 1 << 23;
-TN_DEVICE Cascade cascade_of(int n_levels, float inv_res, uint32_t m, float dt) {
-    const int d1 = (int)m - ((int)0x3F000000 - kExponentOne);  // 0x3F000000: 0.5
-    const int d2 = (int)__float_as_uint(dt) - ((int)__float_as_uint(inv_res) - kExponentOne);
-    const int k = max(d1, d2) & ~(kExponentOne - 1);
-    return Cascade{min(max(k, 0), (n_levels - 1) << 23)};
-}
 // get_dt; dt_min <= dt_max
 TN_DEVICE float step_dt(const MarchStep& st, float t) {
     return __builtin_amdgcn_fmed3f(t * st.cone, st.dt_min, st.dt_max);
 }
 TN_DEVICE uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7FFFFFFFu; }
 
-// occupancy of the cell at (x, y, z); ML: several cascades
-template <bool ML>
-TN_DEVICE bool point_occupied(const MarchGrid& g, const MarchStep& st, float t, float x, float y, float z) {
-    Cascade c{0};
-    if constexpr (ML)
-        c = cascade_of(g.n_levels, g.inv_res, max(max(abs_bits(x), abs_bits(y)), abs_bits(z)),
-                       step_dt(st, t) * g.level_scale);
-    const float s = ML ? c.inv_scale() : 1.0f;
-    const uint32_t xu = min((uint32_t)fmaxf((x * s + 0.5f) * g.res_f, 0.0f), g.lim);
-    const uint32_t yu = min((uint32_t)fmaxf((y * s + 0.5f) * g.res_f, 0.0f), g.lim);
-    const uint32_t zu = min((uint32_t)fmaxf((z * s + 0.5f) * g.res_f, 0.0f), g.lim);
-    return ((g.bits[morton3d(xu, yu, zu)] >> (ML ? c.level() : 0)) & 1u) != 0u;
+// the level, as kLevel0 + k << 23, of a point whose largest |coordinate| has the bits m, at t
+template <typename F>
+TN_DEVICE int level_bits(const MarchGrid& g, const MarchStep& st, uint32_t m, float t) {
+    int e = (int)m;
+    if constexpr (F::DT) e = max(e, __float_as_int(step_dt(st, t) * g.level_scale) - g.dt_bias);
+    // (as floats: these are powers of two, infinity or below level 0)
+    return __float_as_int(__builtin_amdgcn_fmed3f(__int_as_float(e & (int)kExponent), __int_as_float(kLevel0),
+                                                  __int_as_float(g.top)));
 }
 
-// distance to the next cell boundary along one axis: gc the coordinate in
-// cells, h = copysign(0.5, d), id = 1 / d, k the cell's side
+// (v 2^-k + 1/2) res, k the level of `level`
+template <typename F>
+TN_DEVICE float cell_coord(const MarchGrid& g, float v, int level) {
+    if constexpr (F::POW2)
+        return __builtin_fmaf(v, F::SEVERAL ? __int_as_float(g.res_bias - level) : g.res_f, g.half_res);
+    if constexpr (F::SEVERAL) v *= __int_as_float(0x3F800000 + kLevel0 - level);
+    return (v + 0.5f) * g.res_f;
+}
+// index of a cell coordinate: truncated, at least 0 (the conversion takes
+// negative values and NaN to 0), at most the last
+TN_DEVICE uint32_t cell_index(const MarchGrid& g, float c) {
+    uint32_t i;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(i) : "v"(c));
+    return min(i, g.lim);
+}
+// Every third bit of a word. The empty assembly keeps the compiler from
+// merging the stages into more instructions and the last one into a multiply,
+// which takes as long as four.
+TN_DEVICE uint32_t spread_bits(uint32_t v) {
+    v = (v | (v << 16)) & 0x030000FFu;
+    asm("" : "+v"(v));
+    v = (v | (v << 8)) & 0x0300F00Fu;
+    asm("" : "+v"(v));
+    v = (v | (v << 4)) & 0x030C30C3u;
+    asm("" : "+v"(v));
+    v = (v | (v << 2)) & 0x09249249u;
+    asm("" : "+v"(v));
+    return v;
+}
+
+// occupancy of the cell at (x, y, z)
+template <typename F>
+TN_DEVICE bool point_occupied(const MarchGrid& g, const MarchStep& st, float t, float x, float y, float z) {
+    int level = kLevel0;
+    if constexpr (F::SEVERAL) level = level_bits<F>(g, st, max(max(abs_bits(x), abs_bits(y)), abs_bits(z)), t);
+    const uint32_t xu = spread_bits(cell_index(g, cell_coord<F>(g, x, level)));
+    const uint32_t yu = spread_bits(cell_index(g, cell_coord<F>(g, y, level)));
+    const uint32_t zu = spread_bits(cell_index(g, cell_coord<F>(g, z, level)));
+    const uint32_t bits = g.bits[xu | (yu << 1) | (zu << 2)];
+    return ((F::SEVERAL ? bits >> ((level - kLevel0) >> 23) : bits) & 1u) != 0u;
+}
+
+// The distance to the next cell boundary along one axis, gc the coordinate in
+// cells, h = copysign(0.5, d), id = 1 / d, k the cell's side: in one cascade of
+// a power-of-two resolution the side is a constant power of two below 1 and
+// already in id, which rounds alike.
+template <typename F>
 TN_DEVICE float axis_distance(float gc, float h, float id, float k) {
-    return k * ((floorf(h + gc + 0.5f) - gc) * id);
+    const float d = (floorf(h + gc + 0.5f) - gc) * id;
+    return F::POW2 && !F::SEVERAL ? d : k * d;
 }
 
 // max(lo, minimum of v over the quad), a NaN (a ray along a cell face) left out
@@ -129,10 +203,13 @@ TN_DEVICE float axis_distance(float gc, float h, float id, float k) {
 // needs after a vector write are part of it.
 TN_DEVICE float quad_min_above(float v, float lo) {
     float a, b;
-    asm("s_nop 1\n\tv_min_f32_dpp %0, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf" : "=&v"(a) : "v"(v));
-    asm("s_nop 1\n\tv_min_f32_dpp %0, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\tv_max_f32 %0, %2, %0"
-        : "=&v"(b)
-        : "v"(a), "s"(lo));
+    asm("s_nop 1\n\t"
+        "v_min_f32_dpp %0, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_min_f32_dpp %1, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32 %1, %3, %1"
+        : "=&v"(a), "=&v"(b)
+        : "v"(v), "s"(lo));
     return b;
 }
 TN_DEVICE uint32_t quad_max(uint32_t v) {
@@ -140,12 +217,22 @@ TN_DEVICE uint32_t quad_max(uint32_t v) {
     return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true));  // lanes 2 3 0 1
 }
 
+// the group's bits of `ballot`
+template <int G>
+TN_DEVICE uint32_t group_bits(uint64_t ballot) {
+    const uint32_t lane = __lane_id();
+    const uint32_t half = lane < 32u ? (uint32_t)ballot : (uint32_t)(ballot >> 32);
+    return (half >> (lane & 31u & ~(uint32_t)(G - 1))) & ((1u << G) - 1u);
+}
 // index of the group's first lane with a set bit of `ballot`, or G (8 or 16)
 template <int G>
 TN_DEVICE uint32_t group_first(uint64_t ballot) {
-    const uint32_t lane = __lane_id();
-    const uint32_t half = lane < 32u ? (uint32_t)ballot : (uint32_t)(ballot >> 32);
-    return (uint32_t)__builtin_ctz((half >> (lane & 31u & ~(uint32_t)(G - 1))) | (1u << G));
+    return (uint32_t)__builtin_ctz(group_bits<G>(ballot) | (1u << G));
+}
+// the bit of the group's lane j <= G (false for G)
+template <int G>
+TN_DEVICE bool group_bit(uint64_t ballot, uint32_t j) {
+    return ((group_bits<G>(ballot) >> j) & 1u) != 0u;
 }
 // v of the group's lane j
 template <int G>
@@ -163,19 +250,24 @@ TN_DEVICE float group_get(float v, uint32_t j) {
 struct NoLog {
     TN_DEVICE void run(bool, float, uint32_t, float) {}
 };
-template <int G, bool ML, bool COUNT, typename Emit, typename Log>
+template <int G, typename F, bool COUNT, typename Emit, typename Log>
 TN_DEVICE uint32_t march_group(bool active, const MarchRay& r, float t, float t_max, uint32_t max_n,
                                const tn_bbox_t& bbox, const MarchGrid& g, const MarchStep& st, Emit emit, Log& log) {
     const uint32_t lane = __lane_id(), j = lane & (uint32_t)(G - 1), axis = lane & 3u;
     const float oa = axis == 0 ? r.ox : axis == 1 ? r.oy : r.oz;
     const float da = axis == 0 ? r.dx : axis == 1 ? r.dy : r.dz;
-    const float ida = 1.0f / da, ha = 0.5f * copysignf(1.0f, da);
+    const float ha = 0.5f * copysignf(1.0f, da);
+    float ida = 1.0f / da;
+    if constexpr (F::POW2 && !F::SEVERAL) ida *= g.inv_res;  // see axis_distance
     uint32_t n = 0;
     bool done = !active, skip = false, open = false;  // open: the last block's run goes on
-    while (__ballot(!done) != 0ull) {
-        if (__ballot(!done && !skip) != 0ull) {
+    for (;;) {
+        const uint64_t runs = __builtin_amdgcn_ballot_w64(!done && !skip);
+        const uint64_t skips = __builtin_amdgcn_ballot_w64(!done && skip);
+        if ((runs | skips) == 0ull) break;
+        float tj = t;
+        if (runs != 0ull) {
             // a run: lane j's t after j more samples
-            float tj = t;
             if (st.dt_min == st.dt_max) {
 #pragma unroll
                 for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k) tj = j > k ? tj + st.dt_min : tj;
@@ -184,54 +276,50 @@ TN_DEVICE uint32_t march_group(bool active, const MarchRay& r, float t, float t_
                 for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k)
                     tj = j > k ? tj + step_dt(st, tj) : tj;
             }
-            const float x = r.ox + tj * r.dx, y = r.oy + tj * r.dy, z = r.oz + tj * r.dz;
-            const bool inside = bbox_contains(bbox, x, y, z);
-            const bool within = !done && !skip && j < max_n - n && (!COUNT || tj < t_max) && inside;
-            const bool good = within && point_occupied<ML>(g, st, tj, x, y, z);
-            const uint32_t f = group_first<G>(__ballot(!good));
-            const uint32_t e = group_first<G>(__ballot(within && !good));
-            const float tn = tj + step_dt(st, tj);
-            const float t_f = group_get<G>(f < (uint32_t)G ? tj : tn, f < (uint32_t)G ? f : (uint32_t)G - 1u);
-            if (!done && !skip) {
+        }
+        if (skips != 0ull) {
+            // a skip from an empty cell: lane j's t after j + 1 steps
+            float tc = t, ts = t;
+#pragma unroll
+            for (uint32_t k = 0; k < (uint32_t)G; ++k) {
+                const float p = oa + tc * da;
+                int level = kLevel0;
+                float cell = g.inv_res;
+                if constexpr (F::SEVERAL) {
+                    level = level_bits<F>(g, st, quad_max(abs_bits(p)), tc);
+                    cell = __int_as_float(g.cell_bias + level);
+                }
+                const float gc = cell_coord<F>(g, p, level);
+                const float d = quad_min_above(axis_distance<F>(gc, ha, ida, cell), st.dt_min);
+                tc += div_up(d, st.dt_min, st.inv_dt_min) * st.dt_min;
+                ts = j == k ? tc : ts;
+            }
+            tj = skip ? ts : tj;
+        }
+        // one test for both: f is the first lane that ends the group's run or skip
+        const float x = r.ox + tj * r.dx, y = r.oy + tj * r.dy, z = r.oz + tj * r.dz;
+        const bool within = !done && (skip || j < max_n - n) && (!COUNT || tj < t_max) && bbox_contains(bbox, x, y, z);
+        const bool occupied = within && point_occupied<F>(g, st, tj, x, y, z);
+        const uint32_t f = group_first<G>(__builtin_amdgcn_ballot_w64(!within || occupied == skip));
+        const bool in_f = group_bit<G>(__builtin_amdgcn_ballot_w64(within), f);  // false for f == G
+        const float t_end = skip ? tj : tj + step_dt(st, tj);  // of lane G - 1, which a whole block goes on from
+        const float t_f = group_get<G>(f < (uint32_t)G ? tj : t_end, min(f, (uint32_t)G - 1u));
+        if (!done) {
+            if (!skip) {
                 if (j < f) emit(n + j, tj);
                 if (f != 0u) log.run(!open, t, n, t_f);
                 open = f == (uint32_t)G;
                 n += f;
-                t = t_f;
-                skip = f < (uint32_t)G && e == f;  // the run ended at an empty cell
-                if (f < (uint32_t)G && !skip) {
+            }
+            t = t_f;
+            if (f < (uint32_t)G) {
+                if (in_f) {
+                    skip = !skip;
+                } else {
                     if (!COUNT)
                         for (uint32_t k = n + j; k < max_n; k += (uint32_t)G) emit(k, t);
                     done = true;
                 }
-            }
-        }
-        if (__ballot(!done && skip) != 0ull) {
-            // a skip from an empty cell: lane j's t after j + 1 steps
-            float tc = t, tj = t;
-#pragma unroll
-            for (uint32_t k = 0; k < (uint32_t)G; ++k) {
-                const float p = oa + tc * da;
-                float s = 1.0f, cell = g.inv_res;
-                if constexpr (ML) {
-                    const Cascade c = cascade_of(g.n_levels, g.inv_res, quad_max(abs_bits(p)),
-                                                 step_dt(st, tc) * g.level_scale);
-                    s = c.inv_scale();
-                    cell = c.scaled(g.inv_res);
-                }
-                const float gc = (p * s + 0.5f) * g.res_f;
-                const float d = quad_min_above(axis_distance(gc, ha, ida, cell), st.dt_min);
-                tc += div_up(d, st.dt_min, st.inv_dt_min) * st.dt_min;
-                tj = j == k ? tc : tj;
-            }
-            const float x = r.ox + tj * r.dx, y = r.oy + tj * r.dy, z = r.oz + tj * r.dz;
-            const bool within = !done && skip && (!COUNT || tj < t_max) && bbox_contains(bbox, x, y, z);
-            const bool occupied = within && point_occupied<ML>(g, st, tj, x, y, z);
-            const uint32_t f = group_first<G>(__ballot(!within || occupied));
-            const float t_f = group_get<G>(tj, min(f, (uint32_t)G - 1u));
-            if (!done && skip) {
-                t = t_f;
-                skip = f == (uint32_t)G;  // otherwise the run's tests decide at t
             }
         }
     }
@@ -251,10 +339,11 @@ inline unsigned march_blocks(uint32_t n_rays_max) {
 // A group of 16 halves the tests per step and so a ray's latency, one of 8 the
 // waves that a large pass needs. Measured, count pass in us with groups of 16
 // and of 8 (unit box with 8 blobs; 16-unit box with 5 cascades and 128 small
-// blobs): 4,096 rays 51 / 85 and 133 / 166, 16,384 rays 45 / 45 and 150 / 167,
-// 32,768 rays 57 / 45 and 224 / 179, 131,072 rays 120 / 78 and 466 / 304.
-// Groups of 4 took 80 and 310 there and 146 and 237 at 4,096, groups of 32 and
-// 64 were slower at every size, and a ray per lane took 96 and 327 at 131,072.
+// blobs): 2,048 rays 43 / 67 and 109 / 142, 16,384 rays 48 / 47 and 122 / 150,
+// 32,768 rays 49 / 46 and 144 / 155, 131,072 rays 106 / 76 and 302 / 224.
+// Groups of 4 with two or four tests per lane took 79 and 240 at 131,072 and
+// 110 and 206 at 2,048, groups of 8 with two tests per lane 84 and 225 there;
+// groups of 32 and 64 and a ray per lane were slower at every size.
 constexpr uint32_t kGroup16Rays = 24576;
 
 TN_DEVICE MarchRay load_ray(bool active, uint32_t i, uint32_t B, const float* __restrict__ ori,
@@ -294,7 +383,7 @@ struct MarchCountArgs {
     uint2* runs;  // null: none wanted
 };
 
-template <int G, bool ML>
+template <int G, typename F>
 TN_DEVICE void march_count_rays(const MarchCountArgs& a, const tn_bbox_t& bbox, const MarchGrid& g,
                                 const MarchStep& st) {
     const uint32_t n_threads = gridDim.x * blockDim.x, tid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -305,7 +394,7 @@ TN_DEVICE void march_count_rays(const MarchCountArgs& a, const tn_bbox_t& bbox, 
         const bool active = own && a.alive[i] != 0;
         const MarchRay r = load_ray(active, i, a.B, a.ori, a.dir);
         RunLog log{a.runs && active && first ? a.runs + (uint64_t)i * kRunRecords : nullptr};
-        const uint32_t n = march_group<G, ML, true>(active, r, active ? a.t[i] : 0.0f, active ? a.tmax[i] : 0.0f,
+        const uint32_t n = march_group<G, F, true>(active, r, active ? a.t[i] : 0.0f, active ? a.tmax[i] : 0.0f,
                                                     a.max_steps, bbox, g, st, [](uint32_t, float) {}, log);
         log.close();
         if (own && first) {
@@ -315,6 +404,7 @@ TN_DEVICE void march_count_rays(const MarchCountArgs& a, const tn_bbox_t& bbox, 
     }
 }
 
+template <typename F>
 __global__ void __launch_bounds__(64 * kMarchWaves)
 march_count_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ d_n_rays, uint32_t B, tn_bbox_t bbox,
                    tn_occupancy_grid_t grid, float cone, float dt_min, float dt_max, uint32_t max_steps,
@@ -325,13 +415,8 @@ march_count_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ d_n_rays, u
     const MarchGrid g = make_grid(grid);
     const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
     const MarchCountArgs a = {n_rays, B, max_steps, dir, ray_tmax, ori, ray_t, ray_alive, n_steps, runs};
-    if (grid.n_levels == 1) {
-        if (n_rays <= kGroup16Rays) march_count_rays<16, false>(a, bbox, g, st);
-        else march_count_rays<8, false>(a, bbox, g, st);
-    } else {
-        if (n_rays <= kGroup16Rays) march_count_rays<16, true>(a, bbox, g, st);
-        else march_count_rays<8, true>(a, bbox, g, st);
-    }
+    if (n_rays <= kGroup16Rays) march_count_rays<16, F>(a, bbox, g, st);
+    else march_count_rays<8, F>(a, bbox, g, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -465,7 +550,7 @@ struct MarchGenerateArgs {
     float* out_t;
 };
 
-template <int G, bool ML>
+template <int G, typename F>
 TN_DEVICE void march_generate_rays(const MarchGenerateArgs& a, const tn_bbox_t& bbox, const MarchGrid& g,
                                    const MarchStep& st) {
     const uint32_t n_threads = gridDim.x * blockDim.x, tid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -475,7 +560,7 @@ TN_DEVICE void march_generate_rays(const MarchGenerateArgs& a, const tn_bbox_t& 
         const MarchRay r = load_ray(active, i, a.B, a.ori, a.dir);
         const uint32_t off = active ? a.offset[i] : 0u;
         NoLog log;
-        march_group<G, ML, false>(active, r, active ? a.t[i] : 0.0f, INFINITY, active ? a.n_steps[i] : 0u, bbox, g, st,
+        march_group<G, F, false>(active, r, active ? a.t[i] : 0.0f, INFINITY, active ? a.n_steps[i] : 0u, bbox, g, st,
                                   [&](uint32_t n, float t) {
                                       a.out_t[off + n] = t;
                                       a.out_ray[off + n] = i;
@@ -484,6 +569,7 @@ TN_DEVICE void march_generate_rays(const MarchGenerateArgs& a, const tn_bbox_t& 
     }
 }
 
+template <typename F>
 __global__ void __launch_bounds__(64 * kMarchWaves)
 march_generate_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ info, uint32_t B, tn_bbox_t bbox,
                       tn_occupancy_grid_t grid, float dt_min, float dt_max, float cone, const float* __restrict__ ori,
@@ -495,13 +581,8 @@ march_generate_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ info, ui
     const MarchGrid g = make_grid(grid);
     const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
     const MarchGenerateArgs a = {n_rays, B, ori, dir, ray_t, ray_offset, n_ray_steps, ray_alive, out_ray, out_t};
-    if (grid.n_levels == 1) {
-        if (n_rays <= kGroup16Rays) march_generate_rays<16, false>(a, bbox, g, st);
-        else march_generate_rays<8, false>(a, bbox, g, st);
-    } else {
-        if (n_rays <= kGroup16Rays) march_generate_rays<16, true>(a, bbox, g, st);
-        else march_generate_rays<8, true>(a, bbox, g, st);
-    }
+    if (n_rays <= kGroup16Rays) march_generate_rays<16, F>(a, bbox, g, st);
+    else march_generate_rays<8, F>(a, bbox, g, st);
 }
 
 // Sample-parallel second half of generation: from each sample's t and ray
@@ -582,7 +663,7 @@ TN_DEVICE void write_sample(const SampleOut& o, uint32_t sid, float t, const Mar
 // rendered rays, 32 (was 39 + 25) for 130,000 rays and 4.2 M samples, 43 (was
 // 168 + 14) in a scene of 16 units, where most steps are skips. The count
 // pass's 128 bytes per ray cost it 1 to 2 us.
-template <bool ML>
+template <typename F>
 TN_DEVICE void march_generate_from_runs(uint32_t n_rays, uint32_t B, const tn_bbox_t& bbox, const MarchGrid& g,
                                         const MarchStep& st, float inv_aabb, const float* __restrict__ ori,
                                         const float* __restrict__ dir, const float* __restrict__ ray_t,
@@ -637,11 +718,12 @@ TN_DEVICE void march_generate_from_runs(uint32_t n_rays, uint32_t B, const tn_bb
         }
         if (__ballot(active && again) != 0ull) {
             NoLog log;
-            march_group<G, ML, false>(active && again, r, t_min, INFINITY, ns, bbox, g, st, emit, log);
+            march_group<G, F, false>(active && again, r, t_min, INFINITY, ns, bbox, g, st, emit, log);
         }
     }
 }
 
+template <typename F>
 __global__ void __launch_bounds__(64 * kMarchWaves)
 march_generate_runs_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ info, uint32_t B, tn_bbox_t bbox,
                            float inv_aabb, tn_occupancy_grid_t grid, float dt_min, float dt_max, float cone,
@@ -652,12 +734,8 @@ march_generate_runs_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ inf
     const uint32_t n_rays = min(info[0], n_rays_max);
     const MarchGrid g = make_grid(grid);
     const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
-    if (grid.n_levels == 1)
-        march_generate_from_runs<false>(n_rays, B, bbox, g, st, inv_aabb, ori, dir, ray_t, ray_offset, ray_alive,
-                                        n_ray_steps, ray_img_id, runs, o);
-    else
-        march_generate_from_runs<true>(n_rays, B, bbox, g, st, inv_aabb, ori, dir, ray_t, ray_offset, ray_alive,
-                                       n_ray_steps, ray_img_id, runs, o);
+    march_generate_from_runs<F>(n_rays, B, bbox, g, st, inv_aabb, ori, dir, ray_t, ray_offset, ray_alive, n_ray_steps,
+                                ray_img_id, runs, o);
 }
 
 // Next step's ray count: the rays that would fill the sample budget at this
@@ -807,9 +885,11 @@ static int march_count(uint32_t n_rays_max, const uint32_t* d_n_rays, uint32_t s
     TN_CHECK_ARG(n_rays_max <= stride && grid.n_levels >= 1 && grid.n_levels <= 8);
     TN_CHECK_ARG(grid.resolution >= 2 && grid.resolution <= 1024 && dt_min > 0.0f && dt_max >= dt_min);
     if (n_rays_max == 0) return TN_OK;
-    march_count_kernel<<<march_blocks(n_rays_max), 64 * kMarchWaves, 0, stream>>>(
-        n_rays_max, d_n_rays, stride, bbox, grid, cone_angle, dt_min, dt_max, max_steps, dir, ray_tmax,
-        ray_alive, ori, ray_t, n_steps, static_cast<uint2*>(runs));
+    with_grid_form(grid, dt_max, [&](auto form) {
+        march_count_kernel<decltype(form)><<<march_blocks(n_rays_max), 64 * kMarchWaves, 0, stream>>>(
+            n_rays_max, d_n_rays, stride, bbox, grid, cone_angle, dt_min, dt_max, max_steps, dir, ray_tmax,
+            ray_alive, ori, ray_t, n_steps, static_cast<uint2*>(runs));
+    });
     TN_CHECK_LAUNCH();
     return TN_OK;
 }
@@ -870,9 +950,11 @@ extern "C" int tn_march_generate(uint32_t n_rays_max, const uint32_t* info, uint
     TN_CHECK_ARG(n_rays_max <= stride && grid.n_levels >= 1 && grid.n_levels <= 8 && dt_min > 0.0f);
     TN_CHECK_ARG(info != nullptr && sample_stride > 0);
     if (n_rays_max == 0) return TN_OK;
-    march_generate_kernel<<<march_blocks(n_rays_max), 64 * kMarchWaves, 0, stream>>>(
-        n_rays_max, info, stride, bbox, grid, dt_min, dt_max, cone_angle, ori, dir, ray_t, ray_offset, ray_alive,
-        n_ray_steps, out_img_id, out_t);
+    with_grid_form(grid, dt_max, [&](auto form) {
+        march_generate_kernel<decltype(form)><<<march_blocks(n_rays_max), 64 * kMarchWaves, 0, stream>>>(
+            n_rays_max, info, stride, bbox, grid, dt_min, dt_max, cone_angle, ori, dir, ray_t, ray_offset, ray_alive,
+            n_ray_steps, out_img_id, out_t);
+    });
     march_expand_kernel<<<blocks_for(sample_stride, 256), 256, 0, stream>>>(
         n_rays_max, sample_stride, info, stride, sample_stride, inv_aabb, dt_min, dt_max, cone_angle, ray_img_id, ori,
         dir, ray_t, ray_offset, n_ray_steps, out_img_id, out_t, out_pos, out_dir, out_dt, out_m_norm, out_dt_norm);
@@ -894,10 +976,12 @@ extern "C" int tn_march_generate_runs(uint32_t n_rays_max, const uint32_t* info,
     TN_CHECK_ARG(info != nullptr && sample_stride > 0 && runs && (reinterpret_cast<uintptr_t>(runs) & 127) == 0);
     if (runs_bytes < tn_march_runs_bytes(n_rays_max)) return TN_ERR_OUT_OF_MEMORY;
     if (n_rays_max == 0) return TN_OK;
-    march_generate_runs_kernel<<<march_blocks(n_rays_max), 64 * kMarchWaves, 0, stream>>>(
-        n_rays_max, info, stride, bbox, inv_aabb, grid, dt_min, dt_max, cone_angle, ray_img_id, ori, dir, ray_t,
-        ray_offset, ray_alive, n_ray_steps, static_cast<const uint2*>(runs),
-        SampleOut{out_img_id, out_t, out_pos, out_dir, out_dt, out_m_norm, out_dt_norm, sample_stride});
+    with_grid_form(grid, dt_max, [&](auto form) {
+        march_generate_runs_kernel<decltype(form)><<<march_blocks(n_rays_max), 64 * kMarchWaves, 0, stream>>>(
+            n_rays_max, info, stride, bbox, inv_aabb, grid, dt_min, dt_max, cone_angle, ray_img_id, ori, dir, ray_t,
+            ray_offset, ray_alive, n_ray_steps, static_cast<const uint2*>(runs),
+            SampleOut{out_img_id, out_t, out_pos, out_dir, out_dt, out_m_norm, out_dt_norm, sample_stride});
+    });
     TN_CHECK_LAUNCH();
     return TN_OK;
 }
