@@ -765,14 +765,31 @@ TN_DEVICE OpTile<P> masked_ops(const f16v& d, const OpTile<P>& act) {
     }
 }
 
-// add tile C (rows 32*mt.., cols 32*nt..) of a [n_out][n_in] gradient into LDS
-TN_DEVICE void add_dw_tile(float* acc, const f16v& C, int mt, int nt, int n_out, int n_in, int lane) {
+// store tile C (rows 32*mt.., cols 32*nt..) of a [n_out][n_in] gradient
+TN_DEVICE void store_dw_tile(float* out, const f16v& C, int mt, int nt, int n_out, int n_in, int lane) {
     const int col = 32 * nt + (lane & 31), h = lane >> 5;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int row = acc_row(mt, r, h);
-        if (row < n_out && col < n_in) acc[row * n_in + col] += C[r];
+        if (row < n_out && col < n_in) out[row * n_in + col] = C[r];
     }
+}
+
+// a tile's accumulators to and from LDS, 1024 floats, four registers of a lane together
+typedef float f4v __attribute__((ext_vector_type(4)));
+TN_DEVICE void put_acc(float* buf, const f16v& C, int lane) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f4v*>(buf + 256 * q + 4 * lane) = f4v{C[4 * q], C[4 * q + 1], C[4 * q + 2], C[4 * q + 3]};
+}
+TN_DEVICE f16v add_acc(f16v C, const float* buf, int lane) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const f4v v = *reinterpret_cast<const f4v*>(buf + 256 * q + 4 * lane);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) C[4 * q + k] += v[k];
+    }
+    return C;
 }
 
 // sets of group buffers: two in mixed precision; plain fp32 (twice the
@@ -947,23 +964,28 @@ mlp_backward_kernel(uint32_t n_max, const uint32_t* __restrict__ info, uint32_t 
         next_layer<P>(dbuf, abuf, dnext, anext);
     }
 
-    // workgroup sum of the weight gradients (waves in turn, so the sum order
-    // is fixed), then one partial per workgroup
-    float* red = reinterpret_cast<float*>(smem_raw);
-    for (int e = threadIdx.x; e < kNetParams; e += blockDim.x) red[e] = 0.0f;
+    // One partial per workgroup. A four-tile layer's tiles are whole; of a
+    // two-tile layer's the waves of the two K halves, wid and wid ^ 2, hold
+    // one summand each: they exchange two tiles through LDS (where the weights
+    // lay: their last readers are behind the last layer's barrier), each adds
+    // the other's to its own two and stores them, 128 bytes a row. (Waves that
+    // add into one LDS array in turn and a copy of it took 10 us more a launch:
+    // 24 against 13 us at 30 k samples, 62 against 53 at 262 k.)
+    float* const x = reinterpret_cast<float*>(smem_raw);
+    const bool upper = (wid >> 1) != 0;
+    put_acc(x + 2048 * wid, upper ? dW1 : dW3, lane);
+    put_acc(x + 2048 * wid + 1024, upper ? dW2 : dW5, lane);
+    float* const out = dw_partial + (uint64_t)blockIdx.x * kNetParams;
+    store_dw_tile(out + kW4, dW4, wid >> 1, t2, 64, 64, lane);
     __syncthreads();
-    for (int w = 0; w < kMlpWaves; ++w) {
-        if (wid == w) {
-            add_dw_tile(red + kW5, dW5, 0, t2, 3, 64, lane);
-            add_dw_tile(red + kW4, dW4, wid >> 1, t2, 64, 64, lane);
-            add_dw_tile(red + kW3, dW3, t2, 0, 64, 32, lane);
-            add_dw_tile(red + kW2, dW2, 0, t2, 16, 64, lane);
-            add_dw_tile(red + kW1, dW1, t2, 0, 64, 32, lane);
-        }
-        __syncthreads();
+    const float* const other = x + 2048 * (wid ^ 2);
+    if (upper) {
+        store_dw_tile(out + kW3, add_acc(dW3, other, lane), t2, 0, 64, 32, lane);
+        store_dw_tile(out + kW5, add_acc(dW5, other + 1024, lane), 0, t2, 3, 64, lane);
+    } else {
+        store_dw_tile(out + kW1, add_acc(dW1, other, lane), t2, 0, 64, 32, lane);
+        store_dw_tile(out + kW2, add_acc(dW2, other + 1024, lane), 0, t2, 16, 64, lane);
     }
-    for (int e = threadIdx.x; e < kNetParams; e += blockDim.x)
-        dw_partial[(uint64_t)blockIdx.x * kNetParams + e] = red[e];
 }
 
 // grad[e] (+)= sum over partials in a fixed order: a workgroup owns 64
@@ -1008,13 +1030,14 @@ template <class P>
 constexpr size_t bwd_lds_bytes() {
     const size_t w = (size_t)(Net<P>::kFwdElems + Net<P>::kBwdElems) * sizeof(typename P::T);
     const size_t t = 2 * kGrpSets<P> * grp_buf_elems<P>() * sizeof(typename P::T);
-    const size_t r = (size_t)kNetParams * sizeof(float);
-    return (w + t) > r ? (w + t) : r;
+    return w + t;
 }
-
 
 static_assert(bwd_lds_bytes<PrecF16>() <= 160 * 1024 && bwd_lds_bytes<PrecF32>() <= 160 * 1024,
               "the backward kernel's LDS must fit one CU (160 KiB)");
+// its waves exchange two 4 KiB tiles each where the weights lay
+static_assert((Net<PrecF16>::kFwdElems + Net<PrecF16>::kBwdElems) * sizeof(PrecF16::T) >= kMlpWaves * 8192 &&
+              (Net<PrecF32>::kFwdElems + Net<PrecF32>::kBwdElems) * sizeof(PrecF32::T) >= kMlpWaves * 8192);
 
 // Persistent launches: as many workgroups as fit on the device at once (the
 // backward kernel holds one workgroup per CU, the forward two), each looping
