@@ -97,7 +97,8 @@ inline void with_grid_form(const tn_occupancy_grid_t& grid, float dt_max, Fn fn)
 //  * the cascade of a point is formed from exponents, without a loop, and
 //    where the resolution is a power of two or a step cannot decide the
 //    cascade, the kernels are compiled without what that takes (GridForm);
-//  * the groups of a wave that run and those that skip share a block's test.
+//  * the groups of a wave that run and those that skip share a block's test,
+//    whose loads do not wait for the tests against the box and the ray's end.
 // A skip step is 20 vector instructions in one cascade and 28 or 34 in several;
 // a test about 80 and one load. Few rays are bound by the latency of the
 // chain and of that load, many rays by instruction issue: 65,000 rays through
@@ -107,7 +108,7 @@ inline void with_grid_form(const tn_occupancy_grid_t& grid, float dt_max, Fn fn)
 // 8 blobs, and 120 us to count 53 rays; this takes 49, 40 and 39 us. A render
 // pass of 65,000 rays in the 16-unit scene takes 290 us to count (380 with 24
 // and 36 instructions per skip step and a test for runs and skips each).
-// G is 16 for up to kGroup16Rays rays and 8 for more (see there).
+// G and T by the number of rays: see kGroup16Rays.
 struct MarchStep {
     float cone, dt_min, dt_max, inv_dt_min;
 };
@@ -224,35 +225,27 @@ TN_DEVICE uint32_t group_bits(uint64_t ballot) {
     const uint32_t half = lane < 32u ? (uint32_t)ballot : (uint32_t)(ballot >> 32);
     return (half >> (lane & 31u & ~(uint32_t)(G - 1))) & ((1u << G) - 1u);
 }
-// index of the group's first lane with a set bit of `ballot`, or G (8 or 16)
-template <int G>
-TN_DEVICE uint32_t group_first(uint64_t ballot) {
-    return (uint32_t)__builtin_ctz(group_bits<G>(ballot) | (1u << G));
-}
-// the bit of the group's lane j <= G (false for G)
-template <int G>
-TN_DEVICE bool group_bit(uint64_t ballot, uint32_t j) {
-    return ((group_bits<G>(ballot) >> j) & 1u) != 0u;
-}
 // v of the group's lane j
 template <int G>
 TN_DEVICE float group_get(float v, uint32_t j) {
     return __shfl(v, (int)((__lane_id() & ~(uint32_t)(G - 1)) + j), 64);
 }
 
-// One ray per group, all 64 / G of a wave at once. Emits through `emit(n, t)`
+// One ray per group, all 64 / G of a wave at once, G steps per block of a skip
+// and G T per block of a run. Emits through `emit(n, t)`
 // (lane-wise: sample n of the lane's ray at t). COUNT: stops at t_max, at
 // the box and at max_n samples; otherwise (the generate pass) takes max_n
 // samples, and one outside the box, which the count pass cannot have counted,
 // would be emitted without advancing. Each run of samples without a skip in
 // between goes to `log` (its first t and sample, and the t after its last), in
-// pieces of at most G. Returns the ray's sample count.
+// pieces of at most G T. Returns the ray's sample count.
 struct NoLog {
     TN_DEVICE void run(bool, float, uint32_t, float) {}
 };
-template <int G, typename F, bool COUNT, typename Emit, typename Log>
+template <int G, int T, typename F, bool COUNT, typename Emit, typename Log>
 TN_DEVICE uint32_t march_group(bool active, const MarchRay& r, float t, float t_max, uint32_t max_n,
                                const tn_bbox_t& bbox, const MarchGrid& g, const MarchStep& st, Emit emit, Log& log) {
+    constexpr uint32_t S = G * T;  // samples per block of a run
     const uint32_t lane = __lane_id(), j = lane & (uint32_t)(G - 1), axis = lane & 3u;
     const float oa = axis == 0 ? r.ox : axis == 1 ? r.oy : r.oz;
     const float da = axis == 0 ? r.dx : axis == 1 ? r.dy : r.dz;
@@ -265,16 +258,24 @@ TN_DEVICE uint32_t march_group(bool active, const MarchRay& r, float t, float t_
         const uint64_t runs = __builtin_amdgcn_ballot_w64(!done && !skip);
         const uint64_t skips = __builtin_amdgcn_ballot_w64(!done && skip);
         if ((runs | skips) == 0ull) break;
-        float tj = t;
+        float tj[T];  // of the lane's samples j, j + G, ... of the block
+        float t_end = t;
+#pragma unroll
+        for (int q = 0; q < T; ++q) tj[q] = t;
         if (runs != 0ull) {
-            // a run: lane j's t after j more samples
+            // a run: the t's after so many more samples
             if (st.dt_min == st.dt_max) {
 #pragma unroll
-                for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k) tj = j > k ? tj + st.dt_min : tj;
+                for (uint32_t k = 0; k < S; ++k) {
+                    tj[k / G] = j >= k % G ? t_end : tj[k / G];
+                    t_end += st.dt_min;
+                }
             } else {
 #pragma unroll
-                for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k)
-                    tj = j > k ? tj + step_dt(st, tj) : tj;
+                for (uint32_t k = 0; k < S; ++k) {
+                    tj[k / G] = j >= k % G ? t_end : tj[k / G];
+                    t_end += step_dt(st, t_end);
+                }
             }
         }
         if (skips != 0ull) {
@@ -294,25 +295,50 @@ TN_DEVICE uint32_t march_group(bool active, const MarchRay& r, float t, float t_
                 tc += div_up(d, st.dt_min, st.inv_dt_min) * st.dt_min;
                 ts = j == k ? tc : ts;
             }
-            tj = skip ? ts : tj;
+            tj[0] = skip ? ts : tj[0];
+            t_end = skip ? tc : t_end;
         }
-        // one test for both: f is the first lane that ends the group's run or skip
-        const float x = r.ox + tj * r.dx, y = r.oy + tj * r.dy, z = r.oz + tj * r.dz;
-        const bool within = !done && (skip || j < max_n - n) && (!COUNT || tj < t_max) && bbox_contains(bbox, x, y, z);
-        const bool occupied = within && point_occupied<F>(g, st, tj, x, y, z);
-        const uint32_t f = group_first<G>(__builtin_amdgcn_ballot_w64(!within || occupied == skip));
-        const bool in_f = group_bit<G>(__builtin_amdgcn_ballot_w64(within), f);  // false for f == G
-        const float t_end = skip ? tj : tj + step_dt(st, tj);  // of lane G - 1, which a whole block goes on from
-        const float t_f = group_get<G>(f < (uint32_t)G ? tj : t_end, min(f, (uint32_t)G - 1u));
+        // one test for both: f is the first step that ends the group's run or
+        // skip. The cells are looked up for every lane (their indices are
+        // clamped), so that a block's loads are in flight together.
+        uint64_t stop = 0, in = 0;
+        const uint32_t whole = skip ? (uint32_t)G : S;
+        bool occ[T];
+#pragma unroll
+        for (int q = 0; q < T; ++q) {
+            if (q > 0 && runs == 0ull) break;
+            const float x = r.ox + tj[q] * r.dx, y = r.oy + tj[q] * r.dy, z = r.oz + tj[q] * r.dz;
+            occ[q] = point_occupied<F>(g, st, tj[q], x, y, z);
+            const bool within = !done && (skip || j + q * G < max_n - n) && (!COUNT || tj[q] < t_max) &&
+                                bbox_contains(bbox, x, y, z);
+            in |= (uint64_t)group_bits<G>(__builtin_amdgcn_ballot_w64(within)) << (q * G);
+        }
+#pragma unroll
+        for (int q = 0; q < T; ++q) {
+            if (q > 0 && runs == 0ull) break;
+            stop |= (uint64_t)group_bits<G>(__builtin_amdgcn_ballot_w64(occ[q] == skip)) << (q * G);
+        }
+        stop |= ~in;  // a skip's bits from G on and a block's from S on are set
+        if (skip) stop |= ~0ull << G;
+        const uint32_t f = stop != 0ull ? min((uint32_t)__builtin_ctzll(stop), whole) : whole;
+        const bool in_f = f < whole && ((in >> f) & 1ull) != 0ull;
+        float t_f = t_end;
+#pragma unroll
+        for (int q = 0; q < T; ++q) {
+            const float v = group_get<G>(tj[q], f & (uint32_t)(G - 1));
+            t_f = f < whole && f / G == (uint32_t)q ? v : t_f;
+        }
         if (!done) {
             if (!skip) {
-                if (j < f) emit(n + j, tj);
+#pragma unroll
+                for (int q = 0; q < T; ++q)
+                    if (j + q * G < f) emit(n + j + q * G, tj[q]);
                 if (f != 0u) log.run(!open, t, n, t_f);
-                open = f == (uint32_t)G;
+                open = f == S;
                 n += f;
             }
             t = t_f;
-            if (f < (uint32_t)G) {
+            if (f < whole) {
                 if (in_f) {
                     skip = !skip;
                 } else {
@@ -337,13 +363,18 @@ inline unsigned march_blocks(uint32_t n_rays_max) {
 }
 
 // A group of 16 halves the tests per step and so a ray's latency, one of 8 the
-// waves that a large pass needs. Measured, count pass in us with groups of 16
-// and of 8 (unit box with 8 blobs; 16-unit box with 5 cascades and 128 small
-// blobs): 2,048 rays 43 / 67 and 109 / 142, 16,384 rays 48 / 47 and 122 / 150,
-// 32,768 rays 49 / 46 and 144 / 155, 131,072 rays 106 / 76 and 302 / 224.
-// Groups of 4 with two or four tests per lane took 79 and 240 at 131,072 and
-// 110 and 206 at 2,048, groups of 8 with two tests per lane 84 and 225 there;
-// groups of 32 and 64 and a ray per lane were slower at every size.
+// waves that a large pass needs; with few rays, a run goes on for 32 samples
+// at a time, two tests per lane. Measured, count pass in us with groups of 16
+// by two tests, of 16 and of 8 (unit box with 8 blobs; all of it occupied;
+// 16-unit box with 5 cascades and 128 small blobs): 2,048 rays 39 / 40 / 60,
+// 29 / 34 / 60 and 106 / 103 / 134, 8,192 rays 51 / 47 / 62, 33 / 38 / 60 and
+// 113 / 106 / 134, 16,384 rays 52 / 45 / 43, 13 / 14 / 19 and 125 / 118 / 144,
+// 32,768 rays 56 / 51 / 43, 20 / 20 / 20 and 155 / 147 / 146, 131,072 rays
+// 121 / 111 / 70, 47 / 49 / 38 and 319 / 305 / 208. Groups of 16 by four tests
+// gain 2 us of 29 where all is occupied and lose 4 to 6 elsewhere, groups of
+// 8 by two lose above 16,384 rays; groups of 4, 32 and 64 and a ray per lane
+// were slower at every size.
+constexpr uint32_t kTwoBlockRays = 4096;
 constexpr uint32_t kGroup16Rays = 24576;
 
 TN_DEVICE MarchRay load_ray(bool active, uint32_t i, uint32_t B, const float* __restrict__ ori,
@@ -383,7 +414,7 @@ struct MarchCountArgs {
     uint2* runs;  // null: none wanted
 };
 
-template <int G, typename F>
+template <int G, int T, typename F>
 TN_DEVICE void march_count_rays(const MarchCountArgs& a, const tn_bbox_t& bbox, const MarchGrid& g,
                                 const MarchStep& st) {
     const uint32_t n_threads = gridDim.x * blockDim.x, tid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -394,7 +425,7 @@ TN_DEVICE void march_count_rays(const MarchCountArgs& a, const tn_bbox_t& bbox, 
         const bool active = own && a.alive[i] != 0;
         const MarchRay r = load_ray(active, i, a.B, a.ori, a.dir);
         RunLog log{a.runs && active && first ? a.runs + (uint64_t)i * kRunRecords : nullptr};
-        const uint32_t n = march_group<G, F, true>(active, r, active ? a.t[i] : 0.0f, active ? a.tmax[i] : 0.0f,
+        const uint32_t n = march_group<G, T, F, true>(active, r, active ? a.t[i] : 0.0f, active ? a.tmax[i] : 0.0f,
                                                     a.max_steps, bbox, g, st, [](uint32_t, float) {}, log);
         log.close();
         if (own && first) {
@@ -415,8 +446,9 @@ march_count_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ d_n_rays, u
     const MarchGrid g = make_grid(grid);
     const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
     const MarchCountArgs a = {n_rays, B, max_steps, dir, ray_tmax, ori, ray_t, ray_alive, n_steps, runs};
-    if (n_rays <= kGroup16Rays) march_count_rays<16, F>(a, bbox, g, st);
-    else march_count_rays<8, F>(a, bbox, g, st);
+    if (n_rays <= kTwoBlockRays) march_count_rays<16, 2, F>(a, bbox, g, st);
+    else if (n_rays <= kGroup16Rays) march_count_rays<16, 1, F>(a, bbox, g, st);
+    else march_count_rays<8, 1, F>(a, bbox, g, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -550,7 +582,7 @@ struct MarchGenerateArgs {
     float* out_t;
 };
 
-template <int G, typename F>
+template <int G, int T, typename F>
 TN_DEVICE void march_generate_rays(const MarchGenerateArgs& a, const tn_bbox_t& bbox, const MarchGrid& g,
                                    const MarchStep& st) {
     const uint32_t n_threads = gridDim.x * blockDim.x, tid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -560,7 +592,7 @@ TN_DEVICE void march_generate_rays(const MarchGenerateArgs& a, const tn_bbox_t& 
         const MarchRay r = load_ray(active, i, a.B, a.ori, a.dir);
         const uint32_t off = active ? a.offset[i] : 0u;
         NoLog log;
-        march_group<G, F, false>(active, r, active ? a.t[i] : 0.0f, INFINITY, active ? a.n_steps[i] : 0u, bbox, g, st,
+        march_group<G, T, F, false>(active, r, active ? a.t[i] : 0.0f, INFINITY, active ? a.n_steps[i] : 0u, bbox, g, st,
                                   [&](uint32_t n, float t) {
                                       a.out_t[off + n] = t;
                                       a.out_ray[off + n] = i;
@@ -581,8 +613,9 @@ march_generate_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ info, ui
     const MarchGrid g = make_grid(grid);
     const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
     const MarchGenerateArgs a = {n_rays, B, ori, dir, ray_t, ray_offset, n_ray_steps, ray_alive, out_ray, out_t};
-    if (n_rays <= kGroup16Rays) march_generate_rays<16, F>(a, bbox, g, st);
-    else march_generate_rays<8, F>(a, bbox, g, st);
+    if (n_rays <= kTwoBlockRays) march_generate_rays<16, 2, F>(a, bbox, g, st);
+    else if (n_rays <= kGroup16Rays) march_generate_rays<16, 1, F>(a, bbox, g, st);
+    else march_generate_rays<8, 1, F>(a, bbox, g, st);
 }
 
 // Sample-parallel second half of generation: from each sample's t and ray
@@ -718,7 +751,7 @@ TN_DEVICE void march_generate_from_runs(uint32_t n_rays, uint32_t B, const tn_bb
         }
         if (__ballot(active && again) != 0ull) {
             NoLog log;
-            march_group<G, F, false>(active && again, r, t_min, INFINITY, ns, bbox, g, st, emit, log);
+            march_group<G, 1, F, false>(active && again, r, t_min, INFINITY, ns, bbox, g, st, emit, log);
         }
     }
 }
