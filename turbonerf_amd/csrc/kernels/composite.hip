@@ -27,7 +27,7 @@
 //      reference's adjoint (its running "cumsum" subtraction) written for a
 //      lane-parallel scan. Samples after the early-termination point
 //      (T < min_T) get zero gradient, as in the reference.
-// Forward-only compositing (rendering) walks each wave's window of rays.
+// Forward-only compositing (rendering) takes 16 lanes per ray.
 
 #include <mutex>
 
@@ -411,75 +411,97 @@ composite_grad_kernel(const uint32_t* __restrict__ info, uint32_t B, uint32_t PB
     stf(dL_dcolor, s + 2 * (uint64_t)PB, gc_b);
 }
 
+// Inclusive sum over each row of 16 lanes (no segments: a row holds one ray).
+// Lanes without a source add zero, which leaves a compensated sum as it is.
+template <int CTRL>
+TN_DEVICE void row_step(CSum& v) {
+    v = csum_add(v, CSum{dpp_f<CTRL, 0xF>(v.hi), dpp_f<CTRL, 0xF>(v.lo)});
+}
+template <int CTRL>
+TN_DEVICE void row_step(double& v) {
+    v += dpp_d<CTRL, 0xF>(v);
+}
+template <typename R>
+TN_DEVICE Acc<R> row_scan(Acc<R> a) {
+    row_step<0x111>(a.v);
+    row_step<0x112>(a.v);
+    row_step<0x114>(a.v);
+    row_step<0x118>(a.v);
+    return a;
+}
+// a - x, x the last summand (the rounded sum's residue added last, so that a
+// large x does not take the smaller summands' bits along)
+TN_DEVICE float without(const Acc<float>& a, float x) { return (a.v.hi - x) + a.v.lo; }
+TN_DEVICE double without(const Acc<double>& a, double x) { return a.v - x; }
+TN_DEVICE Acc<float> row_last(const Acc<float>& a) {
+    return Acc<float>{CSum{__shfl(a.v.hi, 15, 16), __shfl(a.v.lo, 15, 16)}};
+}
+TN_DEVICE Acc<double> row_last(const Acc<double>& a) { return Acc<double>{__shfl(a.v, 15, 16)}; }
+
 // Forward-only compositing: premultiplied rgb and alpha per ray, with the
 // reference's early termination. `raw_density` selects sigma = exp(min(s,12)-1)
 // of a network output, otherwise the input already is sigma. As in the
 // reference's render compositing (rendering-kernels.cu:570-578, colour divided
 // by alpha only when alpha > 1e-4, else zero), a sample's colour counts only
 // when its alpha exceeds 1e-4; its alpha always counts.
+//
+// 16 lanes per ray take 16 samples at a time: the prefix of sigma dt is a scan
+// over a row of lanes, and each lane keeps its own sums of w c and w, added
+// over the row at the ray's end, so a block of 64 lanes takes one scan of four
+// steps. Bound by instruction issue. (Five scans segmented by ray over 64
+// samples of consecutive rays, six steps each, took 103 us against 25 for
+// 131,000 rays and 4.2 M samples.) A network's sigma is
+// positive, so T only falls and a ray below min_T is left.
+constexpr uint32_t kForwardMaxBlocks = 4096;
+
 template <typename TIn, typename R>
 __global__ void __launch_bounds__(64 * kCompositeWaves)
-composite_forward_kernel(const uint32_t* __restrict__ info, uint32_t B, uint32_t OB, uint32_t S, float min_T,
+composite_forward_kernel(const uint32_t* __restrict__ info, uint32_t B, uint32_t OB, uint32_t max_samples, float min_T,
                          int raw_density, const uint32_t* __restrict__ steps, const uint32_t* __restrict__ offs,
                          const TIn* __restrict__ density, const TIn* __restrict__ color,
                          const float* __restrict__ dtb, float* __restrict__ rgba) {
-    __shared__ int slots[kCompositeWaves][128];
-    const uint32_t wid = threadIdx.x >> 6;
-    const uint32_t lane = __lane_id();
-    const uint32_t w = blockIdx.x * kCompositeWaves + wid;
-    const uint32_t n_rays = info[0], n_samples = info[1];
-    const WaveRange wr = wave_range(w, S, n_rays, n_samples, offs);
-    if (!wr.active) return;
-    int* slot = slots[wid];
-    auto empty_ray = [&](uint32_t r) {
-        rgba[r] = 0.0f;
-        rgba[r + OB] = 0.0f;
-        rgba[r + 2 * OB] = 0.0f;
-        rgba[r + 3 * OB] = 0.0f;
-    };
-    RayWalk wk;
-    wk.r_scan = wr.r0;
-    Acc<R> carry_P = Acc<R>::zero();
-    Acc<R> cr = Acc<R>::zero(), cg = Acc<R>::zero(), cb = Acc<R>::zero(), ca = Acc<R>::zero();
-    ChunkIn in = {};
-    if (wr.s0 < wr.s1) in = load_chunk(wr.s0, wr.s1, lane, density, dtb, color, B);
-    for (uint32_t c = wr.s0; c < wr.s1; c += 64) {
-        const uint64_t s = (uint64_t)c + lane;
-        const bool valid = s < wr.s1;
-        const ChunkIn cur = in;
-        if (c + 64 < wr.s1) in = load_chunk(c + 64, wr.s1, lane, density, dtb, color, B);
-        const int prev_carry = wk.carry_ray;
-        const LaneRay lr = chunk_rays(c, wr.r1, wk, offs, steps, slot, empty_ray);
-        const int ray = valid ? lr.ray : -2 - (int)lane;
-        SampleState<R> st = sample_state<R>(valid, ray, cur, wk.carry_ray, carry_P, min_T, raw_density != 0);
-        const float cR = valid ? cur.cr : 0.0f, cG = valid ? cur.cg : 0.0f, cB = valid ? cur.cb : 0.0f;
-        const R wv = st.inc ? st.w : (R)0;
-        const R wc = st.alpha > (R)1e-4f ? wv : (R)0;
-        Acc<R> sr = Acc<R>::of(wc * (R)cR).scan(ray), sg = Acc<R>::of(wc * (R)cG).scan(ray);
-        Acc<R> sb = Acc<R>::of(wc * (R)cB).scan(ray), sa = Acc<R>::of(wv).scan(ray);
-        if (ray == prev_carry) {
-            sr = sr + cr;
-            sg = sg + cg;
-            sb = sb + cb;
-            sa = sa + ca;
+    const uint32_t n_rays = min(info[0], OB), n_samples = min(info[1], max_samples);
+    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x, j = tid & 15u;
+    for (uint32_t w = tid & ~63u; w / 16 < n_rays; w += gridDim.x * blockDim.x) {
+        const uint32_t r = (w + (tid & 63u)) / 16;
+        const uint32_t s0 = r < n_rays ? min(offs[r], n_samples) : 0u;
+        uint32_t n = r < n_rays ? min(steps[r], n_samples - s0) : 0u;  // 0 once the ray is done
+        Acc<R> before = Acc<R>::zero();
+        Acc<R> sr = Acc<R>::zero(), sg = Acc<R>::zero(), sb = Acc<R>::zero(), sa = Acc<R>::zero();
+        ChunkIn in = {};
+        if (j < n) in = load_chunk(s0 + j, n_samples, 0, density, dtb, color, B);
+        for (uint32_t c = 0; __builtin_amdgcn_ballot_w64(c < n) != 0ull; c += 16) {
+            const bool valid = c + j < n;
+            const ChunkIn cur = in;
+            if (c + 16 + j < n) in = load_chunk(s0 + c + 16 + j, n_samples, 0, density, dtb, color, B);
+            R sigma = 0, dt = 0;
+            if (valid) {
+                sigma = raw_density ? r_exp<R>((R)fminf(cur.d, 12.0f) - (R)1) : (R)cur.d;
+                dt = (R)cur.dt;
+            }
+            const R tau = sigma * dt;
+            const Acc<R> P = before + row_scan(Acc<R>::of(tau));
+            const R T = r_exp<R>(-without(P, tau)), alpha = r_alpha<R>(tau);
+            const R wv = valid && T >= (R)min_T ? T * alpha : (R)0;
+            const R wc = alpha > (R)1e-4f ? wv : (R)0;
+            sr = sr + Acc<R>::of(valid ? wc * (R)cur.cr : (R)0);
+            sg = sg + Acc<R>::of(valid ? wc * (R)cur.cg : (R)0);
+            sb = sb + Acc<R>::of(valid ? wc * (R)cur.cb : (R)0);
+            sa = sa + Acc<R>::of(wv);
+            before = row_last(P);
+            if (raw_density && !(r_exp<R>(-before.val()) >= (R)min_T)) n = 0;
         }
-        const bool tail = valid && s + 1 == (uint64_t)lr.end;
-        if (tail) {
-            const uint32_t rr = (uint32_t)ray;
-            rgba[rr] = (float)sr.val();
-            rgba[rr + OB] = (float)sg.val();
-            rgba[rr + 2 * OB] = (float)sb.val();
-            rgba[rr + 3 * OB] = (float)sa.val();
+        sr = row_scan(sr);
+        sg = row_scan(sg);
+        sb = row_scan(sb);
+        sa = row_scan(sa);
+        if (j == 15 && r < n_rays) {
+            rgba[r] = (float)sr.val();
+            rgba[r + OB] = (float)sg.val();
+            rgba[r + 2 * OB] = (float)sb.val();
+            rgba[r + 3 * OB] = (float)sa.val();
         }
-        const bool tail63 = lane63((int)tail) != 0;
-        cr = sr.bcast(63);
-        cg = sg.bcast(63);
-        cb = sb.bcast(63);
-        ca = sa.bcast(63);
-        wk.carry_end = lane63(lr.end);
-        if (tail63 || !lane63((int)valid)) wk.carry_ray = -1;
     }
-    for (uint32_t r = wk.r_scan + lane; r < wr.r1; r += 64) empty_ray(r);
 }
 
 // deterministic mean of the per-ray losses: (1/n_rays) sum_r sum_ch loss
@@ -648,23 +670,22 @@ extern "C" int tn_composite_forward(int dtype, const uint32_t* info, uint32_t st
                                     const void* color, const float* dt, float* rgba, hipStream_t stream) {
     TN_CHECK_ARG(info && ray_steps && ray_offset && density && color && dt && rgba && max_samples <= stride);
     TN_CHECK_ARG(max_samples < (1u << 31));  // sample offsets fit an int
-    const uint32_t S = 256;
-    const uint32_t waves = (max_samples + S - 1) / S + 1;
-    const uint32_t blocks = (waves + kCompositeWaves - 1) / kCompositeWaves;
+    if (out_stride == 0) return TN_OK;
+    const uint32_t blocks = std::min(blocks_for((uint64_t)out_stride * 16, 64 * kCompositeWaves), kForwardMaxBlocks);
     switch (dtype) {
         case 0:
             composite_forward_kernel<float, float><<<blocks, 64 * kCompositeWaves, 0, stream>>>(
-                info, stride, out_stride, S, min_transmittance, raw_density, ray_steps, ray_offset,
+                info, stride, out_stride, max_samples, min_transmittance, raw_density, ray_steps, ray_offset,
                 static_cast<const float*>(density), static_cast<const float*>(color), dt, rgba);
             break;
         case 1:
             composite_forward_kernel<_Float16, float><<<blocks, 64 * kCompositeWaves, 0, stream>>>(
-                info, stride, out_stride, S, min_transmittance, raw_density, ray_steps, ray_offset,
+                info, stride, out_stride, max_samples, min_transmittance, raw_density, ray_steps, ray_offset,
                 static_cast<const _Float16*>(density), static_cast<const _Float16*>(color), dt, rgba);
             break;
         case 2:
             composite_forward_kernel<float, double><<<blocks, 64 * kCompositeWaves, 0, stream>>>(
-                info, stride, out_stride, S, min_transmittance, raw_density, ray_steps, ray_offset,
+                info, stride, out_stride, max_samples, min_transmittance, raw_density, ray_steps, ray_offset,
                 static_cast<const float*>(density), static_cast<const float*>(color), dt, rgba);
             break;
         default:

@@ -1,11 +1,9 @@
 // Wave64 machinery for per-ray work over compacted samples.
 //
 // Samples of ray r occupy [offset[r], offset[r] + steps[r]) and rays are laid
-// out back to back. A wave owns the rays whose first sample falls in its
-// window [w*S, (w+1)*S) (the last wave also owns any zero-length rays at the
-// end) and walks their samples in chunks of 64, one sample per lane. Inside a
-// chunk, per-ray prefix sums are segmented inclusive scans keyed by ray
-// index; a ray that continues into the next chunk carries its running sums.
+// out back to back. A wave walks samples in chunks of 64, one sample per lane.
+// Inside a chunk, per-ray prefix sums are segmented inclusive scans keyed by
+// ray index.
 // Sums in fp32 are compensated (TwoSum, Knuth TAOCP vol. 2 4.2.2) so a
 // 1024-sample ray accumulates O(log n) rather than O(n) rounding error.
 #pragma once
@@ -196,27 +194,8 @@ TN_DEVICE uint32_t wave_lower_bound(const uint32_t* __restrict__ offs, uint32_t 
     return lo;
 }
 
-// Ray range and sample window of wave `w` with window S.
-struct WaveRange {
-    uint32_t r0, r1, s0, s1;
-    bool active;
-};
-
-TN_DEVICE WaveRange wave_range(uint32_t w, uint32_t S, uint32_t n_rays, uint32_t n_samples,
-                               const uint32_t* __restrict__ offs) {
-    WaveRange wr;
-    const uint32_t n_waves = n_samples == 0 ? 1 : (n_samples + S - 1) / S;
-    wr.active = w < n_waves && n_rays > 0;
-    if (!wr.active) return wr;
-    wr.r0 = w == 0 ? 0 : wave_lower_bound(offs, n_rays, w * S);
-    wr.r1 = (w + 1 == n_waves) ? n_rays : wave_lower_bound(offs, n_rays, (w + 1) * S);
-    wr.s0 = wr.r0 < n_rays ? min(offs[wr.r0], n_samples) : n_samples;
-    wr.s1 = wr.r1 < n_rays ? min(offs[wr.r1], n_samples) : n_samples;
-    return wr;
-}
-
 // ---------------------------------------------------------------------------
-// Walking a window's rays chunk by chunk. Rays with index >= r_scan start at
+// Walking rays chunk by chunk. Rays with index >= r_scan start at
 // or after the current chunk; carry_ray (or -1) continues from the previous
 // chunk and ends at sample carry_end. Each lane caches the offset and step
 // count of ray r_cache + lane, reloaded only when r_scan moves (when rays
