@@ -260,6 +260,17 @@ int tn_occ_update_density(int raw_dtype, uint32_t n_cells, uint32_t start_idx,
     tn_occupancy_grid_t grid, int level, int sample_all_cells, const float* random,
     const void* raw_density, tn_stream_t stream);
 
+/* tn_occ_sample_points and tn_occ_update_density that draw their uniforms
+ * themselves: the 4 stride values that tn_fill_uniform gives for (seed,
+ * offset), the points from the first three slices and the subset rule from the
+ * last (reference trainer.cu:236-295 fills one buffer for both). pos and the
+ * grid's densities are 16-byte aligned. */
+int tn_occ_draw_points(uint32_t n_cells, uint32_t stride, uint32_t start_idx, tn_occupancy_grid_t grid,
+    int level, float inv_aabb, uint64_t seed, uint64_t offset, float* pos, tn_stream_t stream);
+int tn_occ_draw_update(int raw_dtype, uint32_t n_cells, uint32_t stride, uint32_t start_idx,
+    tn_occupancy_grid_t grid, int level, int sample_all_cells, uint64_t seed, uint64_t offset,
+    const void* raw_density, tn_stream_t stream);
+
 /* bitfield byte = sum_k [density_k > threshold] << k (reference
  * update_occupancy_grid_bits_kernel, :118-141). */
 int tn_occ_update_bits(tn_occupancy_grid_t grid, float threshold, tn_stream_t stream);

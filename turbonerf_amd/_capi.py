@@ -170,6 +170,8 @@ _SIGS: dict[str, tuple] = {
     "tn_occ_decay": (C.c_int, [OccupancyGrid, f32, vp]),
     "tn_occ_sample_points": (C.c_int, [u32, u32, u32, OccupancyGrid, C.c_int, f32, vp, vp, vp]),
     "tn_occ_update_density": (C.c_int, [C.c_int, u32, u32, OccupancyGrid, C.c_int, C.c_int, vp, vp, vp]),
+    "tn_occ_draw_points": (C.c_int, [u32, u32, u32, OccupancyGrid, C.c_int, f32, u64, u64, vp, vp]),
+    "tn_occ_draw_update": (C.c_int, [C.c_int, u32, u32, u32, OccupancyGrid, C.c_int, C.c_int, u64, u64, vp, vp]),
     "tn_occ_update_bits": (C.c_int, [OccupancyGrid, f32, vp]),
     "tn_popcount_workspace_bytes": (sz, [u64]),
     "tn_popcount": (C.c_int, [vp, u64, vp, vp, sz, vp]),

@@ -744,16 +744,14 @@ uint32_t Trainer::update_occupancy_grid(Context& ctx, uint32_t training_step) {
         for (uint32_t start = 0; start < vol; start += chunk) {
             const uint32_t n = std::min(chunk, vol - start);
             // the occupancy update draws from its own stream (key seed ^ k)
-            TN_TRY(tn_fill_uniform(4 * (uint64_t)chunk, ctx.rng_seed ^ 0x0cc0cc0cc0cc0cc0ull, ctx.occ_rng_offset,
-                                   ws.random_float.data(), ts));
+            const uint64_t seed = ctx.rng_seed ^ 0x0cc0cc0cc0cc0cc0ull, offset = ctx.occ_rng_offset;
             ctx.occ_rng_offset += 4 * (uint64_t)chunk;
-            TN_TRY(tn_occ_sample_points(n, chunk, start, og.view(), level, 1.0f / aabb, ws.random_float.data(),
-                                        ws.sample_pos.data(), ts));
+            TN_TRY(tn_occ_draw_points(n, chunk, start, og.view(), level, 1.0f / aabb, seed, offset,
+                                      ws.sample_pos.data(), ts));
             nerf.network.inference(s, nerf.params, n, nullptr, chunk, ws.sample_pos.data(), nullptr,
                                    nw.features.data(), nw.density.data(), nullptr, false);
-            TN_TRY(tn_occ_update_density(nerf.network.config.precision, n, start, og.view(), level,
-                                         training_step < 256 ? 1 : 0, ws.random_float.data() + 3 * (size_t)chunk,
-                                         nw.density.data(), ts));
+            TN_TRY(tn_occ_draw_update(nerf.network.config.precision, n, chunk, start, og.view(), level,
+                                      training_step < 256 ? 1 : 0, seed, offset, nw.density.data(), ts));
         }
     }
     TN_TRY(tn_occ_update_bits(og.view(), ctx.occupancy_threshold, ts));

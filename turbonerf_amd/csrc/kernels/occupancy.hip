@@ -22,33 +22,93 @@ __global__ void occ_decay_kernel(uint64_t n, float factor, float* __restrict__ d
     }
 }
 
-// jittered point in cell (start + i) of `level`, normalised by the training
-// box, not clamped (reference :38-76, occupancy-grid.cuh:167-182)
-__global__ void occ_sample_points_kernel(uint32_t n_cells, uint32_t B, uint32_t start_idx, int res, int level,
-                                         float inv_aabb, const float* __restrict__ random, float* __restrict__ pos) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_cells) return;
-    const uint32_t idx = i + start_idx;
+// jittered point in cell idx of `level` (three uniforms u), normalised by the
+// training box, not clamped (reference :38-76, occupancy-grid.cuh:167-182)
+TN_DEVICE void cell_point(uint32_t idx, int res, int level, float inv_aabb, const float u[3], float p[3]) {
     const float inv_res = 1.0f / (float)res;
     const int half_res = res / 2;
     const float level_size = (float)(1 << level);
     const float voxel = level_size * inv_res;
-    const int ix = (int)compact_bits10(idx >> 0);
-    const int iy = (int)compact_bits10(idx >> 1);
-    const int iz = (int)compact_bits10(idx >> 2);
-    const float vx = (float)(ix - half_res) * voxel;
-    const float vy = (float)(iy - half_res) * voxel;
-    const float vz = (float)(iz - half_res) * voxel;
-    const float x = vx + random[i] * voxel;
-    const float y = vy + random[i + B] * voxel;
-    const float z = vz + random[i + 2 * B] * voxel;
-    pos[i] = (x * inv_aabb) + 0.5f;
-    pos[i + B] = (y * inv_aabb) + 0.5f;
-    pos[i + 2 * B] = (z * inv_aabb) + 0.5f;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const int ic = (int)compact_bits10(idx >> c);
+        const float v = (float)(ic - half_res) * voxel;
+        const float x = v + u[c] * voxel;
+        p[c] = (x * inv_aabb) + 0.5f;
+    }
 }
 
-// sigma_cell = max(sigma_cell, exp(min(s,12)-1)), with the reference's random
-// subset rule once training is past warm-up (reference :79-115)
+__global__ void occ_sample_points_kernel(uint32_t n_cells, uint32_t B, uint32_t start_idx, int res, int level,
+                                         float inv_aabb, const float* __restrict__ random, float* __restrict__ pos) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_cells) return;
+    const float u[3] = {random[i], random[i + B], random[i + 2 * B]};
+    float p[3];
+    cell_point(i + start_idx, res, level, inv_aabb, u, p);
+    pos[i] = p[0];
+    pos[i + B] = p[1];
+    pos[i + 2 * B] = p[2];
+}
+
+// elements g .. g + 3 of the uniform stream keyed by (k0, k1): one block of it
+// when g is a multiple of four, else two
+TN_DEVICE void uniform4(uint64_t g, uint32_t k0, uint32_t k1, float u[4]) {
+    const uint64_t block = g >> 2;
+    uint32_t c[8] = {(uint32_t)block, (uint32_t)(block >> 32), 0u, 0u, 0u, 0u, 0u, 0u};
+    philox4x32_10(c, k0, k1);
+    const uint32_t m = (uint32_t)g & 3u;
+    if (m != 0u) {
+        c[4] = (uint32_t)(block + 1);
+        c[5] = (uint32_t)((block + 1) >> 32);
+        philox4x32_10(c + 4, k0, k1);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        u[k] = u32_to_unit(m == 0u ? c[k] : m == 1u ? c[k + 1] : m == 2u ? c[k + 2] : c[k + 3 < 8 ? k + 3 : 7]);
+}
+
+// The two passes of a grid refresh around the network, drawing their uniforms
+// themselves: cell i takes elements i, B + i, 2B + i (its point) and 3B + i (the
+// subset rule) of the stream from `offset` on. Four cells per thread share the
+// generator's blocks of four; each launch is as long as a launch is (5 us for
+// 262,144 cells, their bytes take 1). A fill of 4B uniforms that both passes
+// read was a third such launch per chunk: a refresh of three cascades of 128^3
+// cells took 1.97 ms with it and 1.92 without.
+__global__ void occ_draw_points_kernel(uint32_t n_cells, uint32_t B, uint32_t start_idx, int res, int level,
+                                       float inv_aabb, uint32_t k0, uint32_t k1, uint64_t offset,
+                                       float* __restrict__ pos) {
+    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (i >= n_cells) return;
+    float u[3][4], p[3][4];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) uniform4(offset + (uint64_t)c * B + i, k0, k1, u[c]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float uk[3] = {u[0][k], u[1][k], u[2][k]};
+        float q[3];
+        cell_point(i + k + start_idx, res, level, inv_aabb, uk, q);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) p[c][k] = q[c];
+    }
+    if ((B & 3u) == 0u && i + 4 <= n_cells) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            *reinterpret_cast<float4*>(pos + (uint64_t)c * B + i) = make_float4(p[c][0], p[c][1], p[c][2], p[c][3]);
+    } else {
+        for (uint32_t k = 0; k < 4 && i + k < n_cells; ++k)
+            for (int c = 0; c < 3; ++c) pos[(uint64_t)c * B + i + k] = p[c][k];
+    }
+}
+
+// the reference's random subset rule once training is past warm-up (:79-115)
+TN_DEVICE bool cell_sampled(float r, uint8_t bits, int level) {
+    if (r > 0.5f) return false;
+    return r < 0.25f || ((bits >> level) & 1u) != 0u;
+}
+
+// sigma_cell = max(sigma_cell, exp(min(s,12)-1)) (reference :79-115)
+TN_DEVICE float updated_density(float raw, float density) { return fmaxf(__expf(fminf(raw, 12.0f) - 1.0f), density); }
+
 template <typename TIn>
 __global__ void occ_update_density_kernel(uint32_t n_cells, uint32_t start_idx, uint32_t volume, int level,
                                           int sample_all, const float* __restrict__ random,
@@ -57,14 +117,36 @@ __global__ void occ_update_density_kernel(uint32_t n_cells, uint32_t start_idx, 
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_cells) return;
     const uint32_t idx = i + start_idx;
-    if (!sample_all) {
-        const float r = random[i];
-        if (r > 0.5f) return;
-        if (!(r < 0.25f) && !((bits[idx] >> level) & 1u)) return;
-    }
-    const float sigma = __expf(fminf((float)raw[i], 12.0f) - 1.0f);
+    if (!sample_all && !cell_sampled(random[i], bits[idx], level)) return;
     float* p = density + (uint64_t)level * volume + idx;
-    *p = fmaxf(sigma, *p);
+    *p = updated_density((float)raw[i], *p);
+}
+
+template <typename TIn>
+__global__ void occ_draw_update_kernel(uint32_t n_cells, uint32_t B, uint32_t start_idx, uint32_t volume, int level,
+                                       int sample_all, uint32_t k0, uint32_t k1, uint64_t offset,
+                                       const TIn* __restrict__ raw, const uint8_t* __restrict__ bits,
+                                       float* __restrict__ density) {
+    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    if (i >= n_cells) return;
+    float u[4];
+    if (!sample_all) uniform4(offset + 3 * (uint64_t)B + i, k0, k1, u);
+    const uint32_t idx = i + start_idx;
+    float* const p = density + (uint64_t)level * volume + idx;
+    const bool whole = i + 4 <= n_cells;
+    if (sample_all && whole && ((start_idx | volume) & 3u) == 0u) {
+        float4 v = *reinterpret_cast<const float4*>(p);
+        v.x = updated_density((float)raw[i], v.x);
+        v.y = updated_density((float)raw[i + 1], v.y);
+        v.z = updated_density((float)raw[i + 2], v.z);
+        v.w = updated_density((float)raw[i + 3], v.w);
+        *reinterpret_cast<float4*>(p) = v;
+        return;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        if (i + k < n_cells && (sample_all || cell_sampled(u[k], bits[idx + k], level)))
+            p[k] = updated_density((float)raw[i + k], p[k]);
 }
 
 // byte = sum_k [density_k > threshold] << k (reference :118-141); one thread
@@ -210,6 +292,46 @@ extern "C" int tn_occ_sample_points(uint32_t n_cells, uint32_t stride, uint32_t 
     if (n_cells == 0) return TN_OK;
     occ_sample_points_kernel<<<blocks_for(n_cells, 256), 256, 0, stream>>>(n_cells, stride, start_idx, grid.resolution,
                                                                            level, inv_aabb, random, pos);
+    TN_CHECK_LAUNCH();
+    return TN_OK;
+}
+
+// As tn_occ_sample_points with `random` the 4 stride uniforms of tn_fill_uniform at (seed, offset)
+extern "C" int tn_occ_draw_points(uint32_t n_cells, uint32_t stride, uint32_t start_idx, tn_occupancy_grid_t grid,
+                                  int level, float inv_aabb, uint64_t seed, uint64_t offset, float* pos,
+                                  hipStream_t stream) {
+    TN_CHECK_ARG(pos && n_cells <= stride && level >= 0 && level < grid.n_levels);
+    TN_CHECK_ARG((reinterpret_cast<uintptr_t>(pos) & 15) == 0);
+    const uint32_t volume = (uint32_t)(grid.resolution * grid.resolution * grid.resolution);
+    TN_CHECK_ARG((uint64_t)start_idx + n_cells <= volume);
+    if (n_cells == 0) return TN_OK;
+    occ_draw_points_kernel<<<blocks_for(((uint64_t)n_cells + 3) / 4, 256), 256, 0, stream>>>(
+        n_cells, stride, start_idx, grid.resolution, level, inv_aabb, (uint32_t)seed, (uint32_t)(seed >> 32), offset,
+        pos);
+    TN_CHECK_LAUNCH();
+    return TN_OK;
+}
+
+// As tn_occ_update_density with `random` the last `stride` of those uniforms
+extern "C" int tn_occ_draw_update(int raw_dtype, uint32_t n_cells, uint32_t stride, uint32_t start_idx,
+                                  tn_occupancy_grid_t grid, int level, int sample_all_cells, uint64_t seed,
+                                  uint64_t offset, const void* raw_density, hipStream_t stream) {
+    TN_CHECK_ARG(raw_density && grid.density && grid.bitfield && level >= 0 && level < grid.n_levels);
+    TN_CHECK_ARG(n_cells <= stride && (reinterpret_cast<uintptr_t>(grid.density) & 15) == 0);
+    const uint32_t volume = (uint32_t)(grid.resolution * grid.resolution * grid.resolution);
+    TN_CHECK_ARG((uint64_t)start_idx + n_cells <= volume);
+    if (raw_dtype != 0 && raw_dtype != 1) return TN_ERR_INVALID_ARGUMENT;
+    if (n_cells == 0) return TN_OK;
+    const unsigned blocks = blocks_for(((uint64_t)n_cells + 3) / 4, 256);
+    const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+    if (raw_dtype == 0)
+        occ_draw_update_kernel<float><<<blocks, 256, 0, stream>>>(
+            n_cells, stride, start_idx, volume, level, sample_all_cells, k0, k1, offset,
+            static_cast<const float*>(raw_density), grid.bitfield, grid.density);
+    else
+        occ_draw_update_kernel<_Float16><<<blocks, 256, 0, stream>>>(
+            n_cells, stride, start_idx, volume, level, sample_all_cells, k0, k1, offset,
+            static_cast<const _Float16*>(raw_density), grid.bitfield, grid.density);
     TN_CHECK_LAUNCH();
     return TN_OK;
 }
