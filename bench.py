@@ -79,7 +79,7 @@ KERNEL = {
     "composite": ("composite_chunk_kernel", "composite_ray_kernel", "composite_grad_kernel"),
     "loss_reduce": ("step_metrics_kernel",),
     "march_count": ("march_count_kernel",),
-    "march_generate": ("march_generate_kernel", "march_expand_kernel"),
+    "march_generate": ("march_generate_runs_kernel",),
     "adam": ("adam_kernel",),
 }
 # phases on the network stream: the step's critical path (batch generation
@@ -647,7 +647,8 @@ def _short(name):
     base = name.split("(")[0]
     keys = {k for ks in KERNEL.values() for k in ks} | {
         "scan_tile_sums_kernel", "scan_tile_prefix_kernel", "scan_write_select_kernel", "uniform_kernel",
-        "init_training_rays_kernel", "estimate_rays_kernel", "reduce_partials_kernel",
+        "training_rays_kernel", "batch_select_kernel", "reduce_partials_kernel", "occ_draw_points_kernel",
+        "occ_draw_update_kernel",
         "write_rgba_kernel", "cast_kernel", "composite_forward_kernel", "render_rays_kernel"}
     for key in sorted(keys, key=len, reverse=True):
         if key in base:

@@ -12,9 +12,9 @@
 // distribution once the next layer's weight columns are permuted the same
 // way (dt_in below). Weight gradients dW = delta * act^T use the same MFMA
 // with samples as the K dimension after both tiles are transposed through
-// LDS; each wave keeps its 12 dW accumulator tiles in registers for all the
-// tiles it processes and the workgroup sums them before one partial per
-// workgroup goes to memory.
+// LDS; the four waves of a workgroup share the dW tiles, each keeping five in
+// registers for all the tiles it processes, and one partial per workgroup goes
+// to memory.
 //
 // Mixed precision keeps the fp16 operands of the first layer of each MLP
 // exact to about 2^-22: the hash features, the hidden layer h1, the density
