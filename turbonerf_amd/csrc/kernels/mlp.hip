@@ -626,9 +626,15 @@ TN_DEVICE BwdLds<P> stage_backward(typename P::T* lds, const typename P::T* __re
 constexpr int kGrp = 32 * kMlpWaves;  // samples per workgroup step
 static_assert(kMlpWaves == 4, "the dW split assumes four waves");
 
-// fp32 buffers: [row][sample], row stride 129 (the +1 spreads banks)
+// fp32 buffers: [row][sample], a row's even samples first and its odd ones 80
+// further on, so that a lane's operands of four K-steps (samples 2ks + h of its
+// row) are 16 bytes that one read brings. 80 = 64 + 16 keeps a row's writes on
+// 32 banks, and rows of 148 words (148 = 20 mod 64) put 16 rows' reads on 64.
+// (One value per read from rows of 129: 125 us a launch at 100 k samples, 105
+// with this. With the weights the buffers take all 160 KiB of LDS.)
 template <class P>
-constexpr int kGW = kGrp + 1;
+constexpr int kGW = 148;
+TN_DEVICE int grp_pos(int n) { return (n & 1) * 80 + (n >> 1); }
 // fp16 buffers: [sample][row], sample stride 100 fp16 = 200 bytes (64 rows
 // and padding): 200 = 8 * 25 with 25 odd puts the 8-byte writes of 32
 // consecutive samples in 32 distinct bank pairs, and the four samples of a
@@ -666,7 +672,7 @@ TN_DEVICE void put_grp(typename P::T* buf, int t, int w, const OpTile<P>& A, int
     } else {
         const int n = 32 * w + (lane & 31), h = (lane >> 5) & 1;
 #pragma unroll
-        for (int r = 0; r < (HALF ? 8 : 16); ++r) buf[acc_row(t, r, h) * kGW<P> + n] = op_get<P>(A, r);
+        for (int r = 0; r < (HALF ? 8 : 16); ++r) buf[acc_row(t, r, h) * kGW<P> + grp_pos(n)] = op_get<P>(A, r);
     }
 }
 
@@ -677,7 +683,7 @@ TN_DEVICE void put_grp(typename P::T* buf, int t, int w, const f16v& D, int lane
     } else {
         const int n = 32 * w + (lane & 31), h = (lane >> 5) & 1;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) buf[acc_row(t, r, h) * kGW<P> + n] = D[r];
+        for (int r = 0; r < 16; ++r) buf[acc_row(t, r, h) * kGW<P> + grp_pos(n)] = D[r];
     }
 }
 
@@ -696,36 +702,44 @@ TN_DEVICE void put_grp_nat(typename P::T* buf, int base, int w, const typename P
     } else {
         const int n = 32 * w + (lane & 31), h = (lane >> 5) & 1;
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) buf[(base + nat_in<P>(ks, h, 0)) * kGW<P> + n] = x[ks];
+        for (int ks = 0; ks < NKS; ++ks) buf[(base + nat_in<P>(ks, h, 0)) * kGW<P> + grp_pos(n)] = x[ks];
     }
 }
 
-// operand holding group samples [ks*KC + h*SL, +SL) of row 32*t + (lane & 31)
-template <class P>
-TN_DEVICE typename P::Op grp_rows(const typename P::T* buf, int t, int ks, int lane) {
-    if constexpr (P::SL == 8) {
-        // group G = lane / 16 reads rows 32t + 16(G % 2) + (0..15) of samples
-        // 16ks + 8(G / 2) + (0..7); its lane 4e + q addresses sample e (and
-        // e + 4 in the second read), rows 4q..4q+3 of those 16
-        const int G = lane >> 4, jj = lane & 15;
-        const typename P::T* p =
-            buf + (16 * ks + 8 * (G >> 1) + (jj >> 2)) * kTrRows + 32 * t + 16 * (G & 1) + 4 * (jj & 3);
-        typedef s4v __attribute__((address_space(3))) * lds_s4v;
-        const s4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4v)(p));
-        const s4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4v)(p + 4 * kTrRows));
-        return __builtin_bit_cast(typename P::Op, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
-    } else {
-        const int row = 32 * t + (lane & 31), h = lane >> 5;
-        return buf[row * kGW<P> + ks * P::KC + h * P::SL];
-    }
+// fp32: the operands of K-steps [ks, ks + 4) of row 32*t + (lane & 31), ks a multiple of 4
+typedef float f4v __attribute__((ext_vector_type(4)));
+TN_DEVICE f4v grp_row4(const float* buf, int t, int ks, int lane) {
+    return *reinterpret_cast<const f4v*>(buf + (32 * t + (lane & 31)) * kGW<PrecF32> + (lane >> 5) * 80 + ks);
+}
+
+// fp16: operand holding group samples [ks*KC + h*SL, +SL) of row 32*t + (lane & 31)
+TN_DEVICE h8v grp_rows(const _Float16* buf, int t, int ks, int lane) {
+    // group G = lane / 16 reads rows 32t + 16(G % 2) + (0..15) of samples
+    // 16ks + 8(G / 2) + (0..7); its lane 4e + q addresses sample e (and
+    // e + 4 in the second read), rows 4q..4q+3 of those 16
+    const int G = lane >> 4, jj = lane & 15;
+    const _Float16* p = buf + (16 * ks + 8 * (G >> 1) + (jj >> 2)) * kTrRows + 32 * t + 16 * (G & 1) + 4 * (jj & 3);
+    typedef s4v __attribute__((address_space(3))) * lds_s4v;
+    const s4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4v)(p));
+    const s4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4v)(p + 4 * kTrRows));
+    return __builtin_bit_cast(h8v, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
 // C += delta rows (tile mt) x act rows (tile nt)^T over group K-steps [ks0, ks1)
 template <class P>
 TN_DEVICE f16v dw_tile(f16v c, const typename P::T* dbuf, const typename P::T* abuf, int mt, int nt, int ks0,
                        int ks1, int lane) {
+    if constexpr (P::SL == 8) {
 #pragma unroll 4
-    for (int ks = ks0; ks < ks1; ++ks) c = P::mma(grp_rows<P>(dbuf, mt, ks, lane), grp_rows<P>(abuf, nt, ks, lane), c);
+        for (int ks = ks0; ks < ks1; ++ks) c = P::mma(grp_rows(dbuf, mt, ks, lane), grp_rows(abuf, nt, ks, lane), c);
+    } else {
+#pragma unroll 4
+        for (int ks = ks0; ks < ks1; ks += 4) {
+            const f4v d = grp_row4(dbuf, mt, ks, lane), a = grp_row4(abuf, nt, ks, lane);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) c = P::mma(d[k], a[k], c);
+        }
+    }
     return c;
 }
 
@@ -776,7 +790,6 @@ TN_DEVICE void store_dw_tile(float* out, const f16v& C, int mt, int nt, int n_ou
 }
 
 // a tile's accumulators to and from LDS, 1024 floats, four registers of a lane together
-typedef float f4v __attribute__((ext_vector_type(4)));
 TN_DEVICE void put_acc(float* buf, const f16v& C, int lane) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
