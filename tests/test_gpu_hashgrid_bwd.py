@@ -468,3 +468,59 @@ def test_sorted_fp32_records(cuda, n, log2_T):
     ti, ta = direct(bad).cpu().numpy(), torch.zeros(g.n_params, device="cuda")
     ops.hashgrid_backward(g, n, p, n, bad, ta)
     assert np.array_equal(np.isfinite(ti), np.isfinite(ta.cpu().numpy()))
+
+
+@pytest.mark.parametrize("path", ["atomic", "binned", "planned", "sorted"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_nonfinite_positions_stay_with_their_entries(cuda, path, bad):
+    """Samples with a non-finite coordinate have weights and contributions
+    that are NaN, and no others have: every level's NaN entries are the eight
+    corners of those samples' cells (the conversion to a cell index saturates,
+    and takes NaN to 0), every other entry is the gradient of the batch without
+    them. In the middle and at either end of runs and waves, at few levels with
+    merged runs and at fine ones with hardly any."""
+    import torch
+
+    from turbonerf_amd import _capi, ops
+
+    print(f"[hash bwd non-finite] {path} {bad}", flush=True)
+    g = ops.hashgrid_layout(log2_T=14)
+    rng = np.random.default_rng(5)
+    pos = _rays(rng, 90, 100, 0.0011)
+    n = pos.shape[1]
+    dfeat = rng.normal(size=(32, n)).astype(np.float32)
+    at = np.array([0, 63, 64, 130, 1000, 4321, n - 1])
+    clean, cut = pos.copy(), dfeat.copy()
+    clean[:, at], cut[:, at] = 0.5, 0.0
+    pos[rng.integers(0, 3, len(at)), at] = bad
+    own = np.zeros(g.n_params // 2, bool)
+    lim = np.float64(2 ** 31)
+    for l in range(g.n_levels):
+        s, r, size = np.float32(g.scale[l]), g.resolution[l], g.level_size[l]
+        with np.errstate(invalid="ignore"):
+            x = np.floor((pos[:, at] * s + np.float32(0.5)).astype(np.float32)).astype(np.float64)
+        c = np.where(np.isnan(x), 0.0, np.clip(x, -lim, lim - 1)).astype(np.int64)
+        for k in range(8):
+            q = [(c[a] + ((k >> a) & 1)) & 0xFFFFFFFF for a in range(3)]
+            if g.level_dense[l]:
+                i = ((q[0] + q[1] * r + q[2] * r * r) & 0xFFFFFFFF) % size
+            else:
+                i = (q[0] ^ ((q[1] * 2654435761) & 0xFFFFFFFF) ^ ((q[2] * 805459861) & 0xFFFFFFFF)) & (size - 1)
+            own[g.level_offset[l] + i] = True
+    own = np.repeat(own, 2)
+    ref, mag = _oracle_bwd(g, clean, cut), _oracle_bwd(g, clean, np.abs(cut))
+    p, d = torch.from_numpy(np.ascontiguousarray(pos)).cuda(), torch.from_numpy(dfeat).cuda()
+    t = torch.zeros(g.n_params, device="cuda")
+    if path == "sorted":
+        nb = _capi.query("tn_hashgrid_backward_sorted_bytes", n, g)
+        ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+        _capi.call("tn_hashgrid_backward_sorted", 0, n, None, n, n, g, p.data_ptr(), d.data_ptr(), t.data_ptr(),
+                   ws.data_ptr(), nb, _capi.stream_ptr())
+    else:
+        ops.hashgrid_backward(g, n, p, n, d, t, binned=path == "binned", planned=path == "planned")
+    got = t.cpu().numpy()
+    assert np.array_equal(np.isnan(got), own), (np.isnan(got).sum(), own.sum())
+    # the bin of a NaN sums in fp32 in any order: up to n terms of 2^-24 each
+    # beside the records' own rounding (the module's bar)
+    err = np.abs(got[~own] - ref[~own])
+    assert np.all(err <= (6e-6 + n * 2.0 ** -24) * mag[~own] + 6.4e-8 * np.abs(dfeat).max()), err.max()

@@ -490,8 +490,9 @@ TN_DEVICE void seg_step16(float (&a0)[8], float (&a1)[8], int key) {
     }
 }
 
-// The same step for finite values of less than 2^100: take becomes a factor
-// of 1 or 0 of a fused multiply-add whose product operand is the shifted
+// The same step for weights in [0, 1] and gradients of less than 2^100, both
+// finite (0 times NaN would carry a sample's NaN into other runs): take becomes
+// a factor of 1 or 0 of a fused multiply-add whose product operand is the shifted
 // value, one instruction per value (exact: the factor is 1 or 0). Lanes whose
 // source is outside the row or in a row not selected are not written. The two
 // wait states before a DPP read of a fresh register are part of the block.
@@ -647,7 +648,8 @@ TN_DEVICE void hb_corners(const tn_hashgrid_t& g, int l, bool active, const HbIn
     if (hm != ~0ull) {
         const uint64_t le = lane == 63 ? ~0ull : ((1ull << (lane + 1)) - 1ull);
         constexpr float kSmall = 1.2676506e30f;  // 2^100: sums of a wave's values stay finite
-        const bool large = !(fabsf(v.g0) < kSmall) || !(fabsf(v.g1) < kSmall);
+        // a non-finite coordinate makes all eight weights NaN; others lie in [0, 1]
+        const bool large = !(fabsf(v.g0) < kSmall) || !(fabsf(v.g1) < kSmall) || !(c8.w[0] <= 1.0f);
         seg_sum16(a0, a1, __builtin_popcountll(hm & le), hm, __ballot(large) == 0ull);
     }
 #pragma unroll
