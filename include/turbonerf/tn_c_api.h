@@ -315,8 +315,10 @@ int tn_hashgrid_backward_binned(int dfeat_dtype, uint32_t n_max, const uint32_t*
     void* workspace, size_t workspace_bytes, tn_stream_t stream);
 
 /* The same sort with every contribution kept in fp32 (10-byte records instead
- * of 8): the accuracy of tn_hashgrid_backward, and a result that does not
- * depend on the order of the sums. Same replacement (reference
+ * of 8) and summed in fp64: an entry's error is relative to its own
+ * contributions, as in tn_hashgrid_backward, and its sum is rounded to fp32
+ * once. The order of the sums can show only in an entry whose m contributions
+ * span more than 2^29 / m. Same replacement (reference
  * src/core/nerf-network.cu:760). The workspace (256-byte aligned,
  * tn_hashgrid_backward_sorted_bytes, 0 = layout beyond the bin limits) is
  * scratch; without it the atomic kernel runs. dtable is 8-byte aligned. */

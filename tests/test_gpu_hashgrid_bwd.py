@@ -425,11 +425,13 @@ def test_binned_vs_fp64_central_differences(cuda):
 
 @pytest.mark.parametrize("n,log2_T", [(1, 12), (300, 19), (10_000, 12), (30_000, 19), (70_001, 21)])
 def test_sorted_fp32_records(cuda, n, log2_T):
-    """The sort with fp32 records (through the autograd layer's rule, on both
-    sides of it, and called directly) against float64: no further off than
-    the atomic scatter-add by more than the fixed-point rounding, added to a
-    non-zero table, the same bits from run to run, and a non-finite gradient
-    reaching the entries it belongs to."""
+    """The sort with fp32 records and fp64 sums (through the autograd layer's
+    rule, on both sides of it, and called directly) against float64: no further
+    off in norm than the atomic scatter-add, added to a non-zero table, the
+    same bits from run to run (an entry's contributions here hardly ever span
+    so much that fp64 sums of them round), and a non-finite gradient reaching
+    the entries it belongs to. Small contributions, which a norm does not see:
+    test_sorted_keeps_small_contributions."""
     import torch
 
     from turbonerf_amd import _capi, ops
@@ -458,7 +460,7 @@ def test_sorted_fp32_records(cuda, n, log2_T):
     t = direct(d)
     e_s, e_a = norm_rel(t.cpu().numpy(), ref), norm_rel(atomic.cpu().numpy(), ref)
     print(f"[hashgrid sorted] error {e_s:.2e}, atomic {e_a:.2e}", flush=True)
-    assert e_s <= e_a + 1e-7  # fp32 sums of runs, then exact sums rounded once
+    assert e_s <= e_a + 1e-7  # fp32 sums of runs, then sums rounded once
     assert torch.equal(t, direct(d))
     acc = torch.from_numpy(base).cuda()
     ops.hashgrid_backward_sorted(g, n, p, n, d, acc)
@@ -524,3 +526,36 @@ def test_nonfinite_positions_stay_with_their_entries(cuda, path, bad):
     # beside the records' own rounding (the module's bar)
     err = np.abs(got[~own] - ref[~own])
     assert np.all(err <= (6e-6 + n * 2.0 ** -24) * mag[~own] + 6.4e-8 * np.abs(dfeat).max()), err.max()
+
+
+@pytest.mark.parametrize("n,log2_T", [(30_000, 12), (30_000, 19), ((1 << 19) + 5003, 15)])
+def test_sorted_keeps_small_contributions(cuda, n, log2_T):
+    """Every entry's own relative accuracy, as the atomic scatter-add has it:
+    gradients of 2^-50 to 1 by ray and a second feature of 2^-20 of the first,
+    all within the same bins, per entry against sum |w g| in float64; also in
+    two parts (more than 2^19 samples), the second added to the first's table
+    through the same scratch. The bar: three subtractions, three products, six
+    sums of a run of 64 lanes and the sums' rounding to fp32, 2^-24 each, and
+    two more for the addition of a part."""
+    import torch
+
+    from turbonerf_amd import ops
+
+    print(f"[hashgrid sorted] small contributions: n {n} log2_T {log2_T}", flush=True)
+    g = ops.hashgrid_layout(log2_T=log2_T)
+    rng = np.random.default_rng(n)
+    n_rays = -(-n // 100)
+    pos = np.ascontiguousarray(_rays(rng, n_rays, 100, 0.0011)[:, :n])
+    dfeat = rng.normal(size=(32, n)) * np.repeat(2.0 ** -rng.uniform(0, 50, n_rays), 100)[:n]
+    dfeat[1::2] *= 2.0 ** -20
+    dfeat = dfeat.astype(np.float32)
+    ref, mag = _oracle_bwd(g, pos, dfeat), _oracle_bwd(g, pos, np.abs(dfeat))
+    p, d = torch.from_numpy(pos).cuda(), torch.from_numpy(dfeat).cuda()
+    t = torch.zeros(g.n_params, device="cuda")
+    ops.hashgrid_backward_sorted(g, n, p, n, d, t)
+    got = t.cpu().numpy()
+    bar = 15 * 2.0 ** -24 * mag + 1e-40
+    worst = np.abs(got - ref) / bar
+    print(f"[hashgrid sorted] worst/bar {worst.max():.3f}, entries over {np.sum(worst > 1)} of {np.sum(mag > 0)}, "
+          f"lost {np.sum((got == 0) & (np.abs(ref) > 1e-30))}", flush=True)
+    assert worst.max() <= 1.0

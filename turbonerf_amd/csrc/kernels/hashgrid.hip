@@ -386,12 +386,13 @@ __global__ void __launch_bounds__(256) hashgrid_bwd_kernel(uint32_t n_max, const
 // same bit for bit from run to run. A record is one sample's contribution to
 // both features of one corner entry, after runs of consecutive samples in one
 // cell have been merged; samples whose feature gradients are both zero emit
-// none. Sums in LDS are 64-bit fixed point (integer LDS atomics run several
-// times faster than float ones here): with every |v| < 2^E in the bin and m
+// none. HbRec8's sums in LDS are 64-bit fixed point, the same in any order: with every |v| < 2^E in the bin and m
 // records, the scale 2^S with S = 62 - E - ceil(log2(m + 1)) cannot overflow,
 // and the sum of the records is exact up to the rounding of each value to a
 // multiple of 2^-S (relative 2^-38 of the bin's largest value or better);
-// each record carries its value to 17 significant bits (HbRec8) or whole (HbRec10). Blocks of count and
+// each record carries its value to 17 significant bits. HbRec10's are fp64
+// sums of the whole values, which keep every entry's own relative accuracy
+// whatever its bin holds besides. Blocks of count and
 // scatter work on one level each: block b serves level b % L and the
 // contiguous 256-sample chunks [j, j + 1) * chunk_blocks, j = b / L, so the
 // records of a range of samples can be scattered on their own (the slots of
@@ -425,8 +426,11 @@ struct HbPlan {
 // (The scatter's write and the accumulation's read of the records bound both
 // passes; 12-byte records took 1.5 times as long.) Callers that ask for fp32
 // contributions get HbRec10: both values as they are and the entry in 16 bits,
-// in arrays of their own. All passes, plan included, on 262,144 samples along
-// rays: 172 us with HbRec8, 221 us with HbRec10; 754 us by atomics.
+// in arrays of their own, summed in fp64 (kFixed: in fixed point relative to
+// the bin's largest value, which takes an entry whose values are all below
+// 2^-38 of it to zero). All passes, plan included, on 262,144 samples along
+// rays: 177 us with HbRec8, 198 us with HbRec10 (217 in fixed point, with its
+// maxima); 754 us by atomics. 524,288 samples: 339, 428 (387) and 1,493 us.
 
 // v rounded to 17 significant bits (half away from zero; a carry may raise the
 // exponent, up to inf), low 6 bits cleared; inf and NaN keep their pattern
@@ -437,7 +441,7 @@ TN_DEVICE uint32_t hb_round17(float v) {
 }
 
 struct HbRec8 {
-    static constexpr bool kEntryArray = false;
+    static constexpr bool kEntryArray = false, kFixed = true;
     static constexpr size_t kBytes = 8;
     TN_DEVICE static uint32_t value(float v) { return hb_round17(v); }
     TN_DEVICE static uint2 pack(uint32_t e, uint32_t r0, uint32_t r1) { return make_uint2(r0 | (e & 63u), r1 | (e >> 6)); }
@@ -446,7 +450,7 @@ struct HbRec8 {
     TN_DEVICE static float v1(uint2 r) { return __uint_as_float(r.y & ~63u); }
 };
 struct HbRec10 {
-    static constexpr bool kEntryArray = true;
+    static constexpr bool kEntryArray = true, kFixed = false;
     static constexpr size_t kBytes = 10;
     TN_DEVICE static uint32_t value(float v) { return __float_as_uint(v); }
     TN_DEVICE static uint2 pack(uint32_t, uint32_t r0, uint32_t r1) { return make_uint2(r0, r1); }
@@ -822,7 +826,8 @@ __global__ void __launch_bounds__(1024) hashgrid_bwd_scan_kernel(HbPlan p, const
 // stores go out as runs of whole lines instead of one 8-byte request per
 // record, whose rate bounded the unsorted version. The order of records
 // within a bin depends on the order of the LDS atomics; the accumulation sums
-// them exactly (fixed point), so the result does not.
+// HbRec8's exactly (fixed point), so the result does not, and HbRec10's in
+// fp64, exact too unless the m values of an entry span more than 2^29 / m.
 constexpr uint32_t kHbScatterThreads = 256;
 constexpr uint32_t kHbChunkRecords = 8 * kHbScatterThreads;
 static_assert(kHbMaxLevelBins <= 2 * kHbScatterThreads, "two bins per thread in the chunk scan");
@@ -881,11 +886,11 @@ __global__ void __launch_bounds__(kHbScatterThreads) hashgrid_bwd_scatter_kernel
                 const bool one = bin[k] == bin[k + 1];
                 rank[k] = atomicAdd(&cnt[bin[k]], one ? 2u : 1u);
                 rank[k + 1] = rank[k] + 1u;
-                const uint32_t m0 = one ? max(m[0], m[1]) : m[0];
-                if (m0 != 0u) atomicMax(&bmax[bin[k]], m0);
-                if (!one) {
-                    rank[k + 1] = atomicAdd(&cnt[bin[k + 1]], 1u);
-                    if (m[1] != 0u) atomicMax(&bmax[bin[k + 1]], m[1]);
+                if (!one) rank[k + 1] = atomicAdd(&cnt[bin[k + 1]], 1u);
+                if constexpr (Rec::kFixed) {
+                    const uint32_t m0 = one ? max(m[0], m[1]) : m[0];
+                    if (m0 != 0u) atomicMax(&bmax[bin[k]], m0);
+                    if (!one && m[1] != 0u) atomicMax(&bmax[bin[k + 1]], m[1]);
                 }
             }
         }
@@ -941,9 +946,11 @@ __global__ void __launch_bounds__(kHbScatterThreads) hashgrid_bwd_scatter_kernel
             }
         }
     }
-    __syncthreads();
-    for (uint32_t k = tid; k < nb; k += kHbScatterThreads)
-        binmax[(uint64_t)(p.base[l] + k) * p.level_blocks + j] = bmax[k];
+    if constexpr (Rec::kFixed) {
+        __syncthreads();
+        for (uint32_t k = tid; k < nb; k += kHbScatterThreads)
+            binmax[(uint64_t)(p.base[l] + k) * p.level_blocks + j] = bmax[k];
+    }
 }
 
 // the largest |value| bits of bin k: the maximum over its row of binmax
@@ -959,6 +966,10 @@ TN_DEVICE uint32_t hb_bin_max(const HbPlan& p, const uint32_t* __restrict__ binm
 }
 
 TN_DEVICE long long hb_fixed(float v, int S) { return (long long)rintf(ldexpf(v, S)); }
+// one LDS instruction (ds_add_f64)
+TN_DEVICE void hb_add(double* acc, float v) {
+    __hip_atomic_fetch_add(acc, (double)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 
 // the complete sums (v0, v1) of table entry `entry` added to dtable
 TN_DEVICE void hb_finish_entry(float* __restrict__ dtable, uint32_t entry, float v0, float v1) {
@@ -1109,12 +1120,12 @@ TN_DEVICE int hb_scale(uint32_t bits, uint64_t m) {
     return 62 - E - (32 - __builtin_clz((uint32_t)m + 1u));
 }
 
-// (4) one block per chunk of a bin: fixed-point sums in LDS. A bin summed by
-// one block adds its sums to dtable here; a bin split over several
-// blocks leaves each block's exact 64-bit partial sums in its slot for (5),
-// so the result does not depend on the order the blocks run in. A bin
-// holding a non-finite value sums in float and adds into dtable atomically
-// instead, so inf and NaN reach the table.
+// (4) one block per chunk of a bin: sums in LDS, in fixed point or (not
+// kFixed) in fp64. A bin summed by one block adds its sums to dtable here; a
+// bin split over several blocks leaves each block's 64-bit partial sums in its
+// slot for (5), so the result does not depend on the order the blocks run in.
+// In fixed point, a bin holding a non-finite value sums in float and adds into
+// dtable atomically instead, so inf and NaN reach the table.
 template <class Rec>
 __global__ void __launch_bounds__(512) hashgrid_bwd_accumulate_kernel(tn_hashgrid_t g, HbPlan p,
                                                                       const uint32_t* __restrict__ start,
@@ -1141,13 +1152,16 @@ __global__ void __launch_bounds__(512) hashgrid_bwd_accumulate_kernel(tn_hashgri
     const HbBin bin = hb_bin(g, p, k);
     const uint32_t ne = bin.ne;
     for (uint32_t e = threadIdx.x; e < 2 * ne; e += blockDim.x) acc[e] = 0ull;
-    const uint32_t bits = hb_bin_max(p, binmax, k, &smax);  // its barriers also order the clearing
+    uint32_t bits = 0u;
+    if constexpr (Rec::kFixed) bits = hb_bin_max(p, binmax, k, &smax);  // its barriers also order the clearing
+    else __syncthreads();
     const uint64_t b0 = start[k], b1 = min((uint64_t)start[k + 1], p.cap);
     const uint64_t r0 = b0 + (uint64_t)part * kHbChunk;
     const uint64_t r1 = min(b1, r0 + kHbChunk);
     const bool finite = bits < 0x7F800000u;
     const int S = hb_scale(bits, b1 > b0 ? b1 - b0 : 0);
     float* accf = reinterpret_cast<float*>(acc);
+    double* accd = reinterpret_cast<double*>(acc);
     constexpr int kRecUnroll = 8;  // records in flight per lane
     for (uint64_t r = r0 + threadIdx.x; r < r1; r += kRecUnroll * blockDim.x) {
         uint2 q[kRecUnroll];
@@ -1165,7 +1179,10 @@ __global__ void __launch_bounds__(512) hashgrid_bwd_accumulate_kernel(tn_hashgri
         for (int u = 0; u < kRecUnroll; ++u) {
             const uint32_t e = Rec::entry(q[u], qe[u]);
             if (!in[u] || e >= ne) continue;
-            if (finite) {
+            if constexpr (!Rec::kFixed) {
+                hb_add(&accd[2 * e], Rec::v0(q[u]));
+                hb_add(&accd[2 * e + 1], Rec::v1(q[u]));
+            } else if (finite) {
                 atomicAdd(&acc[2 * e], (unsigned long long)hb_fixed(Rec::v0(q[u]), S));
                 atomicAdd(&acc[2 * e + 1], (unsigned long long)hb_fixed(Rec::v1(q[u]), S));
             } else {
@@ -1205,7 +1222,9 @@ __global__ void __launch_bounds__(512) hashgrid_bwd_accumulate_kernel(tn_hashgri
 #pragma unroll
             for (int f = 0; f < 4; ++f) {
                 float x = 0.0f;
-                if (valid[u] && finite) {
+                if (!Rec::kFixed && valid[u]) {
+                    x = (float)accd[2 * e + f];
+                } else if (valid[u] && finite) {
                     const long long q = (long long)acc[2 * e + f];
                     if (q != 0) x = (float)ldexp((double)q, -S);
                 } else if (valid[u]) {
@@ -1237,11 +1256,12 @@ __global__ void __launch_bounds__(512) hashgrid_bwd_accumulate_kernel(tn_hashgri
 }
 
 // (5) bins split over several blocks: the sum of their partial sums, in slot
-// order (exact in 64 bits), finished like a one-block bin. Work items are
+// order, finished like a one-block bin. Work items are
 // (split bin, 512 entries of it); blocks stride over them.
 constexpr uint32_t kHbFinishThreads = 512;
 constexpr uint32_t kHbFinishItems = kHbBinEntries / kHbFinishThreads;  // per bin
 constexpr uint32_t kHbFinishBlocks = 256;
+template <class Rec>
 __global__ void __launch_bounds__(kHbFinishThreads) hashgrid_bwd_finish_kernel(
     tn_hashgrid_t g, HbPlan p, const uint32_t* __restrict__ start, const uint32_t* __restrict__ chunk_start,
     const uint32_t* __restrict__ binmax, const uint32_t* __restrict__ slot_base, const uint32_t* __restrict__ split_list,
@@ -1252,8 +1272,11 @@ __global__ void __launch_bounds__(kHbFinishThreads) hashgrid_bwd_finish_kernel(
     const float lr = adam.w ? step_lr(adam.lr0, adam.d_step, adam.lr_decay) : 0.0f;
     for (uint32_t w = blockIdx.x; w < items; w += gridDim.x) {
         const uint32_t k = split_list[w / kHbFinishItems];
-        const uint32_t bits = hb_bin_max(p, binmax, k, &smax);
-        __syncthreads();  // smax is rewritten by the next item
+        uint32_t bits = 0u;
+        if constexpr (Rec::kFixed) {
+            bits = hb_bin_max(p, binmax, k, &smax);
+            __syncthreads();  // smax is rewritten by the next item
+        }
         const uint32_t nparts = chunk_start[k + 1] - chunk_start[k], s0 = slot_base[k];
         // non-finite, or beyond the slots: (4) added the bin into dtable
         // atomically; with Adam its step is taken from there
@@ -1264,7 +1287,18 @@ __global__ void __launch_bounds__(kHbFinishThreads) hashgrid_bwd_finish_kernel(
         const bool valid = e < bin.ne;
         const uint32_t entry = g.level_offset[bin.l] + bin.local0 + e;
         float v0 = 0.0f, v1 = 0.0f;
-        if (valid && in_slots) {
+        if (!Rec::kFixed && valid && in_slots) {
+            const double2* src = reinterpret_cast<const double2*>(slots) + (uint64_t)s0 * kHbBinEntries + e;
+            double d0 = 0.0, d1 = 0.0;
+#pragma unroll 4
+            for (uint32_t j = 0; j < nparts; ++j) {
+                const double2 t = src[(uint64_t)j * kHbBinEntries];
+                d0 += t.x;
+                d1 += t.y;
+            }
+            v0 = (float)d0;
+            v1 = (float)d1;
+        } else if (valid && in_slots) {
             const uint64_t b0 = start[k], b1 = min((uint64_t)start[k + 1], p.cap);
             const int S = hb_scale(bits, b1 > b0 ? b1 - b0 : 0);
             const ulonglong2* src = reinterpret_cast<const ulonglong2*>(slots) + (uint64_t)s0 * kHbBinEntries + e;
@@ -1377,7 +1411,9 @@ template <class Rec = HbRec8>
 inline size_t hb_work_area(const HbPlan& p, void* base, HbWorkArea* wa) {
     HbCarver c{static_cast<unsigned char*>(base)};
     HbWorkArea a;
-    a.binmax = reinterpret_cast<uint32_t*>(c.take((size_t)p.n_bins * p.level_blocks * sizeof(uint32_t)));
+    a.binmax = nullptr;
+    if (Rec::kFixed)
+        a.binmax = reinterpret_cast<uint32_t*>(c.take((size_t)p.n_bins * p.level_blocks * sizeof(uint32_t)));
     a.slots = reinterpret_cast<unsigned long long*>(
         c.take((size_t)p.split_slots * 2 * kHbBinEntries * sizeof(unsigned long long)));
     a.rec.val = reinterpret_cast<uint2*>(c.take((size_t)p.cap * sizeof(uint2)));
@@ -1429,9 +1465,10 @@ inline void hb_accumulate(uint32_t n_max, const tn_hashgrid_t& g, const HbPlan& 
 }
 
 // (5)
+template <class Rec>
 inline void hb_finish(const tn_hashgrid_t& g, const HbPlan& p, float* dtable, const HbPlanArea& pa,
                       const HbWorkArea& wa, const HbAdam& adam, hipStream_t stream) {
-    hashgrid_bwd_finish_kernel<<<kHbFinishBlocks, kHbFinishThreads, 0, stream>>>(
+    hashgrid_bwd_finish_kernel<Rec><<<kHbFinishBlocks, kHbFinishThreads, 0, stream>>>(
         g, p, pa.start, pa.chunk_start, wa.binmax, pa.slot_base, pa.split_list, wa.slots, dtable, adam);
 }
 
@@ -1451,7 +1488,7 @@ void hashgrid_backward_planned(uint32_t n_max, const uint32_t* info, uint32_t B,
         hb_scatter<TG, Rec>(n_max, info, B, GB, g, p, pos, dfeat, pa, wa, l0, Lg, 0, p.level_blocks, stream);
         hb_accumulate<Rec>(n_max, g, p, dtable, pa, wa, l0, Lg, adam, stream);
     }
-    hb_finish(g, p, dtable, pa, wa, adam, stream);
+    hb_finish<Rec>(g, p, dtable, pa, wa, adam, stream);
 }
 
 inline bool hb_layout_ok(const tn_hashgrid_t& g) {
@@ -1607,9 +1644,8 @@ extern "C" int tn_hashgrid_backward_binned(int dfeat_dtype, uint32_t n_max, cons
 }
 
 // The scatter-add of tn_hashgrid_backward through the same sort with fp32
-// records (each contribution whole, as the atomic kernel adds it), for callers
-// that want its accuracy without its cost; the result does not depend on the
-// order of the sums. A missing or short workspace, or a layout beyond the bin
+// records (each contribution whole, as the atomic kernel adds it) and sums in
+// fp64, for callers that want its accuracy without its cost. A missing or short workspace, or a layout beyond the bin
 // limits, takes the atomic kernel.
 extern "C" size_t tn_hashgrid_backward_sorted_bytes(uint32_t n_max, tn_hashgrid_t grid) {
     HbPlan p;
@@ -1801,7 +1837,7 @@ static int hb_accumulate_all(uint32_t n_max, tn_hashgrid_t grid, float* dtable, 
     hb_plan_area(p, const_cast<void*>(plan), &pa);
     hb_work_area(p, work, &wa);
     hb_accumulate<HbRec8>(n_max, grid, p, dtable, pa, wa, 0, (uint32_t)grid.n_levels, adam, stream);
-    hb_finish(grid, p, dtable, pa, wa, adam, stream);
+    hb_finish<HbRec8>(grid, p, dtable, pa, wa, adam, stream);
     TN_CHECK_LAUNCH();
     return TN_OK;
 }

@@ -293,13 +293,14 @@ def hashgrid_backward_sorted(grid: _capi.HashGrid, n: int, pos: torch.Tensor, st
                              dtable: torch.Tensor) -> None:
     """dtable += the table gradient, every contribution in fp32 as the atomic
     scatter-add has it. Large batches go through the sort with fp32 records
-    (tn_hashgrid_backward_sorted), in parts of at most 2^19 samples. Small ones
-    take the atomics: those cost 2.9 us per 1,000 samples, the sort 0.7 us and,
-    for its passes over every bin, 30 us with 2^15 entries per level, 48 us
-    with 2^19 and 108 us with 2^21; the two meet at 11,000, 23,000 and 50,000
-    samples. 262,144 samples: 754 us by atomics, 221 us sorted."""
+    and fp64 sums (tn_hashgrid_backward_sorted), in parts of at most 2^19
+    samples. Small ones take the atomics: those cost 2.9 us per 1,000 samples,
+    the sort 0.7 to 1.3 us and, for its passes over every bin, 26 us with 2^15
+    entries per level, 43 us with 2^19 and 103 us with 2^21; the two meet at
+    14,000, 20,000 and 46,000 samples. 262,144 samples: 754 us by atomics, 198
+    us sorted."""
     parts = [(lo, min(_SORTED_SAMPLES, n - lo)) for lo in range(0, n, _SORTED_SAMPLES)]
-    big = n >= 10_000 + grid.n_params // 960 and dtable.data_ptr() % 8 == 0
+    big = n >= 13_000 + grid.n_params // 1250 and dtable.data_ptr() % 8 == 0
     nb = query("tn_hashgrid_backward_sorted_bytes", parts[0][1], grid) if big else 0
     if nb == 0:
         hashgrid_backward(grid, n, pos, stride, dfeat, dtable)
