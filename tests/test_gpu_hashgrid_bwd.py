@@ -559,3 +559,32 @@ def test_sorted_keeps_small_contributions(cuda, n, log2_T):
     print(f"[hashgrid sorted] worst/bar {worst.max():.3f}, entries over {np.sum(worst > 1)} of {np.sum(mag > 0)}, "
           f"lost {np.sum((got == 0) & (np.abs(ref) > 1e-30))}", flush=True)
     assert worst.max() <= 1.0
+
+
+def test_sorted_without_room_for_scratch(cuda):
+    """With less memory free than the sort's scratch takes, the call goes to
+    the atomics, which take none: the same gradient, and the limit's error
+    does not reach the caller."""
+    import torch
+
+    from turbonerf_amd import _capi, ops
+
+    g = ops.hashgrid_layout(log2_T=15)
+    rng = np.random.default_rng(3)
+    pos = _rays(rng, 1000, 100, 0.0011)
+    n = pos.shape[1]
+    p = torch.from_numpy(np.ascontiguousarray(pos)).cuda()
+    d = torch.from_numpy(rng.normal(size=(32, n)).astype(np.float32)).cuda()
+    ref, got = torch.zeros(g.n_params, device="cuda"), torch.zeros(g.n_params, device="cuda")
+    ops.hashgrid_backward(g, n, p, n, d, ref)
+    nb = _capi.query("tn_hashgrid_backward_sorted_bytes", n, g)
+    assert nb > 128 << 20
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (32 << 20)) / total)
+        ops.hashgrid_backward_sorted(g, n, p, n, d, got)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert norm_rel(got.cpu().numpy(), ref.cpu().numpy()) < 1e-6

@@ -298,14 +298,19 @@ def hashgrid_backward_sorted(grid: _capi.HashGrid, n: int, pos: torch.Tensor, st
     the sort 0.7 to 1.3 us and, for its passes over every bin, 26 us with 2^15
     entries per level, 43 us with 2^19 and 103 us with 2^21; the two meet at
     14,000, 20,000 and 46,000 samples. 262,144 samples: 754 us by atomics, 198
-    us sorted."""
+    us sorted. A batch whose scratch cannot be had takes the atomics too."""
     parts = [(lo, min(_SORTED_SAMPLES, n - lo)) for lo in range(0, n, _SORTED_SAMPLES)]
     big = n >= 13_000 + grid.n_params // 1250 and dtable.data_ptr() % 8 == 0
     nb = query("tn_hashgrid_backward_sorted_bytes", parts[0][1], grid) if big else 0
-    if nb == 0:
+    ws = None
+    if nb != 0:
+        try:
+            ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+        except torch.cuda.OutOfMemoryError:  # 1.8 KB a sample; the atomics take no scratch
+            pass
+    if ws is None:
         hashgrid_backward(grid, n, pos, stride, dfeat, dtable)
         return
-    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
     for lo, m in parts:
         call("tn_hashgrid_backward_sorted", _PREC[dfeat.dtype], m, None, stride, stride, grid,
              ptr(pos) + lo * pos.element_size(), ptr(dfeat) + lo * dfeat.element_size(), ptr(dtable), ptr(ws), nb,
