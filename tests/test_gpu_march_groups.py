@@ -84,3 +84,46 @@ def test_march_groups_match_oracle(cuda, n_rays, aabb, levels, res, fill):
         assert np.array_equal(smp.img_id[:ns].cpu().numpy().view(np.uint32), so["img_id"][:ns])
         g = smp.pos.cpu().numpy().reshape(3, cap)[:, :ns]
         assert np.array_equal(g.view(np.uint32), so["pos"].reshape(3, cap)[:, :ns].view(np.uint32))
+
+
+@pytest.mark.parametrize("n_rays", [61, 24577])
+@pytest.mark.parametrize("levels,fill", [(1, 1.0), (1, 0.3), (3, 0.2)])
+def test_generate_with_dt_max_below_dt_min(cuda, n_rays, levels, fill):
+    """tn_march_generate takes steps whose upper bound lies below the lower
+    one (tn_march_count refuses them): every step is then the upper bound, in t
+    and in dt, wherever t times the cone angle lies. Bit for bit against the
+    oracle, the counts from the oracle as well."""
+    import torch
+
+    import oracle
+    from turbonerf_amd import ops, scenes
+
+    print(f"[march dt_max < dt_min] rays {n_rays} levels {levels} fill {fill}", flush=True)
+    rng = np.random.default_rng(n_rays + levels)
+    aabb, res, dt_min, dt_max, cone = float(1 << (levels - 1)), 64, 0.02, 0.01, 0.05
+    bits = np.zeros(res ** 3, np.uint8)
+    for l in range(levels):
+        bits |= ((rng.random(res ** 3) < fill).astype(np.uint8) << l).astype(np.uint8)
+    o, d = _rays(rng, n_rays, aabb)
+    t = rng.uniform(0.0, 0.1, n_rays).astype(np.float32)
+    tmax = rng.uniform(0.0, 2.0 * aabb, n_rays).astype(np.float32)
+    box = scenes.bbox(aabb)
+    rr = dict(ori=o.ravel(), dir=d.ravel(), t=t, tmax=tmax, alive=np.ones(n_rays, np.uint8),
+              img_id=np.arange(n_rays, dtype=np.uint32))
+    n_ref, alive_ref = oracle.march_count(n_rays, n_rays, box, bits, levels, res, cone, dt_min, dt_max, rr, 0xFFFFFFFF)
+    excl = np.concatenate([[0], np.cumsum(n_ref)[:-1]]).astype(np.uint32)
+    ns = int(n_ref.sum())
+    assert ns > n_rays
+    so = oracle.march_generate(n_rays, n_rays, ns, box, 1.0 / aabb, bits, levels, res, dt_min, dt_max, cone, rr, excl,
+                               alive_ref, n_ref)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a).ravel()).cuda()
+    rays = ops.Rays.empty(n_rays)
+    rays.ori, rays.dir, rays.t, rays.tmax, rays.alive = T(o), T(d), T(t), T(tmax), T(alive_ref)
+    rays.img_id, rays.n_steps, rays.offset = (T(a.view(np.int32)) for a in (rr["img_id"], n_ref, excl))
+    smp = ops.Samples.empty(ns)
+    ops.march_generate(rays, smp, n_rays, ops.batch_info(n_rays, ns), box, 1.0 / aabb,
+                       ops.grid_struct(T(bits), None, levels, res), dt_min, dt_max, cone)
+    words = lambda x: np.asarray(x).view(np.uint32)
+    assert np.array_equal(words(smp.t.cpu().numpy()), words(so["t"]))
+    assert np.array_equal(words(smp.dt.cpu().numpy()), words(so["dt"]))
+    assert np.array_equal(words(smp.pos.cpu().numpy()), words(so["pos"]))

@@ -110,8 +110,13 @@ inline void with_grid_form(const tn_occupancy_grid_t& grid, float dt_max, Fn fn)
 // and 36 instructions per skip step and a test for runs and skips each).
 // G and T by the number of rays: see kGroup16Rays.
 struct MarchStep {
-    float cone, dt_min, dt_max, inv_dt_min;
+    float cone, dt_lo, dt_max;  // steps of samples: t cone within [dt_lo, dt_max]
+    float dt_min, inv_dt_min;   // skips: whole multiples of dt_min
 };
+// dt_lo is dt_min, but no more than dt_max, where every step is dt_max (get_dt)
+TN_DEVICE MarchStep make_step(float cone, float dt_min, float dt_max) {
+    return {cone, fminf(dt_min, dt_max), dt_max, dt_min, 1.0f / dt_min};
+}
 
 struct MarchRay {
     float ox, oy, oz, dx, dy, dz;
@@ -130,9 +135,9 @@ TN_DEVICE float div_up(float a, float b, float y) {
     return __uint_as_float(__float_as_uint(q) + below);
 }
 
-// get_dt; dt_min <= dt_max
+// get_dt
 TN_DEVICE float step_dt(const MarchStep& st, float t) {
-    return __builtin_amdgcn_fmed3f(t * st.cone, st.dt_min, st.dt_max);
+    return __builtin_amdgcn_fmed3f(t * st.cone, st.dt_lo, st.dt_max);
 }
 TN_DEVICE uint32_t abs_bits(float v) { return __float_as_uint(v) & 0x7FFFFFFFu; }
 
@@ -264,11 +269,11 @@ TN_DEVICE uint32_t march_group(bool active, const MarchRay& r, float t, float t_
         for (int q = 0; q < T; ++q) tj[q] = t;
         if (runs != 0ull) {
             // a run: the t's after so many more samples
-            if (st.dt_min == st.dt_max) {
+            if (st.dt_lo == st.dt_max) {
 #pragma unroll
                 for (uint32_t k = 0; k < S; ++k) {
                     tj[k / G] = j >= k % G ? t_end : tj[k / G];
-                    t_end += st.dt_min;
+                    t_end += st.dt_max;
                 }
             } else {
 #pragma unroll
@@ -444,7 +449,7 @@ march_count_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ d_n_rays, u
                    uint2* __restrict__ runs) {
     const uint32_t n_rays = d_n_rays ? min(*d_n_rays, n_rays_max) : n_rays_max;
     const MarchGrid g = make_grid(grid);
-    const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
+    const MarchStep st = make_step(cone, dt_min, dt_max);
     const MarchCountArgs a = {n_rays, B, max_steps, dir, ray_tmax, ori, ray_t, ray_alive, n_steps, runs};
     if (n_rays <= kTwoBlockRays) march_count_rays<16, 2, F>(a, bbox, g, st);
     else if (n_rays <= kGroup16Rays) march_count_rays<16, 1, F>(a, bbox, g, st);
@@ -611,7 +616,7 @@ march_generate_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ info, ui
                       float* __restrict__ out_t) {
     const uint32_t n_rays = min(info[0], n_rays_max);
     const MarchGrid g = make_grid(grid);
-    const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
+    const MarchStep st = make_step(cone, dt_min, dt_max);
     const MarchGenerateArgs a = {n_rays, B, ori, dir, ray_t, ray_offset, n_ray_steps, ray_alive, out_ray, out_t};
     if (n_rays <= kTwoBlockRays) march_generate_rays<16, 2, F>(a, bbox, g, st);
     else if (n_rays <= kGroup16Rays) march_generate_rays<16, 1, F>(a, bbox, g, st);
@@ -735,9 +740,9 @@ TN_DEVICE void march_generate_from_runs(uint32_t n_rays, uint32_t B, const tn_bb
                 n1 = q < nr ? n_q : ns;
             }
             float tj = t;
-            if (st.dt_min == st.dt_max) {
+            if (st.dt_lo == st.dt_max) {
 #pragma unroll
-                for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k) tj = j > k ? tj + st.dt_min : tj;
+                for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k) tj = j > k ? tj + st.dt_max : tj;
             } else {
 #pragma unroll
                 for (uint32_t k = 0; k + 1 < (uint32_t)G; ++k) tj = j > k ? tj + step_dt(st, tj) : tj;
@@ -766,7 +771,7 @@ march_generate_runs_kernel(uint32_t n_rays_max, const uint32_t* __restrict__ inf
                            const uint32_t* __restrict__ n_ray_steps, const uint2* __restrict__ runs, SampleOut o) {
     const uint32_t n_rays = min(info[0], n_rays_max);
     const MarchGrid g = make_grid(grid);
-    const MarchStep st = {cone, dt_min, dt_max, 1.0f / dt_min};
+    const MarchStep st = make_step(cone, dt_min, dt_max);
     march_generate_from_runs<F>(n_rays, B, bbox, g, st, inv_aabb, ori, dir, ray_t, ray_offset, ray_alive, n_ray_steps,
                                 ray_img_id, runs, o);
 }
