@@ -63,6 +63,8 @@ def test_march_runs(cuda, n_rays, aabb, levels, res, fill):
         n = int(info[1].item())
         most = int(runs.view(torch.int32).view(n_rays, 32)[:, 0][alive_ref != 0].max().item()) if n else 0
         print(f"  samples {n}, most runs {most}", flush=True)
+        if fill == 0.5 and n_rays > 1 and budget == 1.0:
+            assert most > 15  # rays of more runs than records
         words = lambda x: x.view(torch.int32).view(-1, cap)[:, :n]
         for k in ("img_id", "t", "pos", "dir", "dt", "m_norm", "dt_norm"):
             assert torch.equal(words(getattr(ref, k)), words(getattr(out, k))), k
