@@ -40,8 +40,8 @@ int tn_fill_uniform(uint64_t n, uint64_t seed, uint64_t offset, float* out, tn_s
 
 /* The next n uniforms of the same stream at a position kept on the device:
  * element j is element (*d_offset + j) of tn_fill_uniform's stream, and
- * *d_offset advances by n on the stream. A captured training step draws its
- * batch's uniforms this way, so each replay draws new ones. */
+ * *d_offset advances by n on the stream, so that each replay of a captured
+ * call draws new ones. (A training batch draws its own: tn_training_rays.) */
 int tn_fill_uniform_dev(uint64_t n, uint64_t seed, unsigned long long* d_offset, float* out, tn_stream_t stream);
 
 /* Training rays through random pixels, clipped to the training box.

@@ -67,3 +67,21 @@ def test_batch_select(cuda, n, mean, budget):
     assert ia.tolist() == ib.tolist()
     assert torch.equal(a.offset, b.offset)
     assert int(count.item()) == int(nxt.item()) and int(off.item()) == 7 + 4 * cap
+
+
+@pytest.mark.parametrize("n,offset", [(1, 0), (5, 3), (4096, 1 << 33), (100_003, 6)])
+def test_fill_uniform_dev(cuda, n, offset):
+    """tn_fill_uniform_dev is tn_fill_uniform at the position kept on the
+    device, which advances, call after call."""
+    import torch
+
+    from turbonerf_amd import ops
+    from turbonerf_amd._capi import call, ptr, stream_ptr
+
+    print(f"[fill uniform dev] n {n} offset {offset}", flush=True)
+    off = torch.tensor([offset], dtype=torch.int64, device="cuda")
+    for k in range(3):
+        out = torch.full((n + 9,), -1.0, device="cuda")
+        call("tn_fill_uniform_dev", n, 17, ptr(off), ptr(out), stream_ptr())
+        assert torch.equal(out[:n], ops.fill_uniform(n, 17, offset + k * n)) and bool((out[n:] == -1.0).all())
+        assert int(off.item()) == offset + (k + 1) * n

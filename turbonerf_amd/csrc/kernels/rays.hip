@@ -25,8 +25,8 @@ __global__ void uniform_kernel(uint64_t n, uint32_t k0, uint32_t k1, uint64_t of
     }
 }
 
-// The same stream at an offset read on the device (a captured step replays
-// with the offset advancing on the device); the grid covers any alignment.
+// The same stream at an offset read on the device (each replay of a captured
+// call draws at the offset that the one before left); the grid covers any alignment.
 __global__ void uniform_dev_kernel(uint64_t n, uint32_t k0, uint32_t k1, const unsigned long long* __restrict__ d_off,
                                    float* __restrict__ out) {
     const uint64_t offset = *d_off;
