@@ -270,15 +270,6 @@ void NeRFTrainingController::set_occupancy_from_density(const float* density_hos
     TN_HIP(hipStreamSynchronize(s));
 }
 
-std::vector<float> NeRFTrainingController::get_params() const {
-    const NeRF& nerf = proxy->nerfs[0];
-    std::vector<float> h(nerf.params.params_fp.size());
-    // training work ends with the device stream waiting for it
-    TN_HIP(hipStreamSynchronize(DeviceManager::stream()));
-    TN_HIP(hipMemcpy(h.data(), nerf.params.params_fp.data(), h.size() * sizeof(float), hipMemcpyDeviceToHost));
-    return h;
-}
-
 void NeRFTrainingController::read_params(float* dst) {
     const DeviceBuffer<float>& p = proxy->nerfs[0].params.params_fp;
     // training work ends with the device stream waiting for it

@@ -127,9 +127,8 @@ struct NeRFTrainingController {
     // occupancy bitfield from an external density grid (synthetic scenes)
     void set_occupancy_from_density(const float* density_host, float threshold);
     // raw parameter access (fp32 master weights), for tests and snapshots
-    std::vector<float> get_params() const;
     size_t n_params() const { return proxy->nerfs[0].params.params_fp.size(); }
-    // get_params() into a caller's array of n_params()
+    // into a caller's array of n_params()
     void read_params(float* dst);
     void set_params(const std::vector<float>& p);
 

@@ -140,16 +140,14 @@ def batch_info(n_rays: int, n_samples: int) -> torch.Tensor:
 def composite_train(info: torch.Tensor, n_rays_max: int, stride: int, sample_stride: int, steps: torch.Tensor,
                     offs: torch.Tensor, bg: torch.Tensor, target: torch.Tensor, density: torch.Tensor,
                     color: torch.Tensor, dt: torch.Tensor, grad_scale: float = 1.0, min_T: float = 1e-4,
-                    fp64_accumulate: bool = False, scale_by_rays: bool = False, whole: bool = False):
-    """Returns (loss[4*stride], dL_ddensity[sample_stride], dL_dcolor[3*sample_stride]).
-    whole: info counts every ray and sample of the buffers, so that nothing
-    beyond the batch is left to be zero."""
+                    fp64_accumulate: bool = False, scale_by_rays: bool = False):
+    """Returns (loss[4*stride], dL_ddensity[sample_stride], dL_dcolor[3*sample_stride])."""
     code = 2 if fp64_accumulate else _DTYPE_CODE[density.dtype]
     if fp64_accumulate and density.dtype != torch.float32:
         raise ValueError("fp64 accumulation takes fp32 inputs")
-    loss = _out(4 * stride, whole, torch.float32)
-    dLd = _out(sample_stride, whole, torch.float32)
-    dLc = _out(3 * sample_stride, whole, density.dtype)
+    loss = torch.zeros(4 * stride, dtype=torch.float32, device="cuda")
+    dLd = torch.zeros(sample_stride, dtype=torch.float32, device="cuda")
+    dLc = torch.zeros(3 * sample_stride, dtype=density.dtype, device="cuda")
     nb = query("tn_composite_scratch_bytes", n_rays_max, sample_stride)
     scratch = torch.empty(nb // 4, dtype=torch.float32, device="cuda")
     call("tn_composite_train", code, ptr(info), n_rays_max, stride, sample_stride, grad_scale, int(scale_by_rays), min_T,
