@@ -442,7 +442,6 @@ TN_DEVICE uint32_t hb_round17(float v) {
 
 struct HbRec8 {
     static constexpr bool kEntryArray = false, kFixed = true;
-    static constexpr size_t kBytes = 8;
     TN_DEVICE static uint32_t value(float v) { return hb_round17(v); }
     TN_DEVICE static uint2 pack(uint32_t e, uint32_t r0, uint32_t r1) { return make_uint2(r0 | (e & 63u), r1 | (e >> 6)); }
     TN_DEVICE static uint32_t entry(uint2 r, uint32_t) { return (r.x & 63u) | ((r.y & 63u) << 6); }
@@ -451,7 +450,6 @@ struct HbRec8 {
 };
 struct HbRec10 {
     static constexpr bool kEntryArray = true, kFixed = false;
-    static constexpr size_t kBytes = 10;
     TN_DEVICE static uint32_t value(float v) { return __float_as_uint(v); }
     TN_DEVICE static uint2 pack(uint32_t, uint32_t r0, uint32_t r1) { return make_uint2(r0, r1); }
     TN_DEVICE static uint32_t entry(uint2, uint32_t e) { return e; }
@@ -663,10 +661,6 @@ TN_DEVICE void hb_corners(const tn_hashgrid_t& g, int l, bool active, const HbIn
         hc.a1[c] = a1[c];
     }
     hc.emit = hb_emits(active, hm);
-}
-
-TN_DEVICE uint32_t abs_bits(float a, float b) {
-    return max(__float_as_uint(fabsf(a)), __float_as_uint(fabsf(b)));
 }
 
 // (1) per-block record counts per bin of the block's level (the run
