@@ -881,11 +881,11 @@ __global__ void __launch_bounds__(kHbScatterThreads) hashgrid_bwd_scatter_kernel
                 const bool one = bin[k] == bin[k + 1];
                 rank[k] = atomicAdd(&cnt[bin[k]], one ? 2u : 1u);
                 rank[k + 1] = rank[k] + 1u;
-                if (!one) rank[k + 1] = atomicAdd(&cnt[bin[k + 1]], 1u);
-                if constexpr (Rec::kFixed) {
-                    const uint32_t m0 = one ? max(m[0], m[1]) : m[0];
-                    if (m0 != 0u) atomicMax(&bmax[bin[k]], m0);
-                    if (!one && m[1] != 0u) atomicMax(&bmax[bin[k + 1]], m[1]);
+                const uint32_t m0 = one ? max(m[0], m[1]) : m[0];
+                if (Rec::kFixed && m0 != 0u) atomicMax(&bmax[bin[k]], m0);
+                if (!one) {
+                    rank[k + 1] = atomicAdd(&cnt[bin[k + 1]], 1u);
+                    if (Rec::kFixed && m[1] != 0u) atomicMax(&bmax[bin[k + 1]], m[1]);
                 }
             }
         }
